@@ -1,16 +1,16 @@
 // Conv2D / PartialConv2D / Dense (float32) for gfx950.
 //
-// input_channels % 16 == 0: implicit GEMM on v_mfma_f32_32x32x2_f32,
+// input_channels % 16 == 0: implicit GEMM,
 //      D[co][px] += sum_k  F[co][k] * I[k][px],   k = (tap, ci)
-// MFMA rows are output channels, MFMA columns are output pixels flattened over (image, oh, ow).
+// on v_mfma_f32_32x32x16_bf16: every float32 operand is split into three bf16 numbers that add up to it exactly, and six
+// of the nine products (all but those below half a unit in the last place of a float32 product) are added in float32
+// (Split8 below).  MFMA rows are output channels, MFMA columns are output pixels flattened over (image, oh, ow).
 // With the packed layouts a K-step of 16 (one input-channel block at one filter tap) needs no
 // shuffling at all:
 //   - B operand: lane (px = lane%32, half = lane/32) reads 8 consecutive floats of its pixel's
-//     64-byte channel block: two 16-byte loads straight from global memory into the register the
-//     MFMA consumes.  The two wave halves take channels 0-7 and 8-15, so MFMA number kk of the
-//     step contracts channels {kk, 8+kk}; the pairing of k inside an MFMA is free as long as A
-//     and B agree.  Padded taps load a block of zeros.
-//   - A operand: F[ci = 8*half+kk][co%16] of the channel block's [16 ci][16 co] tile, staged
+//     64-byte channel block, two 16-byte loads straight from global memory, and splits them: channels 8*half .. +7 are the
+//     lane's eight reduction elements.  Padded taps load a block of zeros.
+//   - A operand: F[ci = 8*half + 0..7][co%16] of the channel block's [16 ci][16 co] tile, split and staged
 //     through LDS once per workgroup (conv_lds_tile) or read directly (conv_splitk_tile).
 //   - D: a lane holds 4 consecutive output channels of one pixel per register quad, i.e. 16-byte
 //     stores into the packed [px][16] output, after accumulate / bias / activation in registers.
@@ -37,6 +37,100 @@ namespace
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// ---------------------------------------------------------------------------------------------
+// float32 products on the bf16 matrix pipes.  A float32 number is the exact sum of three bf16 numbers, x = h + m + l with
+// h = bf16(x), m = bf16(x - h), l = x - h - m (24 bits = 3 x 8; round to nearest, so |m| <= 2^-8 |x|, |l| <= 2^-17 |x| and
+// their signs do not follow x's), and a product of two bf16 numbers is exact in float32.  x * y is then added up as
+// hh + (hm + mh + mm + hl + lh); what is left out, ml + lm + ll, is below 2^-24 |x y|, half a unit in the last place of the
+// product.  v_mfma_f32_32x32x16_bf16 multiplies sixteen times as fast as v_mfma_f32_32x32x2_f32, six of them replace
+// eight float32 ones per sixteen channels: 192 matrix cycles instead of 512, and the vector ALU may issue beside them
+// (a float32 MFMA occupies it).
+// hh has an accumulator of its own ("big"): there one addition per sixteen products is rounded where the float32 MFMA
+// chain rounds sixteen, and the small terms are added to a sum of their own size, so that nothing of them is lost
+// against a large total.  Error against float64 (relative 2-norm, K = 16 / 64 / 512 / 2304 / 4608 normal products): the
+// float32 MFMA chain 7.4e-8 / 1.4e-7 / 4.0e-7 / 8.6e-7 / 1.2e-6; see the tests for this form's.
+// Range: |x| below 2^-110 loses bits of m and l (an absolute error of at most 2^-134 |y|); |x| above 3.3895e38 (the
+// largest bf16) counts as infinite.  Infinities and NaN give what float32 products give (split_sum).
+struct Split8
+{
+    bf16x8 h, m, l;      // eight consecutive reduction elements of one row or column: one MFMA operand each
+};
+
+__device__ __forceinline__ unsigned pack_bf16(float a, float b)
+{
+    bf16x2 v;
+    v[0] = (__bf16)a;
+    v[1] = (__bf16)b;
+    unsigned u = __builtin_bit_cast(unsigned, v);
+    asm("" : "+v"(u));   // one v_cvt_pk_bf16_f32: without this the halves are converted again for the subtraction
+    return u;
+}
+__device__ __forceinline__ float bf16_lo(unsigned u) { return __builtin_bit_cast(float, u << 16); }
+__device__ __forceinline__ float bf16_hi(unsigned u) { return __builtin_bit_cast(float, u & 0xffff0000u); }
+
+// a pair of numbers: 11 vector instructions
+__device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l)
+{
+    h = pack_bf16(a, b);
+    a -= bf16_lo(h);
+    b -= bf16_hi(h);
+    m = pack_bf16(a, b);
+    a -= bf16_lo(m);
+    b -= bf16_hi(m);
+    l = pack_bf16(a, b);
+}
+__device__ __forceinline__ Split8 split8(const float (&x)[8])
+{
+    u32x4 h, m, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+    {
+        unsigned hh, mm, ll;
+        split_pair(x[2 * i], x[2 * i + 1], hh, mm, ll);
+        h[i] = hh; m[i] = mm; l[i] = ll;
+    }
+    return Split8{__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
+}
+__device__ __forceinline__ Split8 split8(const float4 &lo, const float4 &hi)
+{
+    const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    return split8(x);
+}
+
+// sixteen channels: COT x PXT tiles of 32 x 32, the order inside each accumulator fixed (the same bits in every kernel)
+template <int COT, int PXT>
+__device__ __forceinline__ void mfma_split(floatx16 (&big)[COT][PXT], floatx16 (&sml)[COT][PXT], const Split8 (&A)[COT],
+                                           const Split8 (&B)[PXT])
+{
+#define SHP_MFMA_(acc_, a_, b_)                                                                               \
+    _Pragma("unroll") for (int t = 0; t < PXT; ++t) _Pragma("unroll") for (int c = 0; c < COT; ++c)           \
+        acc_[c][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[c].a_, B[t].b_, acc_[c][t], 0, 0, 0)
+    SHP_MFMA_(sml, l, h);
+    SHP_MFMA_(sml, h, l);
+    SHP_MFMA_(sml, m, m);
+    SHP_MFMA_(sml, m, h);
+    SHP_MFMA_(sml, h, m);
+    SHP_MFMA_(big, h, h);
+#undef SHP_MFMA_
+}
+// big + small.  An infinite operand leaves an infinity or NaN in big, as float32 products would, and NaN or infinity
+// (inf - inf) in the parts that small sums up: there small is replaced by a finite number.
+__device__ __forceinline__ float split_sum(float big, float sml) { return big + __builtin_amdgcn_fmed3f(sml, -3.0e38f, 3.0e38f); }
+template <int COT, int PXT>
+__device__ __forceinline__ void split_merge(floatx16 (&big)[COT][PXT], const floatx16 (&sml)[COT][PXT])
+{
+#pragma unroll
+    for (int c = 0; c < COT; ++c)
+#pragma unroll
+        for (int t = 0; t < PXT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) big[c][t][r] = split_sum(big[c][t][r], sml[c][t][r]);
+}
+
 struct ConvArgs
 {
     const float *in;
@@ -54,6 +148,7 @@ struct ConvArgs
     int n_px_blocks;     // ceil(P / (32*PXT*4))
     int n_blocks;        // n_co_groups * n_px_blocks
     int per_xcd;         // ceil(n_blocks / 8)
+    int px_first;        // split-K kernel: consecutive workgroups (one XCD) take the pixel blocks of a channel group
     int n_main;          // hybrid kernel: workgroups that run whole tiles (multiple of the CU count)
     // grouped convolution: blockIdx.y walks `slabs` (image, group) slabs of Ci channels that lie in_slab / out_slab
     // floats apart; slab y uses filter block (slab0 + y) % groups.  slabs == 0: an ordinary convolution.
@@ -113,15 +208,13 @@ __device__ __forceinline__ float act_bf(float v, float neg_scale)
     return v > 0.f ? v : n;
 }
 // The same with the kind known at compile time: ReLU is one instruction (a maximum) instead of three, and gives the
-// same bits as act_bf(v, 0) for every input that is a number (negative and -0 -> +0).  A vector instruction costs the
-// matrix pipe of its SIMD about eight cycles whichever wave issues it, so the epilogues' instruction count is launch time.
+// same bits as act_bf(v, 0) for every input that is a number (negative and -0 -> +0).
 template <bool RELU>
 __device__ __forceinline__ float act_k(float v, float neg_scale)
 {
     return RELU ? fmaxf(v, 0.f) : act_bf(v, neg_scale);
 }
 
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr unsigned BUF_OUT_OF_RANGE = 0x80000000u;
 constexpr long long BUF_MAX_BYTES = 1ll << 30;
 constexpr int BUF_RSRC_FLAGS = 0x00020000;            // raw buffer of 32-bit elements
@@ -335,19 +428,21 @@ __device__ __forceinline__ void pool_tile_pixel(const ConvArgs &a, const int til
 // ---------------------------------------------------------------------------------------------
 // The main kernel body: filter operand staged through LDS.  The four waves of a workgroup
 // multiply the same output-channel group, so the step's [16 ci][16 co] filter tiles (COT*2 KiB)
-// are fetched once per workgroup with fully coalesced 16-byte loads, written to LDS (double
-// buffered, one barrier per K-step) and read back by every wave in MFMA operand order: a quarter
-// of the vector-cache accesses of per-wave filter reads, and one 16-byte load per lane instead
-// of 8 strided dword loads per tile.  The activation operand goes straight from global memory to
-// the MFMA register, two 16-byte loads per lane and tile.
-constexpr int A_TILE_FLOATS = 272;   // 256 + 16 pad: consecutive channel blocks start 16 banks apart
+// are fetched once per workgroup (a thread takes consecutive input channels of one output channel), split once,
+// written to LDS in MFMA operand order (double buffered, one barrier per K-step) and read back by every wave
+// with three 16-byte reads per tile.  The activation operand goes straight from global memory to
+// the wave that multiplies it, two 16-byte loads and one split per lane and tile.
+// What bounds it: the matrix pipes at the clock the card's power limit leaves (six products on registers alone run at
+// 1.8 GHz and 290-300 TFLOP/s) and the split's vector instructions, of which a bit more than half hide behind the MFMAs (the
+// loop of a 64 x 32 wave tile without global loads: 209 TFLOP/s, 265 with the split left out).  Batch 64 / 16, before (float32
+// MFMAs) -> now: 3x3 256->256 @56x56 1572 -> 1102 us (215 TFLOP/s), 3x3 1024->1024 @13x13 376 -> 285, 3x3 128->256 @26x26
+// 50.2 -> 45.4, 1x1 512->512 @14x14 50.4 -> 40.0, 1x1 128->128 @56x56 64.5 -> 59.3 (its 206 MB are 40 us of copy).
 
 // s_begin / s_count: only K-steps [s_begin, s_begin + s_count) of the tile (s_count < 0: all of them); raw != nullptr: the
 // accumulators go there as they are ([wave][tile of the wave][register quad][lane] float4) instead of through the epilogue
 // PW: a pointwise convolution (1x1 window, stride 1, no padding): the activation operand of a lane is its own pixel's
 // channel vector, channel block after channel block, so a K-step needs one address instruction per pixel tile where the
-// general form needs about ten (window position, bounds, select).  Every vector instruction between the MFMAs takes an
-// issue slot of the SIMD away from them (measured on a loop of this shape: 12 vector instructions per 16 MFMAs = 4%).
+// general form needs about ten (window position, bounds, select).
 // BLDS: the workgroup runs this body once; its bias values are requested first of all and parked in LDS under the K loop, so
 // the epilogue does not wait for memory once more (a caller that runs several tiles per workgroup would overwrite them
 // while another wave still reads)
@@ -358,8 +453,11 @@ constexpr int A_TILE_FLOATS = 272;   // 256 + 16 pad: consecutive channel blocks
 // launcher allows it for tensors of at most 1 GiB (lane offset + scalar offset + 16 stays below 2^31 on either side of
 // the range check, whether or not the hardware adds the scalar offset before it checks).
 
+template <int COT>
+using FiltStage = unsigned char[2][COT * 3 * 1024];
+
 template <int COT, int PXT, bool POOL = false, bool PW = false, bool BLDS = false, bool BUF = false>
-__device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, float (&lds_a)[2][COT * 2 * A_TILE_FLOATS],
+__device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, FiltStage<COT> &lds_a,
                                               const int cg, const int pxb, const int s_begin = 0, const int s_count = -1,
                                               float *raw = nullptr)
 {
@@ -417,40 +515,25 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, float (&lds_a)[
         if (PW) in_img[t] += (size_t)(oh * a.W + ow) * CB;
     }
 
-    // ---- cooperative filter fetch: COT*2 tiles of 64 float4 each -----------------------------
-    constexpr int A_VECS = COT * 2 * 64;                 // float4 per step and workgroup
-    constexpr int A_PER_THREAD = (A_VECS + 255) / 256;   // 1 for COT <= 2, 2 for COT == 4
-    // Every thread loads and stores (no predicate): with fewer vectors than threads (COT == 1) the
-    // upper threads repeat a lower thread's vector and write the same value to the same place.  A
-    // predicated load would put the wait of the staging store inside a branch, and the compiler
-    // would then have to wait at the top of the loop for loads issued only a step earlier.
-    static_assert(A_VECS >= 256 ? A_VECS % 256 == 0 : 256 % A_VECS == 0, "filter vectors vs workgroup size");
-    const float *a_src[A_PER_THREAD];
-    unsigned a_voff[A_PER_THREAD];
-    int a_dst[A_PER_THREAD];
-#pragma unroll
-    for (int j = 0; j < A_PER_THREAD; ++j)
-    {
-        const int vc = (tid + j * 256) % A_VECS;
-        const int blk = vc >> 6, within = vc & 63;
-        int cob = cg * COT * 2 + blk;
-        cob = cob < CoB ? cob : CoB - 1;                  // rows past Co: garbage, never stored
-        a_src[j] = a.filt + (size_t)cob * CiB * taps * (CB * CB) + within * 4;
-        a_voff[j] = (unsigned)(((size_t)cob * CiB * taps * (CB * CB) + within * 4) * sizeof(float));
-        a_dst[j] = blk * A_TILE_FLOATS + within * 4;
-    }
-    // read position of this lane inside a staged tile pair
-    int a_rd[COT];
-#pragma unroll
-    for (int c = 0; c < COT; ++c) a_rd[c] = (c * 2 + (col >> 4)) * A_TILE_FLOATS + half * 8 * CB + (col & 15);
+    // ---- cooperative filter fetch: a thread owns AE consecutive input channels of one output channel ----------------
+    // (COT 1 / 2 / 4: 2 / 4 / 8 of the lane's eight), splits them and writes its piece of the three operands
+    constexpr int AE = COT * 2, SUBS = 8 / AE;
+    const int a_c = tid / (64 * SUBS), a_u = tid % (64 * SUBS), a_l = a_u / SUBS, a_sub = a_u % SUBS;
+    const int a_ci = 8 * (a_l >> 5) + AE * a_sub;
+    int a_cob = (cg * COT + a_c) * 2 + ((a_l & 31) >> 4);
+    a_cob = a_cob < CoB ? a_cob : CoB - 1;                // rows past Co: garbage, never stored
+    const size_t a_first = (size_t)a_cob * CiB * taps * (CB * CB) + a_ci * CB + (a_l & 15);
+    const float *a_src = a.filt + a_first;
+    const unsigned a_voff = (unsigned)(a_first * sizeof(float));
+    const int a_dst = a_c * 3 * 1024 + a_l * 16 + a_sub * (2 * AE);
 
-    floatx16 acc[COT][PXT];
+    floatx16 acc[COT][PXT], sml[COT][PXT];
 #pragma unroll
     for (int c = 0; c < COT; ++c)
 #pragma unroll
         for (int t = 0; t < PXT; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[c][t][r] = 0.f;
+            for (int r = 0; r < 16; ++r) acc[c][t][r] = sml[c][t][r] = 0.f;
 
     // first step: channel block fastest, then the window column, then the row
     const int tap0 = s_begin / CiB;
@@ -483,13 +566,13 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, float (&lds_a)[
                                                    (int)((size_t)CoB * CiB * taps * (CB * CB) * sizeof(float)), 0x00020000);
         tap_offsets();
     }
-    auto fetch = [&](float4 (&Areg)[A_PER_THREAD], float4 (&B)[PXT][2]) {
+    auto fetch = [&](float (&Areg)[AE], float4 (&B)[PXT][2]) {
         if (BUF)
         {
             const int soff_a = (cib * taps + ta * a.kw + tb) * (CB * CB * (int)sizeof(float));
 #pragma unroll
-            for (int j = 0; j < A_PER_THREAD; ++j)
-                Areg[j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_f, a_voff[j], soff_a, 0));
+            for (int j = 0; j < AE; ++j)
+                Areg[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_f, a_voff + j * (CB * (int)sizeof(float)), soff_a, 0));
             const int soff_b = cib * (in_blk32 * (int)sizeof(float));
 #pragma unroll
             for (int t = 0; t < PXT; ++t)
@@ -522,7 +605,7 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, float (&lds_a)[
         {
             const int woff = cib * (CB * CB);
 #pragma unroll
-            for (int j = 0; j < A_PER_THREAD; ++j) Areg[j] = *reinterpret_cast<const float4 *>(a_src[j] + woff);
+            for (int j = 0; j < AE; ++j) Areg[j] = a_src[woff + j * CB];
             const int cib_off = cib * in_blk32;              // wave-uniform
 #pragma unroll
             for (int t = 0; t < PXT; ++t)
@@ -539,7 +622,7 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, float (&lds_a)[
         // alone and leave the activation loads of the same step in flight
         const int woff = (cib * taps + tap) * (CB * CB);
 #pragma unroll
-        for (int j = 0; j < A_PER_THREAD; ++j) Areg[j] = *reinterpret_cast<const float4 *>(a_src[j] + woff);
+        for (int j = 0; j < AE; ++j) Areg[j] = a_src[woff + j * CB];
         const int cib_off = cib * in_blk32;
 #pragma unroll
         for (int t = 0; t < PXT; ++t)
@@ -564,32 +647,38 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, float (&lds_a)[
         ta = more ? nta : ta;
         live = live && more;
     };
-    auto stage = [&](int buf, const float4 (&Areg)[A_PER_THREAD]) {
+    auto stage = [&](int buf, const float (&Areg)[AE]) {
+        unsigned h[COT], m[COT], l[COT];                     // AE / 2 = COT packed pairs
 #pragma unroll
-        for (int j = 0; j < A_PER_THREAD; ++j) *reinterpret_cast<float4 *>(&lds_a[buf][a_dst[j]]) = Areg[j];
+        for (int i = 0; i < COT; ++i) split_pair(Areg[2 * i], Areg[2 * i + 1], h[i], m[i], l[i]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+        {
+            const unsigned(&q)[COT] = p == 0 ? h : p == 1 ? m : l;
+            unsigned char *d = &lds_a[buf][a_dst + p * 1024];
+            if constexpr (COT == 1) *reinterpret_cast<unsigned *>(d) = q[0];
+            else if constexpr (COT == 2) *reinterpret_cast<uint2 *>(d) = make_uint2(q[0], q[1]);
+            else *reinterpret_cast<uint4 *>(d) = make_uint4(q[0], q[1], q[2], q[3]);
+        }
     };
     auto multiply = [&](int buf, const float4 (&B)[PXT][2]) {
-        float A[COT][8];
+        Split8 A[COT], Bs[PXT];
 #pragma unroll
         for (int c = 0; c < COT; ++c)
+        {
+            const unsigned char *r = &lds_a[buf][c * 3 * 1024 + lane * 16];
+            A[c].h = *reinterpret_cast<const bf16x8 *>(r);
+            A[c].m = *reinterpret_cast<const bf16x8 *>(r + 1024);
+            A[c].l = *reinterpret_cast<const bf16x8 *>(r + 2048);
+        }
 #pragma unroll
-            for (int kk = 0; kk < 8; ++kk) A[c][kk] = lds_a[buf][a_rd[c] + kk * CB];
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk)
-#pragma unroll
-            for (int t = 0; t < PXT; ++t)
-            {
-                const float4 bv = B[t][kk >> 2];
-                const float b = (kk & 3) == 0 ? bv.x : (kk & 3) == 1 ? bv.y : (kk & 3) == 2 ? bv.z : bv.w;
-#pragma unroll
-                for (int c = 0; c < COT; ++c)
-                    acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(A[c][kk], b, acc[c][t], 0, 0, 0);
-            }
+        for (int t = 0; t < PXT; ++t) Bs[t] = split8(B[t][0], B[t][1]);
+        mfma_split<COT, PXT>(acc, sml, A, Bs);
     };
 
     // Schedule per step s:  multiply(s) | stage filter(s+1) into the other LDS buffer | fetch(s+2)
     // | barrier.  The loads of a step are issued a whole step before they are consumed.
-    float4 Areg[A_PER_THREAD];
+    float Areg[AE];
     float4 B0[PXT][2], B1[PXT][2];
     fetch(Areg, B0);                 // step 0
     stage(0, Areg);
@@ -610,6 +699,7 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, float (&lds_a)[
     }
     // an odd step count leaves the last step staged in buffer 0 / B0 (the loop's invariant)
     if (nsteps & 1) multiply(0, B0);
+    split_merge<COT, PXT>(acc, sml);
 
     if (raw)
     {
@@ -633,14 +723,13 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, float (&lds_a)[
     else conv_epilogue<COT, PXT>(a, acc, cg, half, HoWo, pvalid, out_pix, BLDS ? s_bias : nullptr);
 }
 
-// The second launch bound (minimum waves per SIMD: 6 / 5 / 2 for one / two / four MFMA tiles per
-// wave) makes the compiler keep the accumulators in the unified register file and pack tighter
-// (2x1: 108 -> 76 registers, 2x2: 184 -> 131, no spills); measured 1-3% faster, tighter bounds spill.
+// The second launch bound (minimum waves per SIMD: 4 / 3 / 2 for one / two / four MFMA tiles per
+// wave) makes the compiler keep both sets of accumulators in the unified register file: 80 / 126 / 220 registers, no spills.
 template <int COT, int PXT, bool POOL = false, bool PW = false, bool BUF = false>
-__global__ __launch_bounds__(256, (COT * PXT == 2 ? 5 : COT * PXT == 1 ? 6 : 2)) void conv_mfma_f32_lds_kernel(const ConvArgs a0)
+__global__ __launch_bounds__(256, (COT * PXT == 2 ? 3 : COT * PXT == 1 ? 4 : 2)) void conv_mfma_f32_lds_kernel(const ConvArgs a0)
 {
     const ConvArgs a = slab_args(a0);
-    __shared__ float lds_a[2][COT * 2 * A_TILE_FLOATS];
+    __shared__ __align__(16) FiltStage<COT> lds_a;
     const int bid = blockIdx.x;
     const int lid = (bid % NUM_XCD) * a.per_xcd + bid / NUM_XCD;
     if (lid >= a.n_blocks) return;            // whole workgroup leaves together: no barrier is skipped
@@ -649,15 +738,17 @@ __global__ __launch_bounds__(256, (COT * PXT == 2 ? 5 : COT * PXT == 1 ? 6 : 2))
 
 // ---------------------------------------------------------------------------------------------
 // Small outputs (few 32x32 tiles per SIMD: fully connected layers, 7x7 / 13x13 feature maps,
-// batch 1): the four waves of a workgroup take the SAME output tile and one quarter of the K-steps
-// each, then waves 1..3 hand their partial accumulators to wave 0 through LDS, which adds them in
-// the fixed order 0+1+2+3 (deterministic) and runs the epilogue.  Operands go straight from global
-// memory to the MFMA registers (nothing is shared between the waves until the reduction).
+// batch 1): the W waves of a workgroup take the SAME output tile and an equal share of the K-steps
+// each, then the others hand their partial accumulators to wave 0 through LDS, which adds them in
+// wave order (deterministic) and runs the epilogue.  Operands go straight from global
+// memory to the wave's registers (nothing is shared between the waves until the reduction).  Both operands are split for
+// one tile, 88 vector instructions (352 cycles) against 192 matrix cycles per K-step: what bounds the long reductions.
 // POOL: the 32-pixel tiles are the pooling form's groups of 8 windows and the epilogue pools (pool_tile_pixel)
 // BUF: operands through buffer loads, as in conv_lds_tile (each wave has its own K range, so its window position and
 // scalar offsets are the wave's)
-template <int COT, int PXT, bool POOL = false, bool BUF = false>
-__device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)[3][COT * PXT][16][64],
+// W: waves of the workgroup, each with its share of the K-steps
+template <int COT, int PXT, bool POOL = false, bool BUF = false, int W = 4>
+__device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)[W - 1][COT * PXT][16][64],
                                                  const int cg, const int pxb)
 {
     const int lane = threadIdx.x & 63;
@@ -712,17 +803,17 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)
         w_voff[c] = (unsigned)(((size_t)(cc / CB) * CiB * taps * (CB * CB) + (cc % CB) + half * 8 * CB) * sizeof(float));
     }
 
-    floatx16 acc[COT][PXT];
+    floatx16 acc[COT][PXT], sml[COT][PXT];
 #pragma unroll
     for (int c = 0; c < COT; ++c)
 #pragma unroll
         for (int t = 0; t < PXT; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[c][t][r] = 0.f;
+            for (int r = 0; r < 16; ++r) acc[c][t][r] = sml[c][t][r] = 0.f;
 
     // this wave's K range: steps [s_lo, s_hi) of the (tap outer, channel block inner) order
     const int nsteps = taps * CiB;
-    const int per = (nsteps + 3) >> 2;
+    const int per = (nsteps + W - 1) / W;
     const int s_lo = wave * per;
     const int s_hi = (s_lo + per < nsteps) ? s_lo + per : nsteps;
     const int mine = s_hi > s_lo ? s_hi - s_lo : 0;
@@ -763,7 +854,8 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)
                 B[t][0] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_in, voff[t], soff_b, 0));
                 B[t][1] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_in, voff[t] + 16, soff_b, 0));
             }
-            const int soff_a = (cib * taps + ta * a.kw + tb) * (CB * CB * (int)sizeof(float));
+            // past the wave's last step the filter reads zeros as well
+            const int soff_a = left > 0 ? (cib * taps + ta * a.kw + tb) * (CB * CB * (int)sizeof(float)) : (int)BUF_SCALAR_OUT_OF_RANGE;
 #pragma unroll
             for (int c = 0; c < COT; ++c)
 #pragma unroll
@@ -780,7 +872,7 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)
             }
             return;
         }
-        const bool live = left > 0;
+        const bool live = left > 0;                  // (the filter of a step past the last is multiplied by zeros)
         const int tap = ta * a.kw + tb;
 #pragma unroll
         for (int t = 0; t < PXT; ++t)
@@ -810,17 +902,12 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)
         --left;
     };
     auto compute_step = [&](const float (&A)[COT][8], const float4 (&B)[PXT][2]) {
+        Split8 As[COT], Bs[PXT];
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk)
+        for (int c = 0; c < COT; ++c) As[c] = split8(A[c]);
 #pragma unroll
-            for (int t = 0; t < PXT; ++t)
-            {
-                const float4 bv = B[t][kk >> 2];
-                const float b = (kk & 3) == 0 ? bv.x : (kk & 3) == 1 ? bv.y : (kk & 3) == 2 ? bv.z : bv.w;
-#pragma unroll
-                for (int c = 0; c < COT; ++c)
-                    acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(A[c][kk], b, acc[c][t], 0, 0, 0);
-            }
+        for (int t = 0; t < PXT; ++t) Bs[t] = split8(B[t][0], B[t][1]);
+        mfma_split<COT, PXT>(acc, sml, As, Bs);
     };
 
     float A0[COT][8], A1[COT][8];
@@ -835,7 +922,8 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)
         compute_step(A1, B1);
     }
 
-    // ---- reduction over the four K quarters --------------------------------------------------
+    split_merge<COT, PXT>(acc, sml);
+    // ---- reduction over the waves
     if (wave > 0)
     {
 #pragma unroll
@@ -849,7 +937,7 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)
     if (wave == 0)
     {
 #pragma unroll
-        for (int w = 0; w < 3; ++w)
+        for (int w = 0; w < W - 1; ++w)
 #pragma unroll
             for (int c = 0; c < COT; ++c)
 #pragma unroll
@@ -861,15 +949,17 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)
     }
 }
 
-template <int COT, int PXT, bool BUF = false>
-__global__ __launch_bounds__(256) void conv_mfma_f32_splitk_kernel(const ConvArgs a0)
+template <int COT, int PXT, bool BUF = false, int W = 4>
+__global__ __launch_bounds__(64 * W) void conv_mfma_f32_splitk_kernel(const ConvArgs a0)
 {
     const ConvArgs a = slab_args(a0);
-    __shared__ float red[3][COT * PXT][16][64];
+    __shared__ float red[W - 1][COT * PXT][16][64];
     const int bid = blockIdx.x;
     const int lid = (bid % NUM_XCD) * a.per_xcd + bid / NUM_XCD;
     if (lid >= a.n_blocks) return;
-    conv_splitk_tile<COT, PXT, false, BUF>(a, red, lid % a.n_co_groups, lid / a.n_co_groups);
+    const int cg = a.px_first ? lid / a.n_px_blocks : lid % a.n_co_groups;
+    const int pxb = a.px_first ? lid - cg * a.n_px_blocks : lid / a.n_co_groups;
+    conv_splitk_tile<COT, PXT, false, BUF, W>(a, red, cg, pxb);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -881,10 +971,10 @@ __global__ __launch_bounds__(256) void conv_mfma_f32_splitk_kernel(const ConvArg
 // 4*COT*PXT times as many workgroups that each last 1/(4*COT*PXT) as long and spread over every CU.
 // The hardware starts workgroups in block-id order, so the tail follows the whole rounds.
 template <int COT, int PXT, bool POOL = false, bool PW = false, bool BUF = false>
-__global__ __launch_bounds__(256, (COT * PXT == 2 ? 5 : COT * PXT == 1 ? 6 : 2)) void conv_mfma_f32_hybrid_kernel(const ConvArgs a0)
+__global__ __launch_bounds__(256, (COT * PXT == 2 ? 3 : COT * PXT == 1 ? 4 : 2)) void conv_mfma_f32_hybrid_kernel(const ConvArgs a0)
 {
     const ConvArgs a = slab_args(a0);
-    __shared__ float lds_a[2][COT * 2 * A_TILE_FLOATS];
+    __shared__ __align__(16) FiltStage<COT> lds_a;
     __shared__ float red[3][1][16][64];
     const int bid = blockIdx.x;
     if (bid < a.n_main)
@@ -918,9 +1008,9 @@ template <int COT, int PXT>
 constexpr int sk_part_floats() { return 4 * COT * PXT * 16 * WAVE; }
 
 template <int COT, int PXT, bool BUF = false>
-__global__ __launch_bounds__(256, (COT * PXT == 2 ? 5 : COT * PXT == 1 ? 6 : 2)) void conv_mfma_f32_streamk_kernel(const ConvArgs a)
+__global__ __launch_bounds__(256, (COT * PXT == 2 ? 3 : COT * PXT == 1 ? 4 : 2)) void conv_mfma_f32_streamk_kernel(const ConvArgs a)
 {
-    __shared__ float lds_a[2][COT * 2 * A_TILE_FLOATS];
+    __shared__ __align__(16) FiltStage<COT> lds_a;
     const int bid = blockIdx.x;
     const int lid = (bid % NUM_XCD) * a.per_xcd + bid / NUM_XCD;      // consecutive runs (the same tiles) on one XCD
     if (lid >= a.sk_chunks) return;
@@ -1586,18 +1676,19 @@ struct PwDwGeom
 };
 
 template <int S, int COT, int CIB, bool RELU = false>
-__global__ __launch_bounds__(256, 2) void conv_pw_dw3x3_f32_kernel(const ConvArgs a, const StemDwArgs d, const PwDwGeom g)
+__global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kernel(const ConvArgs a, const StemDwArgs d, const PwDwGeom g)
 {
     using TL = PwDwTile<S>;
     constexpr int TOH = TL::TOH, TOW = TL::TOW, PW = TL::PW, NPX = TL::NPX;
     constexpr int CG = 32 * COT;                             // channels of the workgroup
     constexpr int MIDP = CG + 4;                             // floats per parked pixel: 16 bytes of padding spread the banks
-    constexpr int NFT = 2 * COT * CIB;                       // 16 x 16 filter tiles of the workgroup
+    constexpr int FILT_BYTES = CIB * COT * 3 * 1024;          // split filter operands: [K-step][channel tile][h, m, l][lane]
     // the filter slice is dead when the K loop ends and the parked tile is born after it: they share their LDS
-    constexpr int MID_FLOATS = 256 * MIDP, FILT_FLOATS = NFT * A_TILE_FLOATS;
+    constexpr int MID_FLOATS = 256 * MIDP, FILT_FLOATS = FILT_BYTES / 4;
     __shared__ __align__(16) float lds[MID_FLOATS > FILT_FLOATS ? MID_FLOATS : FILT_FLOATS];
     __shared__ __align__(16) float s_bias[CG];
-    float *const filt = lds, *const mid = lds;
+    unsigned char *const filt = reinterpret_cast<unsigned char *>(lds);
+    float *const mid = lds;
 
     // logical id = (tile, channel group), the channel group fastest; consecutive logical ids run on one XCD: the channel
     // groups of a tile find its input pixels in that XCD's L2, and so do neighbouring tiles their shared halo
@@ -1616,13 +1707,19 @@ __global__ __launch_bounds__(256, 2) void conv_pw_dw3x3_f32_kernel(const ConvArg
     const float nscale = act_scale(a.act, a.slope);
 
     // ---- requests first: filter slice to LDS, biases, depthwise taps ------------------------------------------------
-    {
-        // the slice is 2 COT consecutive channel blocks of CIB tiles each: contiguous in memory, tile after tile
-        const float *fsrc = a.filt + (size_t)cg * NFT * (CB * CB) + lane * 4;
+    // filter: unit u of 64 COT CIB = (operand u / 64 = K-step and channel tile, lane u % 64) is eight input channels of one
+    // output channel; the thread that loads them splits them once for the whole workgroup
+    constexpr int NU = 64 * COT * CIB, UPT = (NU + 255) / 256;
+    float fraw[UPT][8];
 #pragma unroll
-        for (int t = wave; t < NFT; t += 4)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(fsrc + t * (CB * CB)),
-                                             (__attribute__((address_space(3))) void *)&filt[t * A_TILE_FLOATS], 16, 0, 0);
+    for (int r = 0; r < UPT; ++r)
+    {
+        const int u = tid + r * 256, ul = u & 63, op = u >> 6, us = op / COT, uc = op - us * COT;
+        const int cob = (cg * COT + uc) * 2 + ((ul & 31) >> 4);
+        const float *src = a.filt + ((size_t)cob * CIB + us) * (CB * CB) + (ul >> 5) * 8 * CB + (ul & 15);
+        if (NU % 256 == 0 || u < NU)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) fraw[r][k] = src[k * CB];
     }
     float my_bias = 0.f;
     if (tid < CG && a.bias) my_bias = a.bias[cg * CG + tid];
@@ -1630,14 +1727,6 @@ __global__ __launch_bounds__(256, 2) void conv_pw_dw3x3_f32_kernel(const ConvArg
     constexpr int NQ = CG / 4, TCOLS = S == 1 ? 16 : 8, NRG = 256 / (NQ * TCOLS), RPG = (TOH + NRG - 1) / NRG;
     const int q = tid % NQ, dslot = tid / NQ, dx = dslot % TCOLS, rg = dslot / TCOLS;
     const int dcob = cg * (CG / CB) + q / 4, dq4 = (q & 3) * 4;   // channel block and first channel inside it
-    float4 w[9];
-    {
-        const float4 *wq = reinterpret_cast<const float4 *>(d.dw_filt + (size_t)dcob * (9 * CB) + dq4);
-#pragma unroll
-        for (int t = 0; t < 9; ++t) w[t] = wq[t * 4];
-    }
-    float4 dbias = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (d.dw_bias) dbias = *reinterpret_cast<const float4 *>(d.dw_bias + dcob * CB + dq4);
 
     // ---- pointwise layer on the patch --------------------------------------------------------------------------------
     // this lane's two pixels: patch index p = (2 wave + t) * 32 + col -> position (p / PW, p % PW)
@@ -1668,41 +1757,57 @@ __global__ __launch_bounds__(256, 2) void conv_pw_dw3x3_f32_kernel(const ConvArg
     fetch(0, 0);
     if (CIB > 1) fetch(1, 1);
     if (tid < CG) s_bias[tid] = my_bias;
-    __builtin_amdgcn_s_waitcnt(0x0F70);                      // vmcnt(0): the filter tiles have landed
+#pragma unroll
+    for (int r = 0; r < UPT; ++r)
+    {
+        const int u = tid + r * 256;
+        if (NU % 256 == 0 || u < NU)
+        {
+            const Split8 f = split8(fraw[r]);
+            unsigned char *d = filt + (u >> 6) * 3 * 1024 + (u & 63) * 16;
+            *reinterpret_cast<bf16x8 *>(d) = f.h;
+            *reinterpret_cast<bf16x8 *>(d + 1024) = f.m;
+            *reinterpret_cast<bf16x8 *>(d + 2048) = f.l;
+        }
+    }
     __syncthreads();
 
-    int a_rd[COT];
-#pragma unroll
-    for (int c = 0; c < COT; ++c) a_rd[c] = (c * 2 + (col >> 4)) * CIB * A_TILE_FLOATS + half * 8 * CB + (col & 15);
-    floatx16 acc[COT][2];
+    floatx16 acc[COT][2], sml[COT][2];
 #pragma unroll
     for (int c = 0; c < COT; ++c)
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[c][t][r] = 0.f;
+            for (int r = 0; r < 16; ++r) acc[c][t][r] = sml[c][t][r] = 0.f;
 #pragma unroll
     for (int s = 0; s < CIB; ++s)
     {
-        float A[COT][8];
+        Split8 A[COT], Bs[2];
 #pragma unroll
         for (int c = 0; c < COT; ++c)
+        {
+            const unsigned char *r = filt + (s * COT + c) * 3 * 1024 + lane * 16;
+            A[c].h = *reinterpret_cast<const bf16x8 *>(r);
+            A[c].m = *reinterpret_cast<const bf16x8 *>(r + 1024);
+            A[c].l = *reinterpret_cast<const bf16x8 *>(r + 2048);
+        }
 #pragma unroll
-            for (int kk = 0; kk < 8; ++kk) A[c][kk] = filt[a_rd[c] + s * A_TILE_FLOATS + kk * CB];
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk)
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-            {
-                const float4 bv = B[s & 1][t][kk >> 2];
-                const float b = (kk & 3) == 0 ? bv.x : (kk & 3) == 1 ? bv.y : (kk & 3) == 2 ? bv.z : bv.w;
-#pragma unroll
-                for (int c = 0; c < COT; ++c)
-                    acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(A[c][kk], b, acc[c][t], 0, 0, 0);
-            }
+        for (int t = 0; t < 2; ++t) Bs[t] = split8(B[s & 1][t][0], B[s & 1][t][1]);
+        mfma_split<COT, 2>(acc, sml, A, Bs);
         if (s + 2 < CIB) fetch(s & 1, s + 2);
     }
 
+    // the depthwise taps: requested here (held through the K loop they would cost a workgroup of occupancy), used after the
+    // parked tile's barrier
+    float4 w[9];
+    {
+        const float4 *wq = reinterpret_cast<const float4 *>(d.dw_filt + (size_t)dcob * (9 * CB) + dq4);
+#pragma unroll
+        for (int t = 0; t < 9; ++t) w[t] = wq[t * 4];
+    }
+    float4 dbias = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (d.dw_bias) dbias = *reinterpret_cast<const float4 *>(d.dw_bias + dcob * CB + dq4);
+    split_merge<COT, 2>(acc, sml);
     __syncthreads();                                         // every wave has read its last filter operand
     // ---- bias, activation, park in LDS: a lane holds channels c*32 + 8 qq + 4 half + 0..3 of its pixel -------------
     // pixels outside the pointwise layer's map are the depthwise layer's padding: those lanes store zeros (a branch on
@@ -1807,8 +1912,15 @@ void launch_splitk(ConvArgs &a, hipStream_t s)
     a.n_px_blocks = (a.P + 32 * PXT - 1) / (32 * PXT);
     a.n_blocks = a.n_co_groups * a.n_px_blocks;
     a.per_xcd = (a.n_blocks + NUM_XCD - 1) / NUM_XCD;
+    // the larger operand is the one that an XCD's workgroups share: 1024 -> 1024 3x3 @13x13 at batch 1 (37.7 MB of filter,
+    // 0.7 MB of input) 40.9 -> 38.1 us with the pixel blocks of a channel group on one XCD
+    a.px_first = (long long)a.Co * a.kh * a.kw > (long long)a.batch * a.H * a.W;
     const dim3 grid(a.per_xcd * NUM_XCD, a.slabs > 0 ? a.slabs : 1);
-    if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT, true>), grid, dim3(256), 0, s, a);
+    // eight waves from 64 K-steps on (that layer 48.7 -> 38.1 us, 256 -> 512 3x3 14.9 -> 12.3, 1024 -> 1024 1x1 @7x7 with 64
+    // steps 8.4 -> 7.7); 16 and 32 steps run level or slower with eight, sixteen waves lose to their reduction everywhere
+    const bool eight = a.kh * a.kw * (a.Ci / CB) >= 64;
+    if (buffer_form(a) && eight) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT, true, 8>), grid, dim3(512), 0, s, a);
+    else if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT, true>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT>), grid, dim3(256), 0, s, a);
 }
 
