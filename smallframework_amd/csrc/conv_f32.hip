@@ -42,19 +42,23 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------------------------
-// float32 products on the bf16 matrix pipes.  A float32 number is the exact sum of three bf16 numbers, x = h + m + l with
-// h = bf16(x), m = bf16(x - h), l = x - h - m (24 bits = 3 x 8; round to nearest, so |m| <= 2^-8 |x|, |l| <= 2^-17 |x| and
-// their signs do not follow x's), and a product of two bf16 numbers is exact in float32.  x * y is then added up as
-// hh + (hm + mh + mm + hl + lh); what is left out, ml + lm + ll, is below 2^-24 |x y|, half a unit in the last place of the
-// product.  v_mfma_f32_32x32x16_bf16 multiplies sixteen times as fast as v_mfma_f32_32x32x2_f32, six of them replace
-// eight float32 ones per sixteen channels: 192 matrix cycles instead of 512, and the vector ALU may issue beside them
-// (a float32 MFMA occupies it).
+// float32 products on the bf16 matrix pipes.  A float32 number is the exact sum of three bf16 numbers, x = h + m + l: h is
+// the upper half of x (rounded toward zero, so that the largest finite numbers stay finite), m = bf16(x - h) to nearest,
+// l = x - h - m, at most eight bits (|m| <= 2^-7 |x|, |l| <= 2^-16 |x|, l's sign does not follow x's), and a product of two
+// bf16 numbers is exact in float32.  x * y is then added up as hh + (hm + mh + mm + hl + lh); what is left out, ml + lm + ll, is
+// below 2^-22 |x y|, 2.4e-8 of it root mean square and of either sign.  v_mfma_f32_32x32x16_bf16 multiplies sixteen times as
+// fast as v_mfma_f32_32x32x2_f32, six of them replace eight float32 ones per sixteen channels: 192 matrix cycles instead of
+// 512, and the vector ALU may issue beside them (a float32 MFMA occupies it).
+// The two truncations take the upper halves of a pair in one v_perm_b32 and need no conversion before the subtraction:
+// against all three parts rounded to nearest Tiny-YOLOv2 batch 1 119.2 -> 114.6 us, the 3x3 layer of 96 channels (batch 7,
+// 30x30) 13.0 -> 12.7, large launches the same to 1%.  Subtracting with v_dot2_f32_bf16 (7 instead of 11 instructions a
+// pair) was slower: it does not run beside the MFMAs.
 // hh has an accumulator of its own ("big"): there one addition per sixteen products is rounded where the float32 MFMA
 // chain rounds sixteen, and the small terms are added to a sum of their own size, so that nothing of them is lost
 // against a large total.  Error against float64 (relative 2-norm, K = 16 / 64 / 512 / 2304 / 4608 normal products): the
 // float32 MFMA chain 7.4e-8 / 1.4e-7 / 4.0e-7 / 8.6e-7 / 1.2e-6; see the tests for this form's.
-// Range: |x| below 2^-110 loses bits of m and l (an absolute error of at most 2^-134 |y|); |x| above 3.3895e38 (the
-// largest bf16) counts as infinite.  Infinities and NaN give what float32 products give (split_sum).
+// Range: |x| below 2^-110 loses bits of m and l (an absolute error of at most 2^-134 |y|).  Infinities and NaN give what
+// float32 products give (split_sum); a NaN is one of those with the quiet bit set, the only ones arithmetic produces.
 struct Split8
 {
     bf16x8 h, m, l;      // eight consecutive reduction elements of one row or column: one MFMA operand each
@@ -72,16 +76,20 @@ __device__ __forceinline__ unsigned pack_bf16(float a, float b)
 __device__ __forceinline__ float bf16_lo(unsigned u) { return __builtin_bit_cast(float, u << 16); }
 __device__ __forceinline__ float bf16_hi(unsigned u) { return __builtin_bit_cast(float, u & 0xffff0000u); }
 
+__device__ __forceinline__ unsigned pack_high(float a, float b)       // the upper halves: bf16 numbers rounded toward zero
+{
+    return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x07060302u);
+}
 // a pair of numbers: 11 vector instructions
 __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l)
 {
-    h = pack_bf16(a, b);
-    a -= bf16_lo(h);
-    b -= bf16_hi(h);
+    h = pack_high(a, b);
+    a -= bf16_hi(__builtin_bit_cast(unsigned, a));
+    b -= bf16_hi(__builtin_bit_cast(unsigned, b));
     m = pack_bf16(a, b);
     a -= bf16_lo(m);
     b -= bf16_hi(m);
-    l = pack_bf16(a, b);
+    l = pack_high(a, b);                                                // at most eight bits are left: exact
 }
 __device__ __forceinline__ Split8 split8(const float (&x)[8])
 {

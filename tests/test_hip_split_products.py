@@ -103,3 +103,15 @@ def test_range():
     tiny = x * np.float32(2.0 ** -24) * np.exp2(-np.linspace(0, 200, 32)).astype(np.float32).reshape(1, 1, 4, 8)
     got, _ = run(shape, tiny, f, None, capi.ACT_NONE)
     assert np.abs(got.astype(np.float64) - tiny).max() <= 2.0 ** -133
+
+
+def test_largest_finite_numbers():
+    """The largest float32 numbers (lowest values used as masks among them) stay finite: they have no bf16 neighbour above."""
+    shape = (1, 1, 1, 16, 16, 4, 8)
+    big = np.finfo(np.float32).max
+    x = synth.normal(41, 16 * 32).reshape(1, 16, 4, 8)
+    x[0, 3], x[0, 5, 1], x[0, 6, 2] = big, -big, np.nextafter(big, 0)
+    f = np.zeros((16, 16, 1, 1), np.float32)
+    f[np.arange(16), np.arange(16)] = 0.25
+    got, _ = run(shape, x, f, None, capi.ACT_NONE)
+    assert np.array_equal(got, x * np.float32(0.25))
