@@ -74,6 +74,7 @@ struct QConvArgs
     QOut q;
     int P, S, S_pad, n_co_groups, n_px_blocks, n_blocks, per_xcd;
     double r_howo, r_wo, r_cib, r_kw;   // reciprocals of Ho*Wo, Wo, Ci/16, kw for udiv_rcp
+    FastDiv fd_plane, fd_row, fd_kpt;   // the same for conv_mfma_u8_lds_kernel: Ho*Wo, Wo, K-step pairs per tap
     // grouped convolution: blockIdx.y walks `slabs` (image, group) slabs that lie in_slab / out_slab bytes apart; slab y
     // uses the prepared filter (slab0 + y) % groups, prep_slab bytes apart.  slabs == 0: an ordinary convolution.
     int slabs, groups, slab0;
@@ -380,6 +381,238 @@ __global__ __launch_bounds__(256) void conv_mfma_u8_kernel(const QConvArgs a0)
     }
 }
 
+// ---- larger launches: filter staged through LDS, 32x32x32 tiles ----------------------------------------------------
+// A workgroup's four waves multiply the same CT x 32 output channels, each by its own PXT x 32 pixels.  A K-step pair (two
+// channel blocks of one tap, 32 bytes of the reduction) of the filter is a 1 KiB operand tile per 32 channels, KP pairs are
+// staged at a time (registers -> LDS, double buffered, one barrier per KP pairs).  The activation operand goes from global
+// memory straight to the wave: lane (pixel, half) reads channel block 2 i + half of its pixel, 16 bytes.  An odd number of
+// channel blocks leaves the last pair of a tap half empty.
+// Padded taps take part with the byte -zI, i.e. with (I + zI) = 0, so that the sum needs no correction per border form:
+//   acc = S + ZI * Wtot[co] + ZF * (sum of the valid raw bytes + (ZI - 128) * Ci * nv),   S over ALL taps
+// (the launcher asks for 0 <= -zI <= 255, every zero point a byte can stand for).  A load outside the image returns zero
+// bytes, which the raw sum ignores and a lane's exclusive-or constant (0x80 inside, the padding's signed byte outside) turns
+// into the padding: no instruction per load is spent on the border, and the lane's offset and constant change with the tap only.
+// What bounds it: matrix cycles, eight vector instructions per 16-byte load (raw sum, exclusive or) and about twelve per
+// output value (requantisation), and on small launches the latency of one load per round; the 16x16 tiles above pay for their
+// addresses in every step and read their filter operand once per wave.  96 -> 96 3x3 @30x30 batch 64: 26.9 -> 12.2 us
+// (780 TOP/s), 64 -> 64 @56x56 batch 64 35.1 -> 21.2, 512 -> 512 1x1 @14x14 batch 16 10.9 -> 5.9.
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+template <int CT, int PXT, int KP, bool ODD>
+__global__ __launch_bounds__(256, CT >= 4 ? 2 : 3) void conv_mfma_u8_lds_kernel(const QConvArgs a0)
+{
+    static_assert(CT * KP % 4 == 0, "whole tiles per wave");
+    const QConvArgs a = slab_args(a0);
+    const int bid = blockIdx.x;
+    const int lid = (bid % NUM_XCD) * a.per_xcd + bid / NUM_XCD;
+    if (lid >= a.n_blocks) return;                      // whole workgroup leaves together
+    const int cg = lid % a.n_co_groups;
+    const int pxb = lid / a.n_co_groups;
+
+    __shared__ __align__(16) uint8_t lds_a[2][KP * CT * 1024];
+    __shared__ __align__(16) int32_t s_w[CT * 32];      // ZI * Wtot of the workgroup's channels
+    __shared__ uint8_t post[512];
+    const bool use_post = a.accum_src != nullptr || a.relu;                    // uniform
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 31, half = lane >> 5;
+    const int HoWo = a.Ho * a.Wo;
+    const int CiB = a.Ci / CB, CoB = a.Co / CB;
+    const int KPT = (CiB + 1) >> 1;                     // pairs per tap; ODD: the last one's upper half is empty
+    const int n_kp = a.kh * a.kw * KPT;
+    const int in_blk = a.H * a.W * CB;                  // bytes of a channel block
+
+    unsigned lane_base[PXT], voff[PXT], xk[PXT], sum[PXT];
+    int ih0[PXT], iw0[PXT], rem_of[PXT], n_of[PXT];
+    bool pvalid[PXT];
+#pragma unroll
+    for (int t = 0; t < PXT; ++t)
+    {
+        const int p = ((pxb * 4 + wave) * PXT + t) * 32 + col;
+        pvalid[t] = p < a.P;
+        const int pc = pvalid[t] ? p : 0;
+        const int n = fast_div(pc, a.fd_plane);
+        const int rem = pc - n * HoWo;
+        const int oh = fast_div(rem, a.fd_row);
+        const int ow = rem - oh * a.Wo;
+        ih0[t] = oh * a.stride_h - a.pt;
+        iw0[t] = ow * a.stride - a.pl;
+        lane_base[t] = (unsigned)((n * CiB + half) * in_blk);
+        rem_of[t] = rem;
+        n_of[t] = n;
+        sum[t] = 0;
+    }
+    const unsigned pad_x = (unsigned)(-a.ZI & 0xff) * 0x01010101u;
+    const unsigned half_oor = half ? 0x80000000u : 0u;
+
+    const __amdgpu_buffer_rsrc_t rsrc_in = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(a.in), 0, (int)((size_t)a.batch * CiB * in_blk), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc_f = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t *>(a.ft), 0, (int)((size_t)CoB * a.S_pad * 256), 0x00020000);
+    const unsigned a_voff = (unsigned)(half * 256 + (lane & 15) * 16), a_second = (unsigned)(((lane & 31) >> 4) * a.S_pad * 256);
+
+    // position of the next pair to be requested: pair i of tap (ta, tb)
+    int kp = 0, pi = 0, ta = 0, tb = 0;
+    auto tap_offsets = [&]() {
+        const bool past = ta >= a.kh;                   // requested past the last pair: zeros
+#pragma unroll
+        for (int t = 0; t < PXT; ++t)
+        {
+            const int ih = ih0[t] + ta, iw = iw0[t] + tb;
+            const bool ok = !past && pvalid[t] && (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
+            voff[t] = ok ? lane_base[t] + (unsigned)((ih * a.W + iw) * CB) : 0x80000000u;
+            xk[t] = ok ? 0x80808080u : past ? 0u : pad_x;
+        }
+    };
+    tap_offsets();
+
+    constexpr int AT = CT * KP / 4;                     // filter tiles a wave stages per round
+    auto fetch = [&](v4i (&Av)[AT], v4i (&Bv)[KP][PXT], unsigned (&Xv)[KP][PXT]) {
+#pragma unroll
+        for (int m = 0; m < AT; ++m)
+        {
+            const int i = wave + 4 * m, j = i / CT, c = i - j * CT;
+            const int k = kp + j;
+            // past the last pair: any step, it is multiplied by nothing
+            const int s0 = k < n_kp ? 2 * k - (ODD ? fast_div(k, a.fd_kpt) : 0) : 0;
+            // channel blocks past the last: any other, never stored
+            int cob = (cg * CT + c) * 2;
+            cob = cob < CoB ? cob : 0;
+            Av[m] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                                                rsrc_f, cob + 1 < CoB ? a_voff + a_second : a_voff, (unsigned)((cob * a.S_pad + s0) * 256), 0));
+        }
+#pragma unroll
+        for (int j = 0; j < KP; ++j)
+        {
+            const bool hole = ODD && pi == KPT - 1;     // the upper half has no channel block
+#pragma unroll
+            for (int t = 0; t < PXT; ++t)
+            {
+                Bv[j][t] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                                                       rsrc_in, hole ? voff[t] | half_oor : voff[t], (unsigned)(2 * pi * in_blk), 0));
+                Xv[j][t] = hole && half ? 0u : xk[t];
+            }
+            if (++pi == KPT)
+            {
+                pi = 0;
+                if (++tb == a.kw) { tb = 0; ++ta; }
+                tap_offsets();
+            }
+        }
+        kp += KP;
+    };
+    auto stage = [&](int buf, const v4i (&Av)[AT]) {
+#pragma unroll
+        for (int m = 0; m < AT; ++m)
+            *reinterpret_cast<v4i *>(&lds_a[buf][(wave + 4 * m) * 1024 + lane * 16]) = Av[m];
+    };
+
+    v16i acc[CT][PXT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int t = 0; t < PXT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[c][t][r] = 0;
+
+    auto consume = [&](int buf, const v4i (&Bv)[KP][PXT], const unsigned (&Xv)[KP][PXT]) {
+        v4i A[2][CT];                                   // a pair ahead
+        auto read_a = [&](int j) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) A[j & 1][c] = *reinterpret_cast<const v4i *>(&lds_a[buf][(j * CT + c) * 1024 + lane * 16]);
+        };
+        read_a(0);
+#pragma unroll
+        for (int j = 0; j < KP; ++j)
+        {
+            if (j + 1 < KP) read_a(j + 1);
+            v4i B[PXT];
+#pragma unroll
+            for (int t = 0; t < PXT; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                {
+                    sum[t] = __builtin_amdgcn_sad_u8((unsigned)Bv[j][t][e], 0u, sum[t]);
+                    B[t][e] = (int)((unsigned)Bv[j][t][e] ^ Xv[j][t]);
+                }
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int t = 0; t < PXT; ++t) acc[c][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[j & 1][c], B[t], acc[c][t], 0, 0, 0);
+        }
+    };
+
+    v4i Av[AT], B0[KP][PXT], B1[KP][PXT];
+    unsigned X0[KP][PXT], X1[KP][PXT];
+    fetch(Av, B0, X0);
+    // channel constants and the post-op table while the first loads are in flight
+    if (threadIdx.x < CT * 32)
+    {
+        const int co = cg * CT * 32 + threadIdx.x;
+        s_w[threadIdx.x] = co < a.Co ? (int32_t)((uint32_t)a.ZI * (uint32_t)a.wpre[(size_t)((a.kh + 1) * (a.kw + 1) - 1) * a.Co + co]) : 0;
+    }
+    if (use_post) build_post_table(post, PostArgs{a.accum_src != nullptr, a.relu, a.zS, a.zO, a.q});
+    stage(0, Av);
+    fetch(Av, B1, X1);
+    __syncthreads();
+    const int rounds = (n_kp + KP - 1) / KP;
+    for (int it = 0; it < rounds >> 1; ++it)
+    {
+        consume(0, B0, X0);
+        stage(1, Av);
+        fetch(Av, B0, X0);
+        __syncthreads();
+        consume(1, B1, X1);
+        stage(0, Av);
+        fetch(Av, B1, X1);
+        __syncthreads();
+    }
+    if (rounds & 1) consume(0, B0, X0);
+
+    // ---- epilogue: a lane holds channels 8 q + 4 half + {0..3} of its pixel in registers 4 q .. 4 q + 3 of a tile -----------
+#pragma unroll
+    for (int t = 0; t < PXT; ++t)
+    {
+        const unsigned si = sum[t] + (unsigned)__shfl_xor((int)sum[t], 32);
+        int a_lo = ih0[t] < 0 ? -ih0[t] : 0, b_lo = iw0[t] < 0 ? -iw0[t] : 0;
+        int a_hi = (a.H - ih0[t]) < a.kh ? (a.H - ih0[t]) : a.kh, b_hi = (a.W - iw0[t]) < a.kw ? (a.W - iw0[t]) : a.kw;
+        a_hi = a_hi > a_lo ? a_hi : a_lo;
+        b_hi = b_hi > b_lo ? b_hi : b_lo;
+        const unsigned nv = (unsigned)((a_hi - a_lo) * (b_hi - b_lo));
+        const unsigned base = (unsigned)a.ZF * (si + (unsigned)(a.ZI - 128) * (unsigned)a.Ci * nv);
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+        {
+            const int cob0 = (cg * CT + c) * 2;                             // uniform
+            if (cob0 >= CoB) continue;
+            uint8_t *o = a.out + (((size_t)n_of[t] * CoB + cob0) * HoWo + rem_of[t]) * CB;
+            unsigned pk[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+            {
+                const int4 w = *reinterpret_cast<const int4 *>(&s_w[c * 32 + 8 * q + 4 * half]);
+                const int w4[4] = {w.x, w.y, w.z, w.w};
+                unsigned sc = 0;
+                if (a.accum_src && pvalid[t] && cob0 + (q >> 1) < CoB)
+                    sc = *reinterpret_cast<const unsigned *>(a.accum_src + (o - a.out) + (size_t)(q >> 1) * HoWo * CB + 8 * (q & 1) + 4 * half);
+                pk[q] = 0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                {
+                    unsigned y = requant_u8_fast((int32_t)((unsigned)acc[c][t][4 * q + r] + base + (unsigned)w4[r]), a.q);
+                    if (use_post) y = post[y + ((sc >> (8 * r)) & 0xffu)];  // sc is 0 without Accum
+                    pk[q] |= y << (8 * r);
+                }
+            }
+            // the two halves of a pixel trade quads: the lower one stores channel block cob0, the upper one cob0 + 1, 16 bytes each
+            const unsigned x0 = (unsigned)__shfl_xor((int)(half ? pk[0] : pk[2]), 32), x1 = (unsigned)__shfl_xor((int)(half ? pk[1] : pk[3]), 32);
+            const uint4 v = half ? make_uint4(x0, pk[2], x1, pk[3]) : make_uint4(pk[0], x0, pk[1], x1);
+            if (pvalid[t] && cob0 + half < CoB) *reinterpret_cast<uint4 *>(o + (size_t)half * HoWo * CB) = v;
+        }
+    }
+}
+
 // ---- first layers (Ci in {1,2,3}): vector ALU, direct (I + zI) * (F + zF) ----------------------------
 struct QSmallArgs
 {
@@ -512,6 +745,21 @@ void launch_q(QConvArgs &a, hipStream_t s)
     a.per_xcd = (a.n_blocks + NUM_XCD - 1) / NUM_XCD;
     a.use_table = a.n_blocks >= table_min_wg();
     hipLaunchKernelGGL((conv_mfma_u8_kernel<COT, PXT>), dim3(a.per_xcd * NUM_XCD, a.slabs > 0 ? a.slabs : 1), dim3(256), 0, s, a);
+}
+
+template <int CT, int PXT, int KP>
+void launch_q_lds(QConvArgs &a, hipStream_t s)
+{
+    a.n_co_groups = (a.Co + 32 * CT - 1) / (32 * CT);
+    a.n_px_blocks = (a.P + 32 * PXT * 4 - 1) / (32 * PXT * 4);
+    a.n_blocks = a.n_co_groups * a.n_px_blocks;
+    a.per_xcd = (a.n_blocks + NUM_XCD - 1) / NUM_XCD;
+    a.fd_plane = make_fast_div((unsigned)(a.Ho * a.Wo));
+    a.fd_row = make_fast_div((unsigned)a.Wo);
+    a.fd_kpt = make_fast_div((unsigned)((a.Ci / CB + 1) / 2));
+    const dim3 grid(a.per_xcd * NUM_XCD, a.slabs > 0 ? a.slabs : 1);
+    if ((a.Ci / CB) & 1) hipLaunchKernelGGL((conv_mfma_u8_lds_kernel<CT, PXT, KP, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((conv_mfma_u8_lds_kernel<CT, PXT, KP, false>), grid, dim3(256), 0, s, a);
 }
 
 int conv_u8_check(const char *op, int batch, int kh, int kw, int stride, int pt, int pb, int pl, int pr, int Co,
@@ -664,7 +912,39 @@ int conv_u8_run(const char *op, int batch, int kh, int kw, int stride, int pt, i
     // comes before operand re-use.
     static const long want = tune_int("convq_min_wg", 512);
     auto nwg = [&](int cot, int pxt) { return (long)((CoB + cot - 1) / cot) * ((P + 64 * pxt - 1) / (64 * pxt)) * n_slabs; };
-    if (CoB % 4 == 0 && nwg(4, 2) >= want) launch_q<4, 2>(a, s);
+    // The LDS form takes buffer offsets (tensors of at most 1 GiB), a zero point that is minus a byte and the short form of the
+    // requantisation.  Half-empty operand tiles (an odd number of channel blocks on either side) cost it up to half or
+    // three quarters of its products: below 70% used it needs a full chip (48 -> 48 3x3 @20x20 batch 3, 56%: 5.1 us on the
+    // kernel above, 5.9 on this; 16 -> 176 5x5 @50x50 batch 20, 46%: 32.8 and 22.1), 16 -> 16 channels never pay (5.7, 6.4).
+    // A few workgroups with a short reduction are a matter of latency (64 -> 128 3x3 @20x20 batch 2, 28 workgroups of 18 pairs:
+    // 4.9 us above, 5.4 here; 1024 -> 64 1x1 @40x40 batch 2, 26 of 32 pairs: 6.5 and 6.2).
+    // Channels per workgroup: fewer products on channels that do not exist, then more tiles per activation read (a
+    // tile's own work is about twice the overhead of a pair), from 1.5 workgroups per compute unit on: 96 -> 96 3x3
+    // @30x30 batch 64 26.9 us on the kernel above, 15.0 / 16.5 / 12.2 with 32 / 64 / 96 channels; batch 7 8.2, 6.1 / 7.4 / 8.9;
+    // 256 -> 256 @14x14 batch 64 34.8, 20.2 / 16.3 / 19.0.  Two pixel tiles a wave only pay with 128 channels and a long
+    // reduction on a full chip (256 -> 256 3x3 @56x56 batch 16: 71.3, 47.4 with one tile, 40.5 with two).
+    const int CoP = (CoB + 1) / 2, KPT = (CiB + 1) / 2;
+    auto nwg_lds = [&](int ct, int pxt) { return (long)((CoP + ct - 1) / ct) * ((P + 128 * pxt - 1) / (128 * pxt)) * n_slabs; };
+    const double used = (double)CoB / (2 * CoP) * CiB / (2 * KPT);
+    constexpr long FULL = 3 * NUM_CU / 2;
+    if (a.q.fast && iq->zero <= 0 && iq->zero >= -255 && (long long)batch * Ci * H * W <= (1ll << 30) &&
+        (long long)Co * a.S_pad * 16 <= (1ll << 30) && (used >= 0.7 || (used >= 0.45 && nwg_lds(1, 1) >= FULL)) &&
+        (nwg_lds(1, 1) >= 64 || taps * KPT >= 24))
+    {
+        int ct = 1;
+        double best = 0;
+        for (int c = 1; c <= 4; ++c)
+        {
+            const double cost = (CoP + c - 1) / c * (c + 0.5);
+            if (c == 1 || (cost < best && nwg_lds(c, 1) >= FULL)) { ct = c; best = cost; }
+        }
+        if (ct == 4 && nwg_lds(4, 2) >= FULL && taps * KPT >= 32) launch_q_lds<4, 2, 2>(a, s);
+        else if (ct == 4) launch_q_lds<4, 1, 4>(a, s);
+        else if (ct == 3) launch_q_lds<3, 1, 4>(a, s);
+        else if (ct == 2) launch_q_lds<2, 1, 4>(a, s);
+        else launch_q_lds<1, 1, 4>(a, s);
+    }
+    else if (CoB % 4 == 0 && nwg(4, 2) >= want) launch_q<4, 2>(a, s);
     else if (CoB % 2 == 0 && nwg(2, 2) >= want) launch_q<2, 2>(a, s);
     else if (nwg(1, 2) >= want) launch_q<1, 2>(a, s);
     else launch_q<1, 1>(a, s);

@@ -42,6 +42,17 @@ __host__ __device__ __forceinline__ int32_t requant_i32(int32_t acc, const QOut 
     return (v >> rs) + ((mod > threshold) ? -1 : 0);
 }
 
+// The short form of requant_u8 below, for q.fast only; a non-positive accumulator counts as 0, which gives 0.
+__host__ __device__ __forceinline__ uint32_t requant_u8_fast(int32_t acc, const QOut q)
+{
+    int32_t shifted = (int32_t)((uint32_t)acc << (q.lshift & 31));
+    shifted = shifted > 0 ? shifted : 0;
+    const uint32_t v = (uint32_t)(((uint64_t)(uint32_t)shifted * (uint64_t)(uint32_t)q.multiplier + (1ull << 30)) >> 31);
+    const uint32_t round_bit = (v >> ((q.rshift - 1) & 31)) & (q.rshift > 0 ? 1u : 0u);
+    const int32_t r = (int32_t)(v >> q.rshift) - (int32_t)round_bit;   // -1 is possible
+    return (uint32_t)(r < 0 ? 0 : (r > 255 ? 255 : r));
+}
+
 // requant_i32 clamped to 0..255.  With a positive multiplier (every practical scale) the clamp makes
 // most of the general form redundant, and the short form below returns the same byte:
 //   - a non-positive (shifted) accumulator gives a product <= 0, VQRDMULH then returns v <= 0, the
