@@ -747,16 +747,19 @@ __global__ __launch_bounds__(256, (COT * PXT == 2 ? 3 : COT * PXT == 1 ? 4 : 2))
 // ---------------------------------------------------------------------------------------------
 // Small outputs (few 32x32 tiles per SIMD: fully connected layers, 7x7 / 13x13 feature maps,
 // batch 1): the W waves of a workgroup take the SAME output tile and an equal share of the K-steps
-// each, then the others hand their partial accumulators to wave 0 through LDS, which adds them in
-// wave order (deterministic) and runs the epilogue.  Operands go straight from global
+// each, then all hand their partial accumulators over through LDS; each of the first waves adds up one register quad of
+// the tile in wave order (deterministic) and finishes it.  Operands go straight from global
 // memory to the wave's registers (nothing is shared between the waves until the reduction).  Both operands are split for
-// one tile, 88 vector instructions (352 cycles) against 192 matrix cycles per K-step: what bounds the long reductions.
+// one tile, 88 vector instructions (about 400 cycles) against 192 matrix cycles per K-step, and the two add up: what bounds
+// the long reductions; the short ones are a launch, a few load latencies and the reduction.  Added up and stored by wave 0
+// alone: 512 -> 512 1x1 @14x14 batch 1 6.4 us, 5.8 now; 128 -> 256 3x3 @26x26 8.8, 7.9; 1024 -> 1024 3x3 @13x13 39.7, 39.6.
+// Three more K-steps in flight (172 registers) were 2 to 8% slower, two channel tiles a wave leave compute units idle (68 us).
 // POOL: the 32-pixel tiles are the pooling form's groups of 8 windows and the epilogue pools (pool_tile_pixel)
 // BUF: operands through buffer loads, as in conv_lds_tile (each wave has its own K range, so its window position and
 // scalar offsets are the wave's)
 // W: waves of the workgroup, each with its share of the K-steps
 template <int COT, int PXT, bool POOL = false, bool BUF = false, int W = 4>
-__device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)[W - 1][COT * PXT][16][64],
+__device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red)[W][COT * PXT * 4][64],
                                                  const int cg, const int pxb)
 {
     const int lane = threadIdx.x & 63;
@@ -918,6 +921,13 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)
         mfma_split<COT, PXT>(acc, sml, As, Bs);
     };
 
+    // the register quad that this wave finishes (tile, four of its channels): its bias is requested before the K loop
+    constexpr int QUADS = COT * PXT * 4;
+    static_assert(QUADS <= W, "one quad per wave");
+    const int my_t = wave / 4 % PXT, my_co4 = (cg * COT + wave / (4 * PXT)) * 32 + 8 * (wave % 4) + 4 * half;
+    float4 my_bias = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (a.bias && wave < QUADS && my_co4 < a.Co) my_bias = *reinterpret_cast<const float4 *>(a.bias + my_co4);
+
     float A0[COT][8], A1[COT][8];
     float4 B0[PXT][2], B1[PXT][2];
     load_step(A0, B0);
@@ -931,37 +941,67 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float (&red)
     }
 
     split_merge<COT, PXT>(acc, sml);
-    // ---- reduction over the waves
-    if (wave > 0)
+    // ---- reduction over the waves: wave w adds up register quad w of all waves, in wave order, and finishes it
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i)
     {
-#pragma unroll
-        for (int c = 0; c < COT; ++c)
-#pragma unroll
-            for (int t = 0; t < PXT; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) red[wave - 1][c * PXT + t][r][lane] = acc[c][t][r];
+        const floatx16 &v = acc[i / (4 * PXT)][i / 4 % PXT];
+        red[wave][i][lane] = make_float4(v[4 * (i % 4)], v[4 * (i % 4) + 1], v[4 * (i % 4) + 2], v[4 * (i % 4) + 3]);
     }
     __syncthreads();
-    if (wave == 0)
+    if (wave >= QUADS) return;
+    float4 v = red[0][wave][lane];
+#pragma unroll
+    for (int w = 1; w < W; ++w)
     {
-#pragma unroll
-        for (int w = 0; w < W - 1; ++w)
-#pragma unroll
-            for (int c = 0; c < COT; ++c)
-#pragma unroll
-                for (int t = 0; t < PXT; ++t)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[c][t][r] += red[w][c * PXT + t][r][lane];
-        if (POOL) conv_epilogue_pool<COT, PXT>(a, acc, cg, half, pool_ok, out_pix);
-        else conv_epilogue<COT, PXT>(a, acc, cg, half, HoWo, pvalid, out_pix);
+        const float4 u = red[w][wave][lane];
+        v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
     }
+    const float nscale = act_scale(a.act, a.slope);
+    bool ok = my_co4 < a.Co && (POOL ? pool_ok[0] : pvalid[0]);
+    size_t pix = out_pix[0];
+    if (PXT == 2 && my_t == 1) { ok = my_co4 < a.Co && (POOL ? pool_ok[PXT - 1] : pvalid[PXT - 1]); pix = out_pix[PXT - 1]; }
+    if (POOL)
+    {
+        const float b4[4] = {my_bias.x, my_bias.y, my_bias.z, my_bias.w}, v4[4] = {v.x, v.y, v.z, v.w};
+        float m[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+        {
+            float x = act_bf(v4[e] + b4[e], nscale);
+            const float u = __shfl_xor(x, 1, WAVE);
+            x = x > u ? x : u;
+            const float y = __shfl_xor(x, 2, WAVE);
+            m[e] = x > y ? x : y;
+        }
+        if (ok) *reinterpret_cast<float4 *>(a.out + pix + (size_t)(my_co4 / CB) * ((a.Ho >> 1) * (a.Wo >> 1)) * CB + my_co4 % CB) =
+                    make_float4(m[0], m[1], m[2], m[3]);
+        return;
+    }
+    float4 *o = reinterpret_cast<float4 *>(a.out + pix + (size_t)(my_co4 / CB) * HoWo * CB + my_co4 % CB);
+    if (!ok) return;
+    if (a.accumulate)
+    {
+        const float4 old = *o;
+        v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
+    }
+    v.x += my_bias.x; v.y += my_bias.y; v.z += my_bias.z; v.w += my_bias.w;
+    if (a.act == SMALL_HIP_ACT_RELU && !a.accumulate)        // as conv_epilogue: a NaN becomes 0
+    {
+        v.x = act_k<true>(v.x, nscale); v.y = act_k<true>(v.y, nscale); v.z = act_k<true>(v.z, nscale); v.w = act_k<true>(v.w, nscale);
+    }
+    else
+    {
+        v.x = act_bf(v.x, nscale); v.y = act_bf(v.y, nscale); v.z = act_bf(v.z, nscale); v.w = act_bf(v.w, nscale);
+    }
+    *o = v;
 }
 
 template <int COT, int PXT, bool BUF = false, int W = 4>
 __global__ __launch_bounds__(64 * W) void conv_mfma_f32_splitk_kernel(const ConvArgs a0)
 {
     const ConvArgs a = slab_args(a0);
-    __shared__ float red[W - 1][COT * PXT][16][64];
+    __shared__ float4 red[W][COT * PXT * 4][64];
     const int bid = blockIdx.x;
     const int lid = (bid % NUM_XCD) * a.per_xcd + bid / NUM_XCD;
     if (lid >= a.n_blocks) return;
@@ -983,7 +1023,7 @@ __global__ __launch_bounds__(256, (COT * PXT == 2 ? 3 : COT * PXT == 1 ? 4 : 2))
 {
     const ConvArgs a = slab_args(a0);
     __shared__ __align__(16) FiltStage<COT> lds_a;
-    __shared__ float red[3][1][16][64];
+    __shared__ float4 red[4][4][64];
     const int bid = blockIdx.x;
     if (bid < a.n_main)
     {
