@@ -418,6 +418,7 @@ class HipExecutor:
             self.plan.append((at(op), at(acc_op) if acc_op else None, relu))
             i = j
         self.out_name = phys.get(model.out, model.out)
+        self.calls = [(self._call_of(entry), entry) for entry in self.plan]
         torch.cuda.synchronize()
 
     @staticmethod
@@ -472,23 +473,13 @@ class HipExecutor:
     def run_entry(self, entry, st):
         """One launch of the plan: a single op, or a fused group."""
         op, acc_op, relu = entry
-        if acc_op is not None and acc_op.kind == "maxpool":
-            self.run_conv_pool_f32(op, acc_op, st)
-        elif acc_op is not None and acc_op.kind == "dw":
-            self.run_conv_dw_f32(op, acc_op, st)
+        call = self._call_of(entry)
+        if call is not None:
+            self._issue(call, st)
         elif acc_op is not None or relu:
             self.run_fused_u8(op, acc_op, relu, st)
         else:
             self.run_op(op, st)
-
-    def run_conv_pool_f32(self, op, pool, st):
-        """Conv2D + activation + MaxPool2D 2x2 stride 2 in one launch."""
-        L, p, b = self.lib, self._p, self.buf
-        act = {None: capi.ACT_NONE, "relu": capi.ACT_RELU, "leaky": capi.ACT_LEAKY}[op.act]
-        t_, b_, l_, r_ = op.pads
-        capi.check(L.small_hip_conv2d_bias_act_maxpool2d_f32(
-            self.batch, op.kh, op.kw, op.stride, t_, b_, l_, r_, 2, 2, 2, 0, 0, 0, 0, op.Co, op.C, op.H, op.W,
-            p(b[op.src]), p(self.w[op.weight]), None, act, op.slope, p(b[pool.dst]), st))
 
     @staticmethod
     def _first_layer_dw(op, dw):
@@ -516,38 +507,61 @@ class HipExecutor:
         fill = hd * wd / float(-(-hd // toh) * toh * -(-wd // tow) * tow)
         return fill >= 0.7
 
-    def run_conv_dw_f32(self, op, dw, st):
-        """Conv2D + activation + DepthwiseConv2D 3x3 + activation in one launch."""
-        L, p, b = self.lib, self._p, self.buf
+    def _call_of(self, entry):
+        """What a launch of the fused float32 plan passes to the library besides the addresses: (function, leading sizes,
+        source buffer, weight names (None: no bias), trailing scalars, destination buffer).  Put together once: the launches of
+        a batch-1 pass are as long as the host takes to issue them (MobileNetV1: 25 launches, 143 us a pass against 129 on the GPU).
+        None for what run_op / run_fused_u8 issue."""
+        op, second, _ = entry
+        if not self.fused or self.model.dtype != "f32" or op.kind not in ("conv", "dw", "dense", "maxpool", "avgpool"):
+            return None
+        L, B = self.lib, self.batch
         act = {None: capi.ACT_NONE, "relu": capi.ACT_RELU, "leaky": capi.ACT_LEAKY}[op.act]
-        t_, b_, l_, r_ = op.pads
-        dt, db, dl, dr = dw.pads
-        capi.check(L.small_hip_conv2d_bias_act_dwconv2d_bias_act_f32(
-            self.batch, op.kh, op.kw, op.stride, t_, b_, l_, r_, 3, 3, dw.stride, dt, db, dl, dr, op.Co, op.C, op.H, op.W,
-            p(b[op.src]), p(self.w[op.weight]), None, p(self.w[dw.weight]), None, act, op.slope, p(b[dw.dst]), st))
+        window = (B, op.kh, op.kw, op.stride) + tuple(op.pads)
+        if op.kind == "dense":
+            return L.small_hip_dense_f32, (B, op.Co, op.C), op.src, (op.weight,), (), op.dst
+        if op.kind in ("maxpool", "avgpool"):
+            fn = L.small_hip_maxpool2d_f32 if op.kind == "maxpool" else L.small_hip_avgpool2d_f32
+            return fn, window + (op.C, op.H, op.W), op.src, (), (), op.dst
+        if op.kind == "dw":
+            return L.small_hip_depthwise_conv2d_bias_act_f32, window + (op.C, op.H, op.W), op.src, (op.weight, None), (act, op.slope), op.dst
+        sizes = (op.Co, op.C, op.H, op.W)
+        if second is None:
+            return L.small_hip_conv2d_bias_act_f32, window + sizes, op.src, (op.weight, None), (act, op.slope), op.dst
+        if second.kind == "maxpool":             # Conv2D + activation + MaxPool2D 2x2 stride 2 in one launch
+            return (L.small_hip_conv2d_bias_act_maxpool2d_f32, window + (2, 2, 2, 0, 0, 0, 0) + sizes, op.src, (op.weight, None),
+                    (act, op.slope), second.dst)
+        # Conv2D + activation + DepthwiseConv2D 3x3 + activation in one launch
+        return (L.small_hip_conv2d_bias_act_dwconv2d_bias_act_f32, window + (3, 3, second.stride) + tuple(second.pads) + sizes, op.src,
+                (op.weight, None, second.weight, None), (act, op.slope), second.dst)
+
+    def _issue(self, call, st):
+        """The buffers and weights are looked up at every launch: a caller may put another tensor into `buf` or `w`."""
+        fn, head, src, weights, tail, dst = call
+        w = [None if k is None else self.w[k].data_ptr() for k in weights]
+        rc = fn(*head, self.buf[src].data_ptr(), *w, *tail, self.buf[dst].data_ptr(), st)
+        if rc:
+            capi.check(rc)
 
     def run_op(self, op: Op, st):
+        call = self._call_of((op, None, False))
+        if call is not None:
+            self._issue(call, st)
+            return
         L, p, B, b = self.lib, self._p, self.batch, self.buf
         src, dst = b[op.src], b[op.dst]
-        act = {None: capi.ACT_NONE, "relu": capi.ACT_RELU, "leaky": capi.ACT_LEAKY}[op.act]
         t_, b_, l_, r_ = op.pads
         if self.model.dtype == "f32":
             if op.kind == "conv":
                 args = (B, op.kh, op.kw, op.stride, t_, b_, l_, r_, op.Co, op.C, op.H, op.W)
-                if self.fused:
-                    rc = L.small_hip_conv2d_bias_act_f32(*args, p(src), p(self.w[op.weight]), None, act, op.slope, p(dst), st)
-                else:
-                    rc = L.small_hip_conv2d_f32(*args, p(src), p(self.w[op.weight]), p(dst), st)
-                    rc = rc or self._act_f32(op, dst, st)
+                rc = L.small_hip_conv2d_f32(*args, p(src), p(self.w[op.weight]), p(dst), st)
+                rc = rc or self._act_f32(op, dst, st)
             elif op.kind == "dense":
                 rc = L.small_hip_dense_f32(B, op.Co, op.C, p(src), p(self.w[op.weight]), p(dst), st)
             elif op.kind == "dw":
                 args = (B, op.kh, op.kw, op.stride, t_, b_, l_, r_, op.C, op.H, op.W)
-                if self.fused:
-                    rc = L.small_hip_depthwise_conv2d_bias_act_f32(*args, p(src), p(self.w[op.weight]), None, act, op.slope, p(dst), st)
-                else:
-                    rc = L.small_hip_depthwise_conv2d_f32(*args, p(src), p(self.w[op.weight]), p(dst), st)
-                    rc = rc or self._act_f32(op, dst, st)
+                rc = L.small_hip_depthwise_conv2d_f32(*args, p(src), p(self.w[op.weight]), p(dst), st)
+                rc = rc or self._act_f32(op, dst, st)
             elif op.kind in ("maxpool", "avgpool"):
                 fn = L.small_hip_maxpool2d_f32 if op.kind == "maxpool" else L.small_hip_avgpool2d_f32
                 rc = fn(B, op.kh, op.kw, op.stride, t_, b_, l_, r_, op.C, op.H, op.W, p(src), p(dst), st)
@@ -594,8 +608,11 @@ class HipExecutor:
 
     def forward(self):
         st = self.stream()
-        for entry in self.plan:
-            self.run_entry(entry, st)
+        for call, entry in self.calls:
+            if call is not None:
+                self._issue(call, st)
+            else:
+                self.run_entry(entry, st)
 
     # ---- the whole model in one launch (uint8 models whose tensors and filters fit one CU's LDS) --------------
     def qmodel_layers(self):
