@@ -1991,6 +1991,26 @@ bool tail_pays(int n_main, int rest, int nsteps)
     return knob == 2 || rest <= 11 * NUM_CU / 16;
 }
 
+// Wave tile in 32-channel x 32-pixel MFMA tiles.  The split of the operands is what a larger tile saves: one pixel tile split
+// for two channel tiles, or one filter tile for two pixel tiles.
+//   2x2  from 16 tiles per SIMD and 32 K-steps with whole pairs of channel tiles (256 -> 256 3x3 @56x56 batch 64: 1160 us, 2x1 1257).
+//   2x1  from 2.25 tiles per SIMD (2 with 72 K-steps; below, the balance of few tiles counts more): 1024 -> 1024 1x1 @7x7 batch 64
+//        (3.1 tiles) 57.3 -> 47.2 us, 512 -> 512 1x1 @14x14 batch 24 (2.3) 21.6 -> 20.4, batch 16 (1.5) 15.2 -> 17.4; where an odd
+//        last channel tile costs at most a tenth (208 channels @21x27 batch 40 75.3 -> 69.3), or a fifth from 16 K-steps on (160
+//        channels 3x3 50.1 -> 47.2, 1x1 of 64 channels 15.0 -> 16.3).
+//   1x2  otherwise from 4 tiles per SIMD and 16 K-steps (96 channels 3x3 @30x30 batch 64 71.0 -> 68.2, batch 16 (1.3) 23.5 -> 25.1,
+//        32 channels @56x56 31.4 -> 29.2).
+inline void wave_tile(int Co, long tiles32, int nsteps, int *cot, int *pxt)
+{
+    const long simds = 4L * NUM_CU;
+    const int c32 = (Co + 31) / 32, pairs = (c32 + 1) / 2;
+    const bool little = 20 * pairs <= 11 * c32 || (5 * pairs <= 3 * c32 && nsteps >= 16);   // channel tiles that do not exist
+    *cot = *pxt = 1;
+    if (Co % 64 == 0 && tiles32 >= 16 * simds && nsteps >= 32) *cot = *pxt = 2;
+    else if (little && (4 * tiles32 >= 9 * simds || (tiles32 >= 2 * simds && nsteps >= 72))) *cot = 2;
+    else if (tiles32 >= 4 * simds && nsteps >= 16) *pxt = 2;
+}
+
 template <int COT, int PXT>
 void launch_mfma(ConvArgs &a, hipStream_t s)
 {
@@ -2186,16 +2206,10 @@ int conv_f32(const char *op, int batch, int kh, int kw, int stride, int pt, int 
         return SMALL_HIP_OK;
     }
 
-    // Wave tile (in 32-channel x 32-pixel MFMA tiles).  Measured on MI355X inside whole-model runs with
-    // the balanced tail in place: 2x2 only pays with many tiles per SIMD and a long reduction (big
-    // 3x3 layers), 2x1 from 4 tiles per SIMD (from 2 when the reduction has at least 72 steps: 128->256 3x3 @26x26 b16, 2.6 tiles per SIMD, 74 -> 69 us; 1024->1024 1x1 @7x7 b64 with 64 steps stays 1x1: 69 against 73 us), 1x1 below (few tiles: balance matters more than
-    // operand re-use).
     const long tiles32 = (long)((Co + 31) / 32) * ((P + 31) / 32) * (grp.slabs > 0 ? grp.slabs : 1);
-    const long simds = 4L * NUM_CU;
     const int nsteps = kh * kw * (Ci / CB);
-    int cot = 1, pxt = 1;
-    if (Co % 64 == 0 && tiles32 >= 16 * simds && nsteps >= 32) { cot = 2; pxt = 2; }
-    else if (Co % 64 == 0 && (tiles32 >= 4 * simds || (tiles32 >= 2 * simds && nsteps >= 72))) { cot = 2; pxt = 1; }
+    int cot, pxt;
+    wave_tile(Co, tiles32, nsteps, &cot, &pxt);
     if (wants_splitk(tiles32, nsteps))
     {
         launch_splitk<1, 1>(a, s);
@@ -2306,10 +2320,11 @@ int conv_pool_f32(const char *op, int batch, int kh, int kw, int stride, int pt,
     a.P = (int)(nwin * 4);
     const long ntiles = (nwin + 7) / 8;
     const long tiles32 = (long)((Co + 31) / 32) * ntiles;
-    const long simds = 4L * NUM_CU;
-    const int nsteps = kh * kw * (Ci / CB);
-    if (Co % 64 == 0 && tiles32 >= 16 * simds && nsteps >= 32) launch_mfma_pool<2, 2>(a, s);
-    else if (Co % 64 == 0 && tiles32 >= 4 * simds) launch_mfma_pool<2, 1>(a, s);
+    int cot, pxt;
+    wave_tile(Co, tiles32, kh * kw * (Ci / CB), &cot, &pxt);
+    if (cot == 2 && pxt == 2) launch_mfma_pool<2, 2>(a, s);
+    else if (cot == 2) launch_mfma_pool<2, 1>(a, s);
+    else if (pxt == 2) launch_mfma_pool<1, 2>(a, s);
     else launch_mfma_pool<1, 1>(a, s);
     SHP_LAUNCH_CHECK(op);
     return SMALL_HIP_OK;

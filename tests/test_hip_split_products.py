@@ -54,6 +54,10 @@ SHAPES = [  # batch, window, stride, Co, Ci, H, W
     (16, 3, 1, 128, 64, 52, 52),      # cut tail
     (8, 3, 1, 512, 160, 13, 13),      # equal shares of the reduction
     (56, 3, 1, 128, 64, 56, 56),      # 2 x 2 tiles
+    (40, 1, 1, 48, 64, 31, 31),       # pairs of channel tiles with a last tile that is half there
+    (20, 3, 1, 208, 48, 23, 25),      # ... that is not there, ragged channels
+    (50, 3, 1, 96, 32, 30, 30),       # one channel tile, two pixel tiles a wave
+    (13, 3, 1, 32, 32, 105, 103),     # the same with one channel tile in all, odd map
 ]
 
 
