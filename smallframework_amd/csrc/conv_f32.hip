@@ -1965,9 +1965,12 @@ void launch_splitk(ConvArgs &a, hipStream_t s)
     a.px_first = (long long)a.Co * a.kh * a.kw > (long long)a.batch * a.H * a.W;
     const dim3 grid(a.per_xcd * NUM_XCD, a.slabs > 0 ? a.slabs : 1);
     // eight waves from 64 K-steps on (that layer 48.7 -> 38.1 us, 256 -> 512 3x3 14.9 -> 12.3, 1024 -> 1024 1x1 @7x7 with 64
-    // steps 8.4 -> 7.7); 16 and 32 steps run level or slower with eight, sixteen waves lose to their reduction everywhere
+    // steps 8.4 -> 7.7), 16 and 32 steps run level or slower with eight; sixteen from 256 steps on where a compute unit has one
+    // workgroup at most (that layer, 576 steps, 38.2 -> 36.3, 512 -> 1024 20.6 -> 19.7; 144 steps 11.0 -> 11.4, 64 steps 10.4 -> 12.7)
     const bool eight = a.kh * a.kw * (a.Ci / CB) >= 64;
-    if (buffer_form(a) && eight) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT, true, 8>), grid, dim3(512), 0, s, a);
+    const bool sixteen = a.kh * a.kw * (a.Ci / CB) >= 256 && a.n_blocks <= NUM_CU && a.slabs == 0;
+    if (buffer_form(a) && sixteen) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT, true, 16>), grid, dim3(1024), 0, s, a);
+    else if (buffer_form(a) && eight) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT, true, 8>), grid, dim3(512), 0, s, a);
     else if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT, true>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT>), grid, dim3(256), 0, s, a);
 }

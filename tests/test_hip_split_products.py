@@ -46,6 +46,7 @@ SHAPES = [  # batch, window, stride, Co, Ci, H, W
     (1, 3, 1, 32, 16, 9, 11),         # 9 steps: odd
     (1, 3, 2, 80, 48, 17, 13),        # split K over four waves, ragged channels
     (1, 3, 1, 96, 128, 13, 13),       # 72 steps: split K over eight waves
+    (1, 3, 1, 48, 464, 6, 7),         # 261 steps: sixteen waves, uneven shares
     (1, 5, 1, 16, 48, 12, 12),        # 75 steps: an uneven share per wave
     (6, 1, 1, 128, 112, 29, 31),      # whole tiles
     (24, 3, 1, 64, 32, 28, 28),
