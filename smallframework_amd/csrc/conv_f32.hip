@@ -337,7 +337,7 @@ __device__ __forceinline__ void conv_epilogue_buf_impl(const ConvArgs &a, floatx
                 float4 v = make_float4(acc[c][t][4 * q + 0], acc[c][t][4 * q + 1], acc[c][t][4 * q + 2], acc[c][t][4 * q + 3]);
                 if (ACC)
                 {
-                    const float4 old = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, ovoff[t], soff, 0));
+                    const float4 old = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, ovoff[t] + soff, 0, 0));
                     v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
                 }
                 v.x += bb.x; v.y += bb.y; v.z += bb.z; v.w += bb.w;
@@ -524,7 +524,7 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, FiltStage<COT> 
     }
 
     // ---- cooperative filter fetch: a thread owns AE consecutive input channels of one output channel ----------------
-    // (COT 1 / 2 / 4: 2 / 4 / 8 of the lane's eight), splits them and writes its piece of the three operands
+    // (COT 1 / 2: 2 / 4 of the lane's eight), splits them and writes its piece of the three operands
     constexpr int AE = COT * 2, SUBS = 8 / AE;
     const int a_c = tid / (64 * SUBS), a_u = tid % (64 * SUBS), a_l = a_u / SUBS, a_sub = a_u % SUBS;
     const int a_ci = 8 * (a_l >> 5) + AE * a_sub;
@@ -656,6 +656,7 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, FiltStage<COT> 
         live = live && more;
     };
     auto stage = [&](int buf, const float (&Areg)[AE]) {
+        static_assert(COT == 1 || COT == 2, "one or two packed pairs per thread");
         unsigned h[COT], m[COT], l[COT];                     // AE / 2 = COT packed pairs
 #pragma unroll
         for (int i = 0; i < COT; ++i) split_pair(Areg[2 * i], Areg[2 * i + 1], h[i], m[i], l[i]);
@@ -665,8 +666,7 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, FiltStage<COT> 
             const unsigned(&q)[COT] = p == 0 ? h : p == 1 ? m : l;
             unsigned char *d = &lds_a[buf][a_dst + p * 1024];
             if constexpr (COT == 1) *reinterpret_cast<unsigned *>(d) = q[0];
-            else if constexpr (COT == 2) *reinterpret_cast<uint2 *>(d) = make_uint2(q[0], q[1]);
-            else *reinterpret_cast<uint4 *>(d) = make_uint4(q[0], q[1], q[2], q[3]);
+            else *reinterpret_cast<uint2 *>(d) = make_uint2(q[0], q[1]);
         }
     };
     auto multiply = [&](int buf, const float4 (&B)[PXT][2]) {
@@ -758,9 +758,8 @@ __global__ __launch_bounds__(256, (COT * PXT == 2 ? 3 : COT * PXT == 1 ? 4 : 2))
 // BUF: operands through buffer loads, as in conv_lds_tile (each wave has its own K range, so its window position and
 // scalar offsets are the wave's)
 // W: waves of the workgroup, each with its share of the K-steps
-template <int COT, int PXT, bool POOL = false, bool BUF = false, int W = 4>
-__device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red)[W][COT * PXT * 4][64],
-                                                 const int cg, const int pxb)
+template <bool POOL = false, bool BUF = false, int W = 4>
+__device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red)[W][4][64], const int cg, const int pxb)
 {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -774,53 +773,33 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red
     const size_t in_blk = (size_t)a.H * a.W * CB;
     const float *zero_half = g_zero_block + half * 8;
 
-    const float *in_img[PXT];
-    unsigned lane_base[PXT];     // BUF: byte offset of (image, channel half) in the input tensor
-    int ih0[PXT], iw0[PXT];
-    bool pvalid[PXT];
-    size_t out_pix[PXT];
-    bool pool_ok[PXT];
-#pragma unroll
-    for (int t = 0; t < PXT; ++t)
+    int n, oh, ow;
+    bool pvalid, pool_ok = false;
+    size_t out_pix;
+    if (POOL)
+        pool_tile_pixel(a, pxb, col, n, oh, ow, pvalid, pool_ok, out_pix);
+    else
     {
-        int n, oh, ow, rem;
-        if (POOL)
-            pool_tile_pixel(a, pxb * PXT + t, col, n, oh, ow, pvalid[t], pool_ok[t], out_pix[t]);
-        else
-        {
-            const int p = (pxb * PXT + t) * 32 + col;
-            pvalid[t] = p < a.P;
-            const int pc = pvalid[t] ? p : 0;
-            n = fast_div(pc, a.fd_plane);
-            rem = pc - n * HoWo;
-            oh = fast_div(rem, a.fd_row);
-            ow = rem - oh * a.Wo;
-            pool_ok[t] = false;
-            out_pix[t] = ((size_t)n * CoB * HoWo + rem) * CB;
-        }
-        ih0[t] = oh * a.stride_h - a.pt;
-        iw0[t] = ow * a.stride - a.pl;
-        in_img[t] = a.in + (size_t)n * CiB * in_blk + half * 8;
-        lane_base[t] = (unsigned)(((size_t)n * CiB * in_blk + half * 8) * sizeof(float));
+        const int p = pxb * 32 + col;
+        pvalid = p < a.P;
+        const int pc = pvalid ? p : 0;
+        n = fast_div(pc, a.fd_plane);
+        const int rem = pc - n * HoWo;
+        oh = fast_div(rem, a.fd_row);
+        ow = rem - oh * a.Wo;
+        out_pix = ((size_t)n * CoB * HoWo + rem) * CB;
     }
-    const float *w_row[COT];
-    unsigned w_voff[COT];        // BUF: byte offset of this lane's filter row in the filter tensor
-#pragma unroll
-    for (int c = 0; c < COT; ++c)
-    {
-        const int co = (cg * COT + c) * 32 + col;
-        const int cc = co < a.Co ? co : a.Co - 1;
-        w_row[c] = a.filt + (size_t)(cc / CB) * CiB * taps * (CB * CB) + (cc % CB) + half * 8 * CB;
-        w_voff[c] = (unsigned)(((size_t)(cc / CB) * CiB * taps * (CB * CB) + (cc % CB) + half * 8 * CB) * sizeof(float));
-    }
+    const int ih0 = oh * a.stride_h - a.pt, iw0 = ow * a.stride - a.pl;
+    const float *in_img = a.in + (size_t)n * CiB * in_blk + half * 8;
+    const unsigned lane_base = (unsigned)(((size_t)n * CiB * in_blk + half * 8) * sizeof(float));   // BUF: (image, channel half) in the input tensor
+    const int co = cg * 32 + col, cc = co < a.Co ? co : a.Co - 1;
+    const size_t w_first = (size_t)(cc / CB) * CiB * taps * (CB * CB) + (cc % CB) + half * 8 * CB;
+    const float *w_row = a.filt + w_first;
+    const unsigned w_voff = (unsigned)(w_first * sizeof(float));                                    // BUF: this lane's row in the filter tensor
 
-    floatx16 acc[COT][PXT], sml[COT][PXT];
+    floatx16 acc[1][1], sml[1][1];
 #pragma unroll
-    for (int c = 0; c < COT; ++c)
-#pragma unroll
-        for (int t = 0; t < PXT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[c][t][r] = sml[c][t][r] = 0.f;
+    for (int r = 0; r < 16; ++r) acc[0][0][r] = sml[0][0][r] = 0.f;
 
     // this wave's K range: steps [s_lo, s_hi) of the (tap outer, channel block inner) order
     const int nsteps = taps * CiB;
@@ -828,23 +807,20 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red
     const int s_lo = wave * per;
     const int s_hi = (s_lo + per < nsteps) ? s_lo + per : nsteps;
     const int mine = s_hi > s_lo ? s_hi - s_lo : 0;
-    int tap0 = (s_lo < nsteps ? s_lo : 0) / CiB;
-    int cib = (s_lo < nsteps ? s_lo : 0) - tap0 * CiB;
+    const int s_first = s_lo < nsteps ? s_lo : 0;
+    int tap0 = s_first / CiB;
+    int cib = s_first - tap0 * CiB;
     int ta = tap0 / a.kw, tb = tap0 - (tap0 / a.kw) * a.kw;
     int left = mine;                 // steps still to be loaded
 
-    // BUF: the window position's lane offsets (out of range for a masked tap, and for every lane once the wave's steps
+    // BUF: the window position's lane offset (out of range for a masked tap, and for every lane once the wave's steps
     // have all been requested)
     const int in_blk32 = a.H * a.W * CB;
-    unsigned voff[PXT];
-    auto tap_offsets = [&]() {
-#pragma unroll
-        for (int t = 0; t < PXT; ++t)
-        {
-            const int ih = ih0[t] + ta, iw = iw0[t] + tb;
-            const bool ok = left > 0 && pvalid[t] && (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
-            voff[t] = ok ? lane_base[t] + (unsigned)((ih * a.W + iw) * (CB * (int)sizeof(float))) : BUF_OUT_OF_RANGE;
-        }
+    unsigned voff;
+    auto tap_offset = [&]() {
+        const int ih = ih0 + ta, iw = iw0 + tb;
+        const bool ok = left > 0 && pvalid && (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
+        voff = ok ? lane_base + (unsigned)((ih * a.W + iw) * (CB * (int)sizeof(float))) : BUF_OUT_OF_RANGE;
     };
     __amdgpu_buffer_rsrc_t rsrc_in, rsrc_f;
     if (BUF)
@@ -853,55 +829,40 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red
                                                     (int)((size_t)a.batch * a.Ci * a.H * a.W * sizeof(float)), BUF_RSRC_FLAGS);
         rsrc_f = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.filt), 0,
                                                    (int)((size_t)CoB * CiB * taps * (CB * CB) * sizeof(float)), BUF_RSRC_FLAGS);
-        tap_offsets();
+        tap_offset();
     }
-    auto load_step = [&](float (&A)[COT][8], float4 (&B)[PXT][2]) {
+    auto load_step = [&](float (&A)[8], float4 (&B)[2]) {
         if (BUF)
         {
             const int soff_b = cib * (in_blk32 * (int)sizeof(float));
+            B[0] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_in, voff, soff_b, 0));
+            B[1] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_in, voff + 16, soff_b, 0));
+            // past the wave's last step the filter reads zeros as well (the lane's offset is out of range, as the input's)
+            const unsigned wv = left > 0 ? w_voff : BUF_OUT_OF_RANGE;
+            const int soff_a = (cib * taps + ta * a.kw + tb) * (CB * CB * (int)sizeof(float));
 #pragma unroll
-            for (int t = 0; t < PXT; ++t)
-            {
-                B[t][0] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_in, voff[t], soff_b, 0));
-                B[t][1] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_in, voff[t] + 16, soff_b, 0));
-            }
-            // past the wave's last step the filter reads zeros as well
-            const int soff_a = left > 0 ? (cib * taps + ta * a.kw + tb) * (CB * CB * (int)sizeof(float)) : (int)BUF_SCALAR_OUT_OF_RANGE;
-#pragma unroll
-            for (int c = 0; c < COT; ++c)
-#pragma unroll
-                for (int kk = 0; kk < 8; ++kk)
-                    A[c][kk] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                             rsrc_f, w_voff[c] + kk * (CB * (int)sizeof(float)), soff_a, 0));
+            for (int kk = 0; kk < 8; ++kk)
+                A[kk] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc_f, wv + kk * (CB * (int)sizeof(float)), soff_a, 0));
             --left;
-            if (left <= 0) tap_offsets();          // nothing more to request: every lane out of range
+            if (left <= 0) tap_offset();           // nothing more to request: every lane out of range
             else if (++cib == CiB)                 // the next window position (wave-uniform, once in Ci/16 steps)
             {
                 cib = 0;
                 if (++tb == a.kw) { tb = 0; ++ta; }
-                tap_offsets();
+                tap_offset();
             }
             return;
         }
         const bool live = left > 0;                  // (the filter of a step past the last is multiplied by zeros)
-        const int tap = ta * a.kw + tb;
+        const int ih = ih0 + ta, iw = iw0 + tb;
+        const bool ok = live && pvalid && ih >= 0 && ih < a.H && iw >= 0 && iw < a.W;
+        const size_t off = (size_t)cib * in_blk + ((size_t)ih * a.W + iw) * CB;
+        const float4 *p = reinterpret_cast<const float4 *>(ok ? in_img + off : zero_half);
+        B[0] = p[0];
+        B[1] = p[1];
+        const float *w = w_row + ((size_t)cib * taps + ta * a.kw + tb) * (CB * CB);
 #pragma unroll
-        for (int t = 0; t < PXT; ++t)
-        {
-            const int ih = ih0[t] + ta, iw = iw0[t] + tb;
-            const bool ok = live && pvalid[t] && ih >= 0 && ih < a.H && iw >= 0 && iw < a.W;
-            const size_t off = (size_t)cib * in_blk + ((size_t)ih * a.W + iw) * CB;
-            const float4 *p = reinterpret_cast<const float4 *>(ok ? in_img[t] + off : zero_half);
-            B[t][0] = p[0];
-            B[t][1] = p[1];
-        }
-#pragma unroll
-        for (int c = 0; c < COT; ++c)
-        {
-            const float *w = w_row[c] + ((size_t)cib * taps + tap) * (CB * CB);
-#pragma unroll
-            for (int kk = 0; kk < 8; ++kk) A[c][kk] = w[kk * CB];
-        }
+        for (int kk = 0; kk < 8; ++kk) A[kk] = w[kk * CB];
         if (left > 1)                // stay on a valid position after the last step
         {
             if (++cib == CiB)
@@ -912,24 +873,19 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red
         }
         --left;
     };
-    auto compute_step = [&](const float (&A)[COT][8], const float4 (&B)[PXT][2]) {
-        Split8 As[COT], Bs[PXT];
-#pragma unroll
-        for (int c = 0; c < COT; ++c) As[c] = split8(A[c]);
-#pragma unroll
-        for (int t = 0; t < PXT; ++t) Bs[t] = split8(B[t][0], B[t][1]);
-        mfma_split<COT, PXT>(acc, sml, As, Bs);
+    auto compute_step = [&](const float (&A)[8], const float4 (&B)[2]) {
+        const Split8 As[1] = {split8(A)}, Bs[1] = {split8(B[0], B[1])};
+        mfma_split<1, 1>(acc, sml, As, Bs);
     };
 
-    // the register quad that this wave finishes (tile, four of its channels): its bias is requested before the K loop
-    constexpr int QUADS = COT * PXT * 4;
-    static_assert(QUADS <= W, "one quad per wave");
-    const int my_t = wave / 4 % PXT, my_co4 = (cg * COT + wave / (4 * PXT)) * 32 + 8 * (wave % 4) + 4 * half;
+    // the register quad (four channels) that this wave finishes: its bias is requested before the K loop
+    static_assert(W >= 4, "a wave for each of the tile's four register quads");
+    const int my_co4 = cg * 32 + 8 * (wave % 4) + 4 * half;
     float4 my_bias = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (a.bias && wave < QUADS && my_co4 < a.Co) my_bias = *reinterpret_cast<const float4 *>(a.bias + my_co4);
+    if (a.bias && wave < 4 && my_co4 < a.Co) my_bias = *reinterpret_cast<const float4 *>(a.bias + my_co4);
 
-    float A0[COT][8], A1[COT][8];
-    float4 B0[PXT][2], B1[PXT][2];
+    float A0[8], A1[8];
+    float4 B0[2], B1[2];
     load_step(A0, B0);
     const int npairs = (per + 1) >> 1;           // uniform over the workgroup
     for (int it = 0; it < npairs; ++it)
@@ -940,16 +896,16 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red
         compute_step(A1, B1);
     }
 
-    split_merge<COT, PXT>(acc, sml);
+    split_merge<1, 1>(acc, sml);
     // ---- reduction over the waves: wave w adds up register quad w of all waves, in wave order, and finishes it
 #pragma unroll
-    for (int i = 0; i < QUADS; ++i)
+    for (int i = 0; i < 4; ++i)
     {
-        const floatx16 &v = acc[i / (4 * PXT)][i / 4 % PXT];
-        red[wave][i][lane] = make_float4(v[4 * (i % 4)], v[4 * (i % 4) + 1], v[4 * (i % 4) + 2], v[4 * (i % 4) + 3]);
+        const floatx16 &v = acc[0][0];
+        red[wave][i][lane] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
     }
     __syncthreads();
-    if (wave >= QUADS) return;
+    if (wave >= 4) return;
     float4 v = red[0][wave][lane];
 #pragma unroll
     for (int w = 1; w < W; ++w)
@@ -958,9 +914,7 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red
         v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
     }
     const float nscale = act_scale(a.act, a.slope);
-    bool ok = my_co4 < a.Co && (POOL ? pool_ok[0] : pvalid[0]);
-    size_t pix = out_pix[0];
-    if (PXT == 2 && my_t == 1) { ok = my_co4 < a.Co && (POOL ? pool_ok[PXT - 1] : pvalid[PXT - 1]); pix = out_pix[PXT - 1]; }
+    const bool ok = my_co4 < a.Co && (POOL ? pool_ok : pvalid);
     if (POOL)
     {
         const float b4[4] = {my_bias.x, my_bias.y, my_bias.z, my_bias.w}, v4[4] = {v.x, v.y, v.z, v.w};
@@ -974,11 +928,11 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red
             const float y = __shfl_xor(x, 2, WAVE);
             m[e] = x > y ? x : y;
         }
-        if (ok) *reinterpret_cast<float4 *>(a.out + pix + (size_t)(my_co4 / CB) * ((a.Ho >> 1) * (a.Wo >> 1)) * CB + my_co4 % CB) =
+        if (ok) *reinterpret_cast<float4 *>(a.out + out_pix + (size_t)(my_co4 / CB) * ((a.Ho >> 1) * (a.Wo >> 1)) * CB + my_co4 % CB) =
                     make_float4(m[0], m[1], m[2], m[3]);
         return;
     }
-    float4 *o = reinterpret_cast<float4 *>(a.out + pix + (size_t)(my_co4 / CB) * HoWo * CB + my_co4 % CB);
+    float4 *o = reinterpret_cast<float4 *>(a.out + out_pix + (size_t)(my_co4 / CB) * HoWo * CB + my_co4 % CB);
     if (!ok) return;
     if (a.accumulate)
     {
@@ -997,17 +951,17 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red
     *o = v;
 }
 
-template <int COT, int PXT, bool BUF = false, int W = 4>
+template <bool BUF = false, int W = 4>
 __global__ __launch_bounds__(64 * W) void conv_mfma_f32_splitk_kernel(const ConvArgs a0)
 {
     const ConvArgs a = slab_args(a0);
-    __shared__ float4 red[W][COT * PXT * 4][64];
+    __shared__ float4 red[W][4][64];
     const int bid = blockIdx.x;
     const int lid = (bid % NUM_XCD) * a.per_xcd + bid / NUM_XCD;
     if (lid >= a.n_blocks) return;
     const int cg = a.px_first ? lid / a.n_px_blocks : lid % a.n_co_groups;
     const int pxb = a.px_first ? lid - cg * a.n_px_blocks : lid / a.n_co_groups;
-    conv_splitk_tile<COT, PXT, false, BUF, W>(a, red, cg, pxb);
+    conv_splitk_tile<false, BUF, W>(a, red, cg, pxb);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1040,7 +994,7 @@ __global__ __launch_bounds__(256, (COT * PXT == 2 ? 3 : COT * PXT == 1 ? 4 : 2))
     const int co32 = (lid % a.n_co_groups) * COT + sub % COT;
     const int px32 = (lid / a.n_co_groups) * (4 * PXT) + sub / COT;
     if (co32 * 32 >= a.Co || px32 * 32 >= a.P) return;     // uniform over the workgroup
-    conv_splitk_tile<1, 1, POOL, BUF>(a, red, co32, px32);
+    conv_splitk_tile<POOL, BUF>(a, red, co32, px32);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1952,12 +1906,11 @@ bool buffer_form(const ConvArgs &a)
     return !off && a.slabs == 0 && in_bytes <= BUF_MAX_BYTES && f_bytes <= BUF_MAX_BYTES && out_bytes <= BUF_MAX_BYTES;
 }
 
-template <int COT, int PXT>
 void launch_splitk(ConvArgs &a, hipStream_t s)
 {
     set_pixel_divisors(a, false);
-    a.n_co_groups = (a.Co + 32 * COT - 1) / (32 * COT);
-    a.n_px_blocks = (a.P + 32 * PXT - 1) / (32 * PXT);
+    a.n_co_groups = (a.Co + 31) / 32;
+    a.n_px_blocks = (a.P + 31) / 32;
     a.n_blocks = a.n_co_groups * a.n_px_blocks;
     a.per_xcd = (a.n_blocks + NUM_XCD - 1) / NUM_XCD;
     // the larger operand is the one that an XCD's workgroups share: 1024 -> 1024 3x3 @13x13 at batch 1 (37.7 MB of filter,
@@ -1969,10 +1922,10 @@ void launch_splitk(ConvArgs &a, hipStream_t s)
     // workgroup at most (that layer, 576 steps, 38.2 -> 36.3, 512 -> 1024 20.6 -> 19.7; 144 steps 11.0 -> 11.4, 64 steps 10.4 -> 12.7)
     const bool eight = a.kh * a.kw * (a.Ci / CB) >= 64;
     const bool sixteen = a.kh * a.kw * (a.Ci / CB) >= 256 && a.n_blocks <= NUM_CU && a.slabs == 0;
-    if (buffer_form(a) && sixteen) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT, true, 16>), grid, dim3(1024), 0, s, a);
-    else if (buffer_form(a) && eight) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT, true, 8>), grid, dim3(512), 0, s, a);
-    else if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT, true>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<COT, PXT>), grid, dim3(256), 0, s, a);
+    if (buffer_form(a) && sixteen) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<true, 16>), grid, dim3(1024), 0, s, a);
+    else if (buffer_form(a) && eight) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<true, 8>), grid, dim3(512), 0, s, a);
+    else if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((conv_mfma_f32_splitk_kernel<>), grid, dim3(256), 0, s, a);
 }
 
 // Whole rounds + cut tail (conv_mfma_f32_hybrid_kernel) or whole tiles only?  A split-K piece multiplies about half as
@@ -2215,7 +2168,7 @@ int conv_f32(const char *op, int batch, int kh, int kw, int stride, int pt, int 
     wave_tile(Co, tiles32, nsteps, &cot, &pxt);
     if (wants_splitk(tiles32, nsteps))
     {
-        launch_splitk<1, 1>(a, s);
+        launch_splitk(a, s);
         SHP_LAUNCH_CHECK(op);
         return SMALL_HIP_OK;
     }
