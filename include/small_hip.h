@@ -17,6 +17,11 @@
  *     reference's (batch-1) call on image n: bit for bit on the uint8 path, within float32
  *     rounding on the float path (the kernel variant, and with it the summation order, is chosen
  *     from the launch shape).  The reference has no batch argument.
+ *   - float32 convolutions with 16 or more input channels multiply operands split into three bf16 parts each, which hold
+ *     them exactly, and leave out products of at most 2^-24 of a float32 product: a sum of two or more products is as close
+ *     to the exact result as float32 products rounded and added in some order (long sums are closer), a single product is
+ *     within 1.7 * 2^-24 of itself instead of 2^-24.  Infinities, NaN, overflow and sums below 2^-64 are as float32 products
+ *     give them; an operand below 2^-110 times one above 2^40 keeps an absolute error of 2^-133 times the latter.
  *   - Pads are given in the reference's public order: top, bottom, left, right.
  *   - Output height/width follow include/small/utils.hpp:159-165 applied to the padded input.
  *   - `stream` is a hipStream_t (NULL = the default stream).  Calls are asynchronous with

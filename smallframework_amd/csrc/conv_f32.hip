@@ -3,8 +3,8 @@
 // input_channels % 16 == 0: implicit GEMM,
 //      D[co][px] += sum_k  F[co][k] * I[k][px],   k = (tap, ci)
 // on v_mfma_f32_32x32x16_bf16: every float32 operand is split into three bf16 numbers that add up to it exactly, and six
-// of the nine products (all but those below half a unit in the last place of a float32 product) are added in float32
-// (Split8 below).  MFMA rows are output channels, MFMA columns are output pixels flattened over (image, oh, ow).
+// of the nine products are added in float32; the three left out are at most 2^-24 of a product together (Split8 below).
+// MFMA rows are output channels, MFMA columns are output pixels flattened over (image, oh, ow).
 // With the packed layouts a K-step of 16 (one input-channel block at one filter tap) needs no
 // shuffling at all:
 //   - B operand: lane (px = lane%32, half = lane/32) reads 8 consecutive floats of its pixel's
@@ -42,23 +42,30 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------------------------
-// float32 products on the bf16 matrix pipes.  A float32 number is the exact sum of three bf16 numbers, x = h + m + l: h is
-// the upper half of x (rounded toward zero, so that the largest finite numbers stay finite), m = bf16(x - h) to nearest,
-// l = x - h - m, at most eight bits (|m| <= 2^-7 |x|, |l| <= 2^-16 |x|, l's sign does not follow x's), and a product of two
-// bf16 numbers is exact in float32.  x * y is then added up as hh + (hm + mh + mm + hl + lh); what is left out, ml + lm + ll, is
-// below 2^-22 |x y|, 2.4e-8 of it root mean square and of either sign.  v_mfma_f32_32x32x16_bf16 multiplies sixteen times as
-// fast as v_mfma_f32_32x32x2_f32, six of them replace eight float32 ones per sixteen channels: 192 matrix cycles instead of
-// 512, and the vector ALU may issue beside them (a float32 MFMA occupies it).
-// The two truncations take the upper halves of a pair in one v_perm_b32 and need no conversion before the subtraction:
-// against all three parts rounded to nearest Tiny-YOLOv2 batch 1 119.2 -> 114.6 us, the 3x3 layer of 96 channels (batch 7,
-// 30x30) 13.0 -> 12.7, large launches the same to 1%.  Subtracting with v_dot2_f32_bf16 (7 instead of 11 instructions a
-// pair) was slower: it does not run beside the MFMAs.
+// float32 products on the bf16 matrix pipes.  A float32 number is the exact sum of three bf16 numbers, x = h + m + l: h =
+// bf16(x) and m = bf16(x - h), both rounded to nearest, l = x - h - m, at most eight bits (|m| <= 2^-8 |x|, |l| <= 2^-17 |x|,
+// either sign), and a product of two bf16 numbers is exact in float32.  x * y is then added up as
+// hh + (hm + mh + mm + hl + lh); what is left out, ml + lm + ll, is at most 2^-24 |x y| and 5e-9 of it root mean square.
+// v_mfma_f32_32x32x16_bf16 multiplies sixteen times as fast as v_mfma_f32_32x32x2_f32, six of them replace eight float32
+// ones per sixteen channels: 192 matrix cycles instead of 512, and the vector ALU may issue beside them (a float32 MFMA
+// occupies it).  Nine products less ll would leave nothing out but take 256 cycles: 3x3 256->256 @56x56 batch 64 1137 -> 1404 us,
+// Tiny-YOLOv2 batch 16 747 -> 871 (float32 MFMAs 1622 and 915), and launches of one or two tiles per SIMD slower than float32 MFMAs.
+// h truncated instead of rounded (the upper halves of a pair in one v_perm_b32, |m| <= 2^-7 |x|) leaves out up to 2^-22 |x y|:
+// 1 to 3% faster, but a single product is then off by up to 2.6e-7 and by 3.4e-8 root mean square.  Subtracting with
+// v_dot2_f32_bf16 (7 instead of 11 instructions a pair) was slower: it does not run beside the MFMAs.
 // hh has an accumulator of its own ("big"): there one addition per sixteen products is rounded where the float32 MFMA
 // chain rounds sixteen, and the small terms are added to a sum of their own size, so that nothing of them is lost
-// against a large total.  Error against float64 (relative 2-norm, K = 16 / 64 / 512 / 2304 / 4608 normal products): the
-// float32 MFMA chain 7.4e-8 / 1.4e-7 / 4.0e-7 / 8.6e-7 / 1.2e-6; see the tests for this form's.
-// Range: |x| below 2^-110 loses bits of m and l (an absolute error of at most 2^-134 |y|).  Infinities and NaN give what
-// float32 products give (split_sum); a NaN is one of those with the quiet bit set, the only ones arithmetic produces.
+// against a large total.  Error against float64 (relative 2-norm), float32 MFMAs and this form, sums of
+//   1 / 2 / 3 / 6 / 16 products among zeros:   2.5e-8 / 3.1e-8 / 3.6e-8 / 4.7e-8 / 7.3e-8    2.6e-8 / 2.7e-8 / 2.8e-8 / 2.9e-8 / 3.5e-8
+//   2304 normal products:   8.6e-7    2.9e-7
+// A sum of one product is off by up to 9.9e-8 of it, where a float32 product is rounded once (6.0e-8); two or more are not
+// worse.  (Each workgroup that takes a share of a reduction rounds its own part: 2.6e-8 / 3.7e-8 / 4.3e-8 / 5.0e-8 / 6.7e-8 at most.)
+// Range: operands from 2^-110 up are split exactly.  Sums that are not finite, or below 2^-64 without being zero, are made
+// again with float32 MFMAs (split_odd, mfma_f32_wave): infinities and NaN of any payload, operands next to the largest finite
+// number, whose h is infinite, and operands or products among the smallest give what float32 products give.  What is
+// left: an operand below 2^-110 that is multiplied by one above 2^40 has an absolute error of 2^-133 times the latter.
+constexpr float SPLIT_LEAST = 0x1p-64f;
+
 struct Split8
 {
     bf16x8 h, m, l;      // eight consecutive reduction elements of one row or column: one MFMA operand each
@@ -80,12 +87,12 @@ __device__ __forceinline__ unsigned pack_high(float a, float b)       // the upp
 {
     return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x07060302u);
 }
-// a pair of numbers: 11 vector instructions
+// a pair of numbers: 12 vector instructions
 __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l)
 {
-    h = pack_high(a, b);
-    a -= bf16_hi(__builtin_bit_cast(unsigned, a));
-    b -= bf16_hi(__builtin_bit_cast(unsigned, b));
+    h = pack_bf16(a, b);
+    a -= bf16_lo(h);
+    b -= bf16_hi(h);
     m = pack_bf16(a, b);
     a -= bf16_lo(m);
     b -= bf16_hi(m);
@@ -109,34 +116,67 @@ __device__ __forceinline__ Split8 split8(const float4 &lo, const float4 &hi)
     return split8(x);
 }
 
-// sixteen channels: COT x PXT tiles of 32 x 32, the order inside each accumulator fixed (the same bits in every kernel)
+// sixteen channels, the small products first; the order inside an accumulator is the same in every kernel, and so are the bits
+#define SHP_SPLIT_PRODUCTS_(X) X(sml, l, h) X(sml, h, l) X(sml, m, m) X(sml, m, h) X(sml, h, m) X(big, h, h)
+// one 32 x 32 tile
+__device__ __forceinline__ void mfma_split(floatx16 &big, floatx16 &sml, const Split8 &A, const Split8 &B)
+{
+#define SHP_MFMA_(acc_, a_, b_) acc_ = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.a_, B.b_, acc_, 0, 0, 0);
+    SHP_SPLIT_PRODUCTS_(SHP_MFMA_)
+#undef SHP_MFMA_
+}
+// COT x PXT tiles, each product for all tiles in turn
 template <int COT, int PXT>
 __device__ __forceinline__ void mfma_split(floatx16 (&big)[COT][PXT], floatx16 (&sml)[COT][PXT], const Split8 (&A)[COT],
                                            const Split8 (&B)[PXT])
 {
 #define SHP_MFMA_(acc_, a_, b_)                                                                               \
     _Pragma("unroll") for (int t = 0; t < PXT; ++t) _Pragma("unroll") for (int c = 0; c < COT; ++c)           \
-        acc_[c][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[c].a_, B[t].b_, acc_[c][t], 0, 0, 0)
-    SHP_MFMA_(sml, l, h);
-    SHP_MFMA_(sml, h, l);
-    SHP_MFMA_(sml, m, m);
-    SHP_MFMA_(sml, m, h);
-    SHP_MFMA_(sml, h, m);
-    SHP_MFMA_(big, h, h);
+        acc_[c][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[c].a_, B[t].b_, acc_[c][t], 0, 0, 0);
+    SHP_SPLIT_PRODUCTS_(SHP_MFMA_)
 #undef SHP_MFMA_
 }
-// big + small.  An infinite operand leaves an infinity or NaN in big, as float32 products would, and NaN or infinity
-// (inf - inf) in the parts that small sums up: there small is replaced by a finite number.
-__device__ __forceinline__ float split_sum(float big, float sml) { return big + __builtin_amdgcn_fmed3f(sml, -3.0e38f, 3.0e38f); }
+#undef SHP_SPLIT_PRODUCTS_
+// big + small; true for a wave that may have to multiply again (see above; split_odd tells).  An infinity or a NaN times
+// zero is a NaN, which a chain of fused multiply-adds keeps.
 template <int COT, int PXT>
-__device__ __forceinline__ void split_merge(floatx16 (&big)[COT][PXT], const floatx16 (&sml)[COT][PXT])
+__device__ __forceinline__ bool split_merge(floatx16 (&big)[COT][PXT], const floatx16 (&sml)[COT][PXT], const bool (&pvalid)[PXT])
 {
+    float nan = 0.f, least = 1.f;
+#pragma unroll
+    for (int t = 0; t < PXT; ++t)
+    {
+        float l = 1.f;
+#pragma unroll
+        for (int c = 0; c < COT; ++c)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+            {
+                const float v = big[c][t][r] + sml[c][t][r];
+                nan = fmaf(v, 0.f, nan);
+                l = fminf(l, fabsf(v));
+                big[c][t][r] = v;
+            }
+        least = fminf(least, pvalid[t] ? l : 1.f);
+    }
+    return __any(nan != 0.f || least < SPLIT_LEAST);
+}
+// cold: zeros (dead inputs, channels without weights) are told from very small sums
+template <int COT, int PXT>
+__device__ __forceinline__ bool split_odd(const floatx16 (&v)[COT][PXT])
+{
+    bool odd = false;
 #pragma unroll
     for (int c = 0; c < COT; ++c)
 #pragma unroll
         for (int t = 0; t < PXT; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) big[c][t][r] = split_sum(big[c][t][r], sml[c][t][r]);
+            for (int r = 0; r < 16; ++r)
+            {
+                const float m = fabsf(v[c][t][r]);
+                odd |= (m != 0.f) & !((m >= SPLIT_LEAST) & (m <= 3.402823466e38f));
+            }
+    return __any(odd);
 }
 
 struct ConvArgs
@@ -434,6 +474,83 @@ __device__ __forceinline__ void pool_tile_pixel(const ConvArgs &a, const int til
 }
 
 // ---------------------------------------------------------------------------------------------
+// float32 products (v_mfma_f32_32x32x2_f32) of one wave: K-steps [s_begin, s_begin + count) of its COT x PXT tiles, operands
+// straight from global memory a step ahead, channels kk and 8 + kk of a block in MFMA number kk.
+template <int COT, int PXT>
+__device__ __forceinline__ void mfma_f32_wave(const ConvArgs &a, floatx16 (&acc)[COT][PXT], const int cg, const int col, const int half,
+                                              const float *const (&in_img)[PXT], const int (&ih0)[PXT], const int (&iw0)[PXT],
+                                              const bool (&pvalid)[PXT], const int s_begin, const int count)
+{
+    const int CiB = a.Ci / CB, taps = a.kh * a.kw;
+    const size_t in_blk = (size_t)a.H * a.W * CB;
+    const float *zero_half = g_zero_block + half * 8;
+    const float *w_row[COT];
+#pragma unroll
+    for (int c = 0; c < COT; ++c)
+    {
+        const int co = (cg * COT + c) * 32 + col;
+        const int cc = co < a.Co ? co : a.Co - 1;                 // rows past Co: garbage, never stored
+        w_row[c] = a.filt + (size_t)(cc / CB) * CiB * taps * (CB * CB) + (cc % CB) + half * 8 * CB;
+    }
+#pragma unroll
+    for (int c = 0; c < COT; ++c)
+#pragma unroll
+        for (int t = 0; t < PXT; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[c][t][r] = 0.f;
+    const int tap0 = s_begin / CiB;
+    int cib = s_begin - tap0 * CiB, ta = tap0 / a.kw, tb = tap0 - (tap0 / a.kw) * a.kw;
+    auto request = [&](const int k4, float (&A)[COT][4], float4 (&B)[PXT]) {      // a quarter of the block's channels per wave half
+#pragma unroll
+        for (int t = 0; t < PXT; ++t)
+        {
+            const int ih = ih0[t] + ta, iw = iw0[t] + tb;
+            const bool ok = pvalid[t] && (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
+            const float *p = ok ? in_img[t] + ((size_t)cib * in_blk + ((size_t)ih * a.W + iw) * CB) : zero_half;
+            B[t] = *reinterpret_cast<const float4 *>(p + 4 * k4);
+        }
+#pragma unroll
+        for (int c = 0; c < COT; ++c)
+        {
+            const float *w = w_row[c] + ((size_t)cib * taps + ta * a.kw + tb) * (CB * CB) + k4 * 4 * CB;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) A[c][k] = w[k * CB];
+        }
+    };
+    auto advance = [&]() {
+        if (++cib == CiB)
+        {
+            cib = 0;
+            if (++tb == a.kw) { tb = 0; ++ta; }
+        }
+    };
+    auto multiply = [&](const float (&A)[COT][4], const float4 (&B)[PXT]) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int t = 0; t < PXT; ++t)
+            {
+                const float b = k == 0 ? B[t].x : k == 1 ? B[t].y : k == 2 ? B[t].z : B[t].w;
+#pragma unroll
+                for (int c = 0; c < COT; ++c) acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(A[c][k], b, acc[c][t], 0, 0, 0);
+            }
+    };
+#pragma unroll 1
+    for (int s = 0; s < count; ++s)
+    {
+#pragma unroll
+        for (int k4 = 0; k4 < 2; ++k4)
+        {
+            float A[COT][4];
+            float4 B[PXT];
+            request(k4, A, B);
+            multiply(A, B);
+        }
+        advance();
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
 // The main kernel body: filter operand staged through LDS.  The four waves of a workgroup
 // multiply the same output-channel group, so the step's [16 ci][16 co] filter tiles (COT*2 KiB)
 // are fetched once per workgroup (a thread takes consecutive input channels of one output channel), split once,
@@ -443,8 +560,8 @@ __device__ __forceinline__ void pool_tile_pixel(const ConvArgs &a, const int til
 // What bounds it: the matrix pipes at the clock the card's power limit leaves (six products on registers alone run at
 // 1.8 GHz and 290-300 TFLOP/s) and the split's vector instructions, of which a bit more than half hide behind the MFMAs (the
 // loop of a 64 x 32 wave tile without global loads: 209 TFLOP/s, 265 with the split left out).  Batch 64 / 16, before (float32
-// MFMAs) -> now: 3x3 256->256 @56x56 1572 -> 1102 us (215 TFLOP/s), 3x3 1024->1024 @13x13 376 -> 285, 3x3 128->256 @26x26
-// 50.2 -> 45.4, 1x1 512->512 @14x14 50.4 -> 40.0, 1x1 128->128 @56x56 64.5 -> 59.3 (its 206 MB are 40 us of copy).
+// MFMAs) -> now: 3x3 256->256 @56x56 1600 -> 1123 us (211 TFLOP/s), 3x3 1024->1024 @13x13 411 -> 301, 3x3 128->256 @26x26
+// 51.6 -> 41.2, 1x1 512->512 @14x14 55.9 -> 40.1, 1x1 128->128 @56x56 64.8 -> 51.5 (its 206 MB are 40 us of copy).
 
 // s_begin / s_count: only K-steps [s_begin, s_begin + s_count) of the tile (s_count < 0: all of them); raw != nullptr: the
 // accumulators go there as they are ([wave][tile of the wave][register quad][lane] float4) instead of through the epilogue
@@ -523,6 +640,29 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, FiltStage<COT> 
         if (PW) in_img[t] += (size_t)(oh * a.W + ow) * CB;
     }
 
+    // the wave's finished sums: raw, or through the epilogue
+    auto finish = [&](floatx16 (&acc)[COT][PXT]) {
+        if (raw)
+        {
+            float4 *r4 = reinterpret_cast<float4 *>(raw) + (size_t)wave * (COT * PXT * 4 * WAVE) + lane;
+    #pragma unroll
+            for (int c = 0; c < COT; ++c)
+    #pragma unroll
+                for (int t = 0; t < PXT; ++t)
+    #pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        r4[((c * PXT + t) * 4 + q) * WAVE] = make_float4(acc[c][t][4 * q], acc[c][t][4 * q + 1], acc[c][t][4 * q + 2], acc[c][t][4 * q + 3]);
+            return;
+        }
+        if (BUF && BLDS)
+        {
+            if (POOL) conv_epilogue_pool<COT, PXT, true>(a, acc, cg, half, pool_ok, out_pix, s_bias, ovoff);
+            else conv_epilogue_buf<COT, PXT>(a, acc, cg, half, HoWo, ovoff, s_bias);
+            return;
+        }
+        if (POOL) conv_epilogue_pool<COT, PXT>(a, acc, cg, half, pool_ok, out_pix, BLDS ? s_bias : nullptr);
+        else conv_epilogue<COT, PXT>(a, acc, cg, half, HoWo, pvalid, out_pix, BLDS ? s_bias : nullptr);
+    };
     // ---- cooperative filter fetch: a thread owns AE consecutive input channels of one output channel ----------------
     // (COT 1 / 2: 2 / 4 of the lane's eight), splits them and writes its piece of the three operands
     constexpr int AE = COT * 2, SUBS = 8 / AE;
@@ -707,28 +847,15 @@ __device__ __forceinline__ void conv_lds_tile(const ConvArgs &a, FiltStage<COT> 
     }
     // an odd step count leaves the last step staged in buffer 0 / B0 (the loop's invariant)
     if (nsteps & 1) multiply(0, B0);
-    split_merge<COT, PXT>(acc, sml);
-
-    if (raw)
+    if (__builtin_expect(split_merge<COT, PXT>(acc, sml, pvalid), 0) && split_odd<COT, PXT>(acc))
     {
-        float4 *r4 = reinterpret_cast<float4 *>(raw) + (size_t)wave * (COT * PXT * 4 * WAVE) + lane;
+        const float *img[PXT];
 #pragma unroll
-        for (int c = 0; c < COT; ++c)
-#pragma unroll
-            for (int t = 0; t < PXT; ++t)
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    r4[((c * PXT + t) * 4 + q) * WAVE] = make_float4(acc[c][t][4 * q], acc[c][t][4 * q + 1], acc[c][t][4 * q + 2], acc[c][t][4 * q + 3]);
-        return;
+        for (int t = 0; t < PXT; ++t)
+            img[t] = BUF ? a.in + lane_base[t] / sizeof(float) : PW ? in_img[t] - (ih0[t] * a.W + iw0[t]) * CB : in_img[t];
+        mfma_f32_wave<COT, PXT>(a, acc, cg, col, half, img, ih0, iw0, pvalid, s_begin, nsteps);
     }
-    if (BUF && BLDS)
-    {
-        if (POOL) conv_epilogue_pool<COT, PXT, true>(a, acc, cg, half, pool_ok, out_pix, s_bias, ovoff);
-        else conv_epilogue_buf<COT, PXT>(a, acc, cg, half, HoWo, ovoff, s_bias);
-        return;
-    }
-    if (POOL) conv_epilogue_pool<COT, PXT>(a, acc, cg, half, pool_ok, out_pix, BLDS ? s_bias : nullptr);
-    else conv_epilogue<COT, PXT>(a, acc, cg, half, HoWo, pvalid, out_pix, BLDS ? s_bias : nullptr);
+    finish(acc);
 }
 
 // The second launch bound (minimum waves per SIMD: 4 / 3 / 2 for one / two / four MFMA tiles per
@@ -874,8 +1001,8 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red
         --left;
     };
     auto compute_step = [&](const float (&A)[8], const float4 (&B)[2]) {
-        const Split8 As[1] = {split8(A)}, Bs[1] = {split8(B[0], B[1])};
-        mfma_split<1, 1>(acc, sml, As, Bs);
+        const Split8 As = split8(A), Bs = split8(B[0], B[1]);
+        mfma_split(acc[0][0], sml[0][0], As, Bs);
     };
 
     // the register quad (four channels) that this wave finishes: its bias is requested before the K loop
@@ -896,7 +1023,13 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red
         compute_step(A1, B1);
     }
 
-    split_merge<1, 1>(acc, sml);
+    const bool ok1[1] = {pvalid};
+    if (__builtin_expect(split_merge<1, 1>(acc, sml, ok1), 0) && split_odd<1, 1>(acc))
+    {
+        const float *const img[1] = {in_img};
+        const int h1[1] = {ih0}, w1[1] = {iw0};
+        mfma_f32_wave<1, 1>(a, acc, cg, col, half, img, h1, w1, ok1, s_first, mine);
+    }
     // ---- reduction over the waves: wave w adds up register quad w of all waves, in wave order, and finishes it
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -952,7 +1085,7 @@ __device__ __forceinline__ void conv_splitk_tile(const ConvArgs &a, float4 (&red
 }
 
 template <bool BUF = false, int W = 4>
-__global__ __launch_bounds__(64 * W) void conv_mfma_f32_splitk_kernel(const ConvArgs a0)
+__global__ __launch_bounds__(64 * W, 4) void conv_mfma_f32_splitk_kernel(const ConvArgs a0)
 {
     const ConvArgs a = slab_args(a0);
     __shared__ float4 red[W][4][64];
@@ -1652,9 +1785,9 @@ __global__ __launch_bounds__(256, 4) void conv_stem3x3_dw3x3_f32_kernel(const Co
 // pointwise layer's output, the largest tensor of such a pair, is neither written nor read.
 // A workgroup owns 32 * COT channels and a tile of TOH x TOW depthwise outputs of one image (14 x 14 at stride 1, 7 x 8 at
 // stride 2).  The PH x PW pointwise pixels under that tile (16 x 16 / 15 x 17, at most 256) are eight 32-pixel MFMA tiles,
-// two per wave; the filter slice of the workgroup is staged in LDS once (memory pipeline, padded 16 x 16 tiles), the
-// activation operand goes from memory to the MFMA register as in conv_lds_tile, and the K loop is unrolled: no barrier
-// and no staging inside it.  The products are added in conv_lds_tile's order.  The activated result is parked in LDS as
+// two per wave; the filter slice of the workgroup is split and staged in LDS once, in MFMA operand order, the activation
+// operand goes from memory to the wave's registers and is split there as in conv_lds_tile, and the K loop is unrolled: no
+// barrier and no staging inside it.  The products are added in conv_lds_tile's order.  The activated result is parked in LDS as
 // [pixel][channel] (zeros outside the pointwise layer's map: the depthwise layer's padding) and the depthwise window
 // runs on it like dw3x3_f32_tile_kernel (a lane = four channels of one column, a run of rows, the same order of operations).
 // The halo is computed again by the neighbouring workgroups: 256 / 196 = 1.31 x the pointwise work at stride 1,
@@ -1708,21 +1841,6 @@ __global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kerne
     const int HW = a.H * a.W, CoB = a.Co / CB;
     const float nscale = act_scale(a.act, a.slope);
 
-    // ---- requests first: filter slice to LDS, biases, depthwise taps ------------------------------------------------
-    // filter: unit u of 64 COT CIB = (operand u / 64 = K-step and channel tile, lane u % 64) is eight input channels of one
-    // output channel; the thread that loads them splits them once for the whole workgroup
-    constexpr int NU = 64 * COT * CIB, UPT = (NU + 255) / 256;
-    float fraw[UPT][8];
-#pragma unroll
-    for (int r = 0; r < UPT; ++r)
-    {
-        const int u = tid + r * 256, ul = u & 63, op = u >> 6, us = op / COT, uc = op - us * COT;
-        const int cob = (cg * COT + uc) * 2 + ((ul & 31) >> 4);
-        const float *src = a.filt + ((size_t)cob * CIB + us) * (CB * CB) + (ul >> 5) * 8 * CB + (ul & 15);
-        if (NU % 256 == 0 || u < NU)
-#pragma unroll
-            for (int k = 0; k < 8; ++k) fraw[r][k] = src[k * CB];
-    }
     float my_bias = 0.f;
     if (tid < CG && a.bias) my_bias = a.bias[cg * CG + tid];
     // depthwise phase: lane = (channel quad q, column dx, row group rg)
@@ -1745,6 +1863,22 @@ __global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kerne
         pidx[t] = pp;
         in_px[t] = pin[t] ? a.in + ((size_t)n * CIB * HW + oh * a.W + ow) * CB + half * 8 : g_zero_block + half * 8;
     }
+    if (tid < CG) s_bias[tid] = my_bias;
+    // ---- requests first: filter slice, the first two steps' pixels -----------------------------------------------
+    // filter: unit u of 64 COT CIB = (operand u / 64 = K-step and channel tile, lane u % 64) is eight input channels of one
+    // output channel; the thread that loads them splits them once for the whole workgroup
+    constexpr int NU = 64 * COT * CIB, UPT = (NU + 255) / 256;
+    float fraw[UPT][8];
+#pragma unroll
+    for (int r = 0; r < UPT; ++r)
+    {
+        const int u = tid + r * 256, ul = u & 63, op = u >> 6, us = op / COT, uc = op - us * COT;
+        const int cob = (cg * COT + uc) * 2 + ((ul & 31) >> 4);
+        const float *src = a.filt + ((size_t)cob * CIB + us) * (CB * CB) + (ul >> 5) * 8 * CB + (ul & 15);
+        if (NU % 256 == 0 || u < NU)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) fraw[r][k] = src[k * CB];
+    }
     const int in_blk32 = HW * CB;
     float4 B[2][2][2];                                       // [buffer][pixel tile][half of the eight channels]
     auto fetch = [&](const int buf, const int cib) {
@@ -1758,7 +1892,6 @@ __global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kerne
     };
     fetch(0, 0);
     if (CIB > 1) fetch(1, 1);
-    if (tid < CG) s_bias[tid] = my_bias;
 #pragma unroll
     for (int r = 0; r < UPT; ++r)
     {
@@ -1781,10 +1914,8 @@ __global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kerne
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[c][t][r] = sml[c][t][r] = 0.f;
-#pragma unroll
-    for (int s = 0; s < CIB; ++s)
-    {
-        Split8 A[COT], Bs[2];
+    auto step = [&](const int buf, const int s) {
+        Split8 A[COT];
 #pragma unroll
         for (int c = 0; c < COT; ++c)
         {
@@ -1794,11 +1925,37 @@ __global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kerne
             A[c].l = *reinterpret_cast<const bf16x8 *>(r + 2048);
         }
 #pragma unroll
-        for (int t = 0; t < 2; ++t) Bs[t] = split8(B[s & 1][t][0], B[s & 1][t][1]);
-        mfma_split<COT, 2>(acc, sml, A, Bs);
-        if (s + 2 < CIB) fetch(s & 1, s + 2);
-    }
+        for (int t = 0; t < 2; ++t)                          // (tile after tile: both split at once would not fit the registers)
+        {
+            const Split8 Bs = split8(B[buf][t][0], B[buf][t][1]);
+#pragma unroll
+            for (int c = 0; c < COT; ++c) mfma_split(acc[c][t], sml[c][t], A[c], Bs);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (s + 2 < CIB) fetch(buf, s + 2);
+    };
+#pragma unroll
+    for (int s = 0; s < CIB; ++s) step(s & 1, s);
 
+    if (__builtin_expect(split_merge<COT, 2>(acc, sml, pin), 0) && split_odd<COT, 2>(acc))
+    {
+        // (positions from the lane number again: kept for this they would cost the K loop registers)
+        int l = lane;
+        asm("" : "+v"(l));
+        const float *img[2];
+        int ih[2], iw[2];
+        bool in[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+        {
+            const int pp = (2 * wave + t) * 32 + (l & 31), py = pp / PW;
+            ih[t] = py0 + py;
+            iw[t] = px0 + pp - py * PW;
+            in[t] = pp < NPX;
+            img[t] = a.in + (size_t)n * CIB * HW * CB + (l >> 5) * 8;
+        }
+        mfma_f32_wave<COT, 2>(a, acc, cg, l & 31, l >> 5, img, ih, iw, in, 0, CIB);
+    }
     // the depthwise taps: requested here (held through the K loop they would cost a workgroup of occupancy), used after the
     // parked tile's barrier
     float4 w[9];
@@ -1809,7 +1966,6 @@ __global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kerne
     }
     float4 dbias = make_float4(0.f, 0.f, 0.f, 0.f);
     if (d.dw_bias) dbias = *reinterpret_cast<const float4 *>(d.dw_bias + dcob * CB + dq4);
-    split_merge<COT, 2>(acc, sml);
     __syncthreads();                                         // every wave has read its last filter operand
     // ---- bias, activation, park in LDS: a lane holds channels c*32 + 8 qq + 4 half + 0..3 of its pixel -------------
     // pixels outside the pointwise layer's map are the depthwise layer's padding: those lanes store zeros (a branch on
@@ -1929,12 +2085,13 @@ void launch_splitk(ConvArgs &a, hipStream_t s)
 }
 
 // Whole rounds + cut tail (conv_mfma_f32_hybrid_kernel) or whole tiles only?  A split-K piece multiplies about half as
-// fast as a whole tile (operands straight from global memory, one MFMA chain per wave), so the cut tail wins while the
-// left-over tiles fill at most two thirds of a round and loses beyond, whatever the wave tile and the number of whole rounds.
-// Batch sweeps, left-over tiles of 256 -> gain (+) or loss (-) in us: 1x1 256->256 @28x28 (16 K-steps) 32: +3, 128: +1,
-// 224: -3; 512->512 @14x14 (32) 80: +2..6, 176: -2, 224: -6; 3x3 64->128 @52x52 (36) 84: +1, 168: -3, 252: -7;
-// 3x3 128->256 @26x26 (72) 20: +25, 84: +10, 128: +4, 168: -3, 216: -10; 3x3 256->512 @13x13 (144) 40: +42, 128: +13,
-// 168: -12, 216: -27.
+// fast as a whole tile (operands straight from global memory, both split for one MFMA tile), so the cut tail wins while the
+// left-over tiles fill at most two thirds of a round.  Batch sweeps, left-over tiles of 256: us with whole tiles only -> with the
+// cut tail.  Wave tile 1x1: 128->128 1x1 @20x20 (8 K-steps) 30: 11.6 -> 10.0, 213: 9.7 -> 10.5; 192->256 @14x14 (12) 125: 11.3 ->
+// 10.5, 200: 11.6 -> 13.0; 3x3 64->128 @52x52 (36) 82: 16.9 -> 15.0, 167: 17.5 -> 16.8, 250: 18.9 -> 20.1; 3x3 128->256 @26x26
+// (72) 82: 29.4 -> 27.2, 169: 31.9 -> 30.8, 250: level.  Wave tile 2x1, which loses from half a round on already: 192->256
+// @14x14 174: 13.0 -> 14.8; 256->256 1x1 @28x28 (16) 38: 14.4 -> 11.3, 136: 15.0 -> 15.1, 186: 15.6 -> 16.5; 512->512 @14x14 (32) 112: 24.2 -> 21.5,
+// 162: 25.2 -> 26.7; 3x3 64->64 @56x56 (36) 136: 27.2 -> 28.6; 3x3 128->256 @26x26 40: 45.7 -> 37.1, 126: 49.2 -> 46.1.
 template <int COT, int PXT>
 bool tail_pays(int n_main, int rest, int nsteps)
 {
@@ -1942,8 +2099,6 @@ bool tail_pays(int n_main, int rest, int nsteps)
     static const int knob = tune_int("conv_tail", 1);
     (void)n_main;
     if (knob == 0 || rest == 0 || nsteps < 8) return false;
-    // with the split-K pieces on buffer loads the break-even moved up: left-over tiles 160..168 now gain 3..8 us (3x3
-    // 128->256 @26x26, 64->128 @52x52 with pooling), 212..252 still lose 1..4 us
     return knob == 2 || rest <= 11 * NUM_CU / 16;
 }
 
@@ -2012,8 +2167,10 @@ struct GroupSlabs
 // The equal-share split of a launch: fills the sk_* fields and the tile counts; returns the scratch bytes it needs, 0 when
 // the shape does not qualify.  Few tiles that do not fill whole rounds and a long reduction (measured, batch 16 on 13x13
 // maps: 512 -> 1024 3x3 287 -> 264 us, 1024 -> 1024 519 -> 467 us, 256 -> 512 (144 steps) 81 -> 69 us; with 72 steps or
-// fewer the fix-up pass costs more than the balance gains).  SMALL_HIP_TUNE keys conv_streamk=<workgroups per compute
-// unit> (default 3: 512 -> 1024 @13x13 b16 200.8 -> 198.2 us, 1024 -> 1024 420 -> 416 against 2; 0 = never), conv_streamk_min=<steps> (default 128)
+// fewer the fix-up pass costs more than the balance gains).  Those are float32 MFMAs; with split products, without -> with, batch
+// 16: 512 -> 1024 162.9 -> 158.2 us, 1024 -> 1024 319.6 -> 301.3, 256 -> 512 52.8 -> 50.2 (batch 26, 20 tiles over a round: 67.0 -> 73.6),
+// and with 72 steps 40.9 -> 50.2.  SMALL_HIP_TUNE keys conv_streamk=<workgroups per compute unit> (default 3, against 2 level to 3% better; 0 = never),
+// conv_streamk_min=<steps> (default 128)
 template <int COT, int PXT>
 size_t streamk_plan(ConvArgs &a)
 {
@@ -2055,8 +2212,9 @@ int launch_streamk(const char *op, ConvArgs &a, hipStream_t s, bool *done)
     return SMALL_HIP_OK;
 }
 
-// few tiles and a long reduction: K split over the four waves of a workgroup (measured: from one tile per SIMD the
-// whole-rounds + tail kernel with 1x1 wave tiles is ahead, e.g. 256->512 3x3 @13x13 batch 16, 1360 tiles: 81 us against 91 us)
+// few tiles and a long reduction: K split over the 4, 8 or 16 waves of a workgroup.  From one tile per SIMD the whole-rounds +
+// tail kernel with 1x1 wave tiles is ahead: 3x3 128->256 @13x13 (72 K-steps) batch 24 (0.99 tiles) 22.6 us split, 24.9 whole, batch 28
+// (1.16) 27.0, 24.8; below sixteen K-steps always (192 -> 128 1x1 @20x20 batch 16, twelve: 7.5, 6.8)
 inline bool wants_splitk(long tiles32, int nsteps)
 {
     static const int force = tune_int("conv_splitk", -1);
@@ -2206,8 +2364,12 @@ void launch_mfma_pool(ConvArgs &a, hipStream_t s)
         if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_hybrid_kernel<COT, PXT, true, false, true>), dim3(n_main + rest * 4 * COT * PXT), dim3(256), 0, s, a);
         else hipLaunchKernelGGL((conv_mfma_f32_hybrid_kernel<COT, PXT, true>), dim3(n_main + rest * 4 * COT * PXT), dim3(256), 0, s, a);
     }
-    else if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_lds_kernel<COT, PXT, true, false, true>), dim3(a.per_xcd * NUM_XCD), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((conv_mfma_f32_lds_kernel<COT, PXT, true>), dim3(a.per_xcd * NUM_XCD), dim3(256), 0, s, a);
+    else
+    {
+        const dim3 grid(a.per_xcd * NUM_XCD);
+        if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_lds_kernel<COT, PXT, true, false, true>), grid, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((conv_mfma_f32_lds_kernel<COT, PXT, true>), grid, dim3(256), 0, s, a);
+    }
 }
 
 // Conv2D + bias + activation + MaxPool2D 2x2 stride 2 (no pool padding) in one launch
