@@ -2108,7 +2108,11 @@ bool tail_pays(int n_main, int rest, int nsteps)
 //   2x1  from 2.25 tiles per SIMD (2 with 72 K-steps; below, the balance of few tiles counts more): 1024 -> 1024 1x1 @7x7 batch 64
 //        (3.1 tiles) 57.3 -> 47.2 us, 512 -> 512 1x1 @14x14 batch 24 (2.3) 21.6 -> 20.4, batch 16 (1.5) 15.2 -> 17.4; where an odd
 //        last channel tile costs at most a tenth (208 channels @21x27 batch 40 75.3 -> 69.3), or a fifth from 16 K-steps on (160
-//        channels 3x3 50.1 -> 47.2, 1x1 of 64 channels 15.0 -> 16.3).
+//        channels 3x3 50.1 -> 47.2, 1x1 of 64 channels 15.0 -> 16.3).  Below 16 K-steps from 3.25: at 2.3 to 3.2 tiles 1x1 is
+//        ahead (64 -> 128 1x1 @7x7 batch 385 (2.3) 7.0 us, 2x1 7.6; 128 -> 512 @28x29 batch 8 (3.2) 10.5, 11.7), from 3.4 on behind
+//        (192 -> 256 @14x14 batch 80 (3.8) 2x1 0.91 of 1x1's time).  Never with one to three, which are bound by their tensors:
+//        there the fewer registers of 1x1 keep more loads in flight (16 -> 128 @28x28 batch 64 9.4, 10.5; 32 -> 64 @56x56 17.3, 18.3;
+//        48 -> 128 @28x28 11.5, 12.9; 32 -> 512 @28x28 batch 10 7.8, 8.0; 48 -> 512 the other way round, 8.6, 8.3).
 //   1x2  otherwise from 4 tiles per SIMD and 16 K-steps (96 channels 3x3 @30x30 batch 64 71.0 -> 68.2, batch 16 (1.3) 23.5 -> 25.1,
 //        32 channels @56x56 31.4 -> 29.2).
 inline void wave_tile(int Co, long tiles32, int nsteps, int *cot, int *pxt)
@@ -2117,8 +2121,9 @@ inline void wave_tile(int Co, long tiles32, int nsteps, int *cot, int *pxt)
     const int c32 = (Co + 31) / 32, pairs = (c32 + 1) / 2;
     const bool little = 20 * pairs <= 11 * c32 || (5 * pairs <= 3 * c32 && nsteps >= 16);   // channel tiles that do not exist
     *cot = *pxt = 1;
+    if (nsteps <= 3) return;
     if (Co % 64 == 0 && tiles32 >= 16 * simds && nsteps >= 32) *cot = *pxt = 2;
-    else if (little && (4 * tiles32 >= 9 * simds || (tiles32 >= 2 * simds && nsteps >= 72))) *cot = 2;
+    else if (little && (4 * tiles32 >= (nsteps >= 16 ? 9 : 13) * simds || (tiles32 >= 2 * simds && nsteps >= 72))) *cot = 2;
     else if (tiles32 >= 4 * simds && nsteps >= 16) *pxt = 2;
 }
 
