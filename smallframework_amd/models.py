@@ -20,6 +20,7 @@ import numpy as np
 from . import capi, layout, synth
 
 CB = 16
+ACTS = {None: capi.ACT_NONE, "relu": capi.ACT_RELU, "leaky": capi.ACT_LEAKY}
 
 
 @dataclass
@@ -418,7 +419,6 @@ class HipExecutor:
             self.plan.append((at(op), at(acc_op) if acc_op else None, relu))
             i = j
         self.out_name = phys.get(model.out, model.out)
-        self.calls = [(self._call_of(entry), entry) for entry in self.plan]
         torch.cuda.synchronize()
 
     @staticmethod
@@ -473,13 +473,25 @@ class HipExecutor:
     def run_entry(self, entry, st):
         """One launch of the plan: a single op, or a fused group."""
         op, acc_op, relu = entry
-        call = self._call_of(entry)
-        if call is not None:
-            self._issue(call, st)
+        if acc_op is not None and acc_op.kind == "maxpool":
+            self.run_conv_pool_f32(op, acc_op, st)
+        elif acc_op is not None and acc_op.kind == "dw":
+            self.run_conv_dw_f32(op, acc_op, st)
         elif acc_op is not None or relu:
             self.run_fused_u8(op, acc_op, relu, st)
         else:
             self.run_op(op, st)
+
+    # The launches of a batch-1 pass take about as long as the host needs to issue them (MobileNetV1: 25 launches in 125 us), so
+    # the float32 methods pass plain addresses (no c_void_p objects) and look each thing up once.
+    def run_conv_pool_f32(self, op, pool, st):
+        """Conv2D + activation + MaxPool2D 2x2 stride 2 in one launch."""
+        b = self.buf
+        rc = self.lib.small_hip_conv2d_bias_act_maxpool2d_f32(
+            self.batch, op.kh, op.kw, op.stride, *op.pads, 2, 2, 2, 0, 0, 0, 0, op.Co, op.C, op.H, op.W,
+            b[op.src].data_ptr(), self.w[op.weight].data_ptr(), None, ACTS[op.act], op.slope, b[pool.dst].data_ptr(), st)
+        if rc:
+            capi.check(rc)
 
     @staticmethod
     def _first_layer_dw(op, dw):
@@ -507,74 +519,53 @@ class HipExecutor:
         fill = hd * wd / float(-(-hd // toh) * toh * -(-wd // tow) * tow)
         return fill >= 0.7
 
-    def _call_of(self, entry):
-        """What a launch of the fused float32 plan passes to the library besides the addresses: (function, leading sizes,
-        source buffer, weight names (None: no bias), trailing scalars, destination buffer).  Put together once: the launches of
-        a batch-1 pass are as long as the host takes to issue them (MobileNetV1: 25 launches, 143 us a pass against 129 on the GPU).
-        None for what run_op / run_fused_u8 issue."""
-        op, second, _ = entry
-        if not self.fused or self.model.dtype != "f32" or op.kind not in ("conv", "dw", "dense", "maxpool", "avgpool"):
-            return None
-        L, B = self.lib, self.batch
-        act = {None: capi.ACT_NONE, "relu": capi.ACT_RELU, "leaky": capi.ACT_LEAKY}[op.act]
-        window = (B, op.kh, op.kw, op.stride) + tuple(op.pads)
-        if op.kind == "dense":
-            return L.small_hip_dense_f32, (B, op.Co, op.C), op.src, (op.weight,), (), op.dst
-        if op.kind in ("maxpool", "avgpool"):
-            fn = L.small_hip_maxpool2d_f32 if op.kind == "maxpool" else L.small_hip_avgpool2d_f32
-            return fn, window + (op.C, op.H, op.W), op.src, (), (), op.dst
-        if op.kind == "dw":
-            return L.small_hip_depthwise_conv2d_bias_act_f32, window + (op.C, op.H, op.W), op.src, (op.weight, None), (act, op.slope), op.dst
-        sizes = (op.Co, op.C, op.H, op.W)
-        if second is None:
-            return L.small_hip_conv2d_bias_act_f32, window + sizes, op.src, (op.weight, None), (act, op.slope), op.dst
-        if second.kind == "maxpool":             # Conv2D + activation + MaxPool2D 2x2 stride 2 in one launch
-            return (L.small_hip_conv2d_bias_act_maxpool2d_f32, window + (2, 2, 2, 0, 0, 0, 0) + sizes, op.src, (op.weight, None),
-                    (act, op.slope), second.dst)
-        # Conv2D + activation + DepthwiseConv2D 3x3 + activation in one launch
-        return (L.small_hip_conv2d_bias_act_dwconv2d_bias_act_f32, window + (3, 3, second.stride) + tuple(second.pads) + sizes, op.src,
-                (op.weight, None, second.weight, None), (act, op.slope), second.dst)
-
-    def _issue(self, call, st):
-        """The buffers and weights are looked up at every launch: a caller may put another tensor into `buf` or `w`."""
-        fn, head, src, weights, tail, dst = call
-        w = [None if k is None else self.w[k].data_ptr() for k in weights]
-        rc = fn(*head, self.buf[src].data_ptr(), *w, *tail, self.buf[dst].data_ptr(), st)
+    def run_conv_dw_f32(self, op, dw, st):
+        """Conv2D + activation + DepthwiseConv2D 3x3 + activation in one launch."""
+        b, w = self.buf, self.w
+        rc = self.lib.small_hip_conv2d_bias_act_dwconv2d_bias_act_f32(
+            self.batch, op.kh, op.kw, op.stride, *op.pads, 3, 3, dw.stride, *dw.pads, op.Co, op.C, op.H, op.W,
+            b[op.src].data_ptr(), w[op.weight].data_ptr(), None, w[dw.weight].data_ptr(), None, ACTS[op.act], op.slope,
+            b[dw.dst].data_ptr(), st)
         if rc:
             capi.check(rc)
 
     def run_op(self, op: Op, st):
-        call = self._call_of((op, None, False))
-        if call is not None:
-            self._issue(call, st)
-            return
-        L, p, B, b = self.lib, self._p, self.batch, self.buf
-        src, dst = b[op.src], b[op.dst]
-        t_, b_, l_, r_ = op.pads
+        L, B, kind = self.lib, self.batch, op.kind
         if self.model.dtype == "f32":
-            if op.kind == "conv":
-                args = (B, op.kh, op.kw, op.stride, t_, b_, l_, r_, op.Co, op.C, op.H, op.W)
-                rc = L.small_hip_conv2d_f32(*args, p(src), p(self.w[op.weight]), p(dst), st)
-                rc = rc or self._act_f32(op, dst, st)
-            elif op.kind == "dense":
-                rc = L.small_hip_dense_f32(B, op.Co, op.C, p(src), p(self.w[op.weight]), p(dst), st)
-            elif op.kind == "dw":
-                args = (B, op.kh, op.kw, op.stride, t_, b_, l_, r_, op.C, op.H, op.W)
-                rc = L.small_hip_depthwise_conv2d_f32(*args, p(src), p(self.w[op.weight]), p(dst), st)
-                rc = rc or self._act_f32(op, dst, st)
-            elif op.kind in ("maxpool", "avgpool"):
-                fn = L.small_hip_maxpool2d_f32 if op.kind == "maxpool" else L.small_hip_avgpool2d_f32
-                rc = fn(B, op.kh, op.kw, op.stride, t_, b_, l_, r_, op.C, op.H, op.W, p(src), p(dst), st)
-            elif op.kind == "relu":
-                rc = L.small_hip_relu_f32(B, op.C, op.H, op.W, p(src), p(dst), st)
-            elif op.kind == "leaky":
-                rc = L.small_hip_leaky_relu_f32(B, op.C, op.H, op.W, p(src), op.slope, p(dst), st)
-            elif op.kind == "accum":
-                rc = L.small_hip_accum_f32(B, op.C, op.H, op.W, p(src), p(dst), st)
+            src, dst = self.buf[op.src].data_ptr(), self.buf[op.dst].data_ptr()
+            if kind == "conv":
+                w = self.w[op.weight].data_ptr()
+                if self.fused:
+                    rc = L.small_hip_conv2d_bias_act_f32(B, op.kh, op.kw, op.stride, *op.pads, op.Co, op.C, op.H, op.W, src, w, None,
+                                                         ACTS[op.act], op.slope, dst, st)
+                else:
+                    rc = L.small_hip_conv2d_f32(B, op.kh, op.kw, op.stride, *op.pads, op.Co, op.C, op.H, op.W, src, w, dst, st)
+                    rc = rc or self._act_f32(op, dst, st)
+            elif kind == "dense":
+                rc = L.small_hip_dense_f32(B, op.Co, op.C, src, self.w[op.weight].data_ptr(), dst, st)
+            elif kind == "dw":
+                w = self.w[op.weight].data_ptr()
+                if self.fused:
+                    rc = L.small_hip_depthwise_conv2d_bias_act_f32(B, op.kh, op.kw, op.stride, *op.pads, op.C, op.H, op.W, src, w, None,
+                                                                   ACTS[op.act], op.slope, dst, st)
+                else:
+                    rc = L.small_hip_depthwise_conv2d_f32(B, op.kh, op.kw, op.stride, *op.pads, op.C, op.H, op.W, src, w, dst, st)
+                    rc = rc or self._act_f32(op, dst, st)
+            elif kind in ("maxpool", "avgpool"):
+                fn = L.small_hip_maxpool2d_f32 if kind == "maxpool" else L.small_hip_avgpool2d_f32
+                rc = fn(B, op.kh, op.kw, op.stride, *op.pads, op.C, op.H, op.W, src, dst, st)
+            elif kind == "relu":
+                rc = L.small_hip_relu_f32(B, op.C, op.H, op.W, src, dst, st)
+            elif kind == "leaky":
+                rc = L.small_hip_leaky_relu_f32(B, op.C, op.H, op.W, src, op.slope, dst, st)
+            elif kind == "accum":
+                rc = L.small_hip_accum_f32(B, op.C, op.H, op.W, src, dst, st)
             else:
                 raise ValueError(op.kind)
         else:
-            q = self.q
+            p, b, q = self._p, self.buf, self.q
+            src, dst = b[op.src], b[op.dst]
+            t_, b_, l_, r_ = op.pads
             iq, oq = C.byref(q[op.src]), C.byref(q[op.dst])
             if op.kind in ("conv", "dense"):
                 kh, kw, s = (op.kh, op.kw, op.stride) if op.kind == "conv" else (1, 1, 1)
@@ -596,23 +587,21 @@ class HipExecutor:
                 rc = L.small_hip_accum_u8(B, op.C, op.H, op.W, p(src), iq, p(dst), oq, st)
             else:
                 raise ValueError(op.kind)
-        capi.check(rc)
+        if rc:
+            capi.check(rc)
 
     def _act_f32(self, op, dst, st):
         c, h, w = op.out_shape()
         if op.act == "relu":
-            return self.lib.small_hip_relu_f32(self.batch, c, h, w, self._p(dst), self._p(dst), st)
+            return self.lib.small_hip_relu_f32(self.batch, c, h, w, dst, dst, st)
         if op.act == "leaky":
-            return self.lib.small_hip_leaky_relu_f32(self.batch, c, h, w, self._p(dst), op.slope, self._p(dst), st)
+            return self.lib.small_hip_leaky_relu_f32(self.batch, c, h, w, dst, op.slope, dst, st)
         return 0
 
     def forward(self):
         st = self.stream()
-        for call, entry in self.calls:
-            if call is not None:
-                self._issue(call, st)
-            else:
-                self.run_entry(entry, st)
+        for entry in self.plan:
+            self.run_entry(entry, st)
 
     # ---- the whole model in one launch (uint8 models whose tensors and filters fit one CU's LDS) --------------
     def qmodel_layers(self):
@@ -659,13 +648,12 @@ class HipExecutor:
         ops = self.model.ops
         ids = {"in": capi.QM_INPUT}
         layers = (capi.FLayer * len(ops))()
-        act = {None: capi.ACT_NONE, "relu": capi.ACT_RELU, "leaky": capi.ACT_LEAKY}
         for i, op in enumerate(ops):
             L = layers[i]
             L.src = ids[op.src] if op.src in ids else ids.setdefault(op.src, len(ids) - 1)
             L.dst = capi.QM_OUTPUT if i == len(ops) - 1 else (ids[op.dst] if op.dst in ids else ids.setdefault(op.dst, len(ids) - 1))
             L.input_channels, L.input_height, L.input_width = op.C, op.H, op.W
-            L.act, L.slope = act[op.act], op.slope
+            L.act, L.slope = ACTS[op.act], op.slope
             L.kernel_height, L.kernel_width, L.stride = op.kh, op.kw, op.stride
             L.t_pad, L.b_pad, L.l_pad, L.r_pad = op.pads
             if op.kind in ("conv", "dense"):

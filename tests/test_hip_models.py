@@ -202,3 +202,50 @@ def test_hip_graph_replays_match_eager(name, batch):
             assert_equal_exact(got, want, "graph replay %d" % rep)
         torch.cuda.synchronize()
     assert eager.shape == got.shape
+
+
+def test_forward_follows_the_executor():
+    """forward() issues what `plan`, `fused` and the ops say at the time of the call, through run_entry."""
+    import torch
+    model = models.mobilenet_v1()
+    ex = models.HipExecutor(model, 1)
+    ex.forward()
+    want = ex.output()
+    plan = ex.plan
+    assert any(second is not None for _, second, _ in plan)              # a fused pair: two ops in one launch
+
+    seen = []
+    class Traced(models.HipExecutor):
+        def run_entry(self, entry, st):
+            seen.append(entry)
+            super().run_entry(entry, st)
+    ex.__class__ = Traced
+    ex.buf[ex.out_name].zero_()
+    ex.forward()
+    assert len(seen) == len(plan) and np.array_equal(ex.output(), want)
+    ex.__class__ = models.HipExecutor
+
+    ex.fused = False                                                     # separate activations; the plan's pairs stay pairs
+    ex.buf[ex.out_name].zero_()
+    ex.forward()
+    assert_close_f32(ex.output(), want, what="activations as launches of their own")
+    ex.fused = True
+
+    first = plan[0][1] if plan[0][1] is not None else plan[0][0]
+    for name, t in ex.buf.items():
+        if name != "in":
+            t.zero_()
+    ex.plan = plan[:1]
+    ex.forward()
+    torch.cuda.synchronize()
+    assert all(bool(t.any()) == (name == first.dst) for name, t in ex.buf.items() if name != "in")
+
+    ex.plan = plan
+    conv = plan[-3][0]
+    assert (conv.kind, conv.act) == ("conv", "relu")
+    conv.act = None                                                      # an op changed after the executor was built
+    ex.forward()
+    assert not np.array_equal(ex.output(), want)
+    conv.act = "relu"
+    ex.forward()
+    assert np.array_equal(ex.output(), want)
