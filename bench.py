@@ -24,7 +24,9 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 PEAK_HBM = 8.0e12          # B/s, MI355X HBM3E
-PEAK_MFMA_F32 = 157.3e12   # FLOP/s, dense fp32 MFMA
+PEAK_MFMA_F32 = 157.3e12   # FLOP/s, dense fp32 MFMA (the whole-model float32 kernel)
+PEAK_MFMA_BF16 = 2.5e15    # FLOP/s, dense bf16 MFMA
+PEAK_SPLIT_F32 = PEAK_MFMA_BF16 / 6   # float32 convolutions with 16 or more input channels: six bf16 products each
 PEAK_MFMA_I8 = 5.0e15      # OP/s, dense int8 MFMA
 
 # HBM bytes per launch of the dominant kernel come from the committed counter summary (rocprofv3 --pmc FETCH_SIZE and
@@ -139,7 +141,7 @@ def op_bytes(model, op, batch):
 def op_bound(model, op, batch):
     """-> (seconds at the roofline, 'hbm' | 'mfma')."""
     t_hbm = op_bytes(model, op, batch) / PEAK_HBM
-    peak = PEAK_MFMA_F32 if model.dtype == "f32" else PEAK_MFMA_I8
+    peak = PEAK_SPLIT_F32 if model.dtype == "f32" else PEAK_MFMA_I8
     on_mfma = op.kind in ("conv", "dense") and op.C % 16 == 0
     t_mfma = batch * op.flops() / peak if on_mfma else 0.0
     return (t_mfma, "mfma") if t_mfma > t_hbm else (t_hbm, "hbm")
@@ -253,7 +255,7 @@ def layer_table(model, batch, ms):
             nbytes = batch * (op.act_elems()[0] + ops[i + 1].act_elems()[1]) * es + \
                 (op.weight_elems() + ops[i + 1].weight_elems()) * es
             # the fused launch's own roofline: its bytes at the HBM peak, or the convolution's flops at the MFMA peak
-            t_mfma = batch * op.flops() / (PEAK_MFMA_F32 if model.dtype == "f32" else PEAK_MFMA_I8) if op.C % 16 == 0 else 0.0
+            t_mfma = batch * op.flops() / (PEAK_SPLIT_F32 if model.dtype == "f32" else PEAK_MFMA_I8) if op.C % 16 == 0 else 0.0
             tb, kind = (t_mfma, "mfma") if t_mfma > nbytes / PEAK_HBM else (nbytes / PEAK_HBM, "hbm")
         rows.append({"layer": op.name, "ms": round(t, 5), "bound": kind,
                      "roofline_frac": round(tb / (t * 1e-3), 4) if t > 0 else None,
@@ -546,7 +548,7 @@ def sweep_only(args, torch, models):
            "dtype": "f32", "data": "synthetic",
            "config": {"workload": "single layers at C=256, 56x56, batch %d: Conv2D 3x3 s1 same, DepthwiseConv2D "
                                   "3x3 s1, MaxPool2D 3x3 s2 valid, ReLU" % batch, "batch": batch},
-           "roofline": {"bound": "mfma", "achieved": r["TFLOP/s"], "peak": round(PEAK_MFMA_F32 / 1e12, 1),
+           "roofline": {"bound": "mfma", "achieved": r["TFLOP/s"], "peak": round(PEAK_SPLIT_F32 / 1e12, 1),
                         "unit": "TFLOP/s", "frac": r["roofline_frac"], "traffic": None,
                         "kernel": "conv_mfma_f32_*", "launches_per_step": 1, "avg_launch_ms": r["ms"],
                         "algorithmic_per_launch": {"GFLOP": round(batch * op.flops() / 1e9, 3),
@@ -684,7 +686,7 @@ def main():
     dom = max(per_kernel, key=lambda k: per_kernel[k]["ms"])
     d = per_kernel[dom]
     if "mfma" in dom:
-        peak = (PEAK_MFMA_F32 if model.dtype == "f32" else PEAK_MFMA_I8) / 1e12
+        peak = (PEAK_SPLIT_F32 if model.dtype == "f32" else PEAK_MFMA_I8) / 1e12
         ach = d["flops"] / (d["ms"] * 1e-3) / 1e12
         roof = {"bound": "mfma", "achieved": round(ach, 2), "peak": round(peak, 1), "unit": "TFLOP/s",
                 "frac": round(ach / peak, 4), "traffic": None}
@@ -720,7 +722,7 @@ def main():
                 "note": "instruction-, LDS- and latency-bound: one workgroup per image, 16 waves per compute unit, only "
                         "`batch` of the 256 compute units busy"}
     if model.dtype == "f32" and not args.no_extras:
-        # what the float32 matrix pipes sustain on registers alone, beside the published peak used in `roofline`
+        # what the float32 MFMA instructions sustain on registers alone, beside their published peak (the whole-model kernel uses them)
         extras.update(calib)
         extras["fresh_process_ms_per_step"] = round(fresh * 1e3, 4)
         # the same forward pass replayed from a HIP graph (no host work between the launches)
