@@ -45,7 +45,9 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // float32 products on the bf16 matrix pipes.  A float32 number is the exact sum of three bf16 numbers, x = h + m + l: h =
 // bf16(x) and m = bf16(x - h), both rounded to nearest, l = x - h - m, at most eight bits (|m| <= 2^-8 |x|, |l| <= 2^-17 |x|,
 // either sign), and a product of two bf16 numbers is exact in float32.  x * y is then added up as
-// hh + (hm + mh + mm + hl + lh); what is left out, ml + lm + ll, is at most 2^-24 |x y| and 5e-9 of it root mean square.
+// hh + (hm + mh + mm + hl + lh) (three parts and six products: Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations", ARITH 2019); what is left out, ml + lm + ll, is at most 2^-24 |x y|
+// and 5e-9 of it root mean square.
 // v_mfma_f32_32x32x16_bf16 multiplies sixteen times as fast as v_mfma_f32_32x32x2_f32, six of them replace eight float32
 // ones per sixteen channels: 192 matrix cycles instead of 512, and the vector ALU may issue beside them (a float32 MFMA
 // occupies it).  Nine products less ll would leave nothing out but take 256 cycles: 3x3 256->256 @56x56 batch 64 1137 -> 1404 us,
@@ -2652,9 +2654,10 @@ int small_hip_conv2d_dwconv2d_one_launch_f32(int batch, int kh, int kw, int stri
         return nt <= 0x7fffffffL && (long)batch * Co * Ho * Wo <= 0x7fffffffL * 4L ? 1 : 0;
     }
     // a pointwise convolution parked in LDS under 14 x 14 (stride 2: 7 x 8) depthwise tiles (pw_dw_f32): short reductions
-    // on maps that fill those tiles to 70%, where the recomputed halo costs less than the second launch.  Measured on
-    // MobileNetV1's pairs at batch 64: 32 -> 64 @112x112 stride 2 104 -> 54 us, 64 -> 128 @56x56 70 -> 54 us, 128 -> 256
-    // @28x28 53 -> 46 us; 128 -> 128 @56x56 stride 2 81 -> 85 us (two launches stay)
+    // on maps that fill those tiles to 70%, where the recomputed halo costs less than the second launch.  Batch 64:
+    // 32 -> 64 @112x112 stride 2 113 -> 51 us, 64 -> 128 @56x56 67 -> 48, 128 -> 256 @28x28 45 -> 37, 96 -> 192 @28x28
+    // 34 -> 25.  96 and 128 channels at stride 2 stay two launches from when the products were float32 MFMAs (128 -> 128
+    // @56x56 81 -> 85 us); with split bf16 products that pair is 70 -> 59
     if (kh != 1 || kw != 1 || stride != 1 || pt || pb || pl || pr || Ci % CB != 0 || Co % 32 != 0 || (dw_stride != 1 && dw_stride != 2))
         return 0;
     const int cib = Ci / CB;

@@ -394,8 +394,8 @@ __global__ __launch_bounds__(256) void conv_mfma_u8_kernel(const QConvArgs a0)
 // into the padding: no instruction per load is spent on the border, and the lane's offset and constant change with the tap only.
 // What bounds it: matrix cycles, eight vector instructions per 16-byte load (raw sum, exclusive or) and about twelve per
 // output value (requantisation), and on small launches the latency of one load per round; the 16x16 tiles above pay for their
-// addresses in every step and read their filter operand once per wave.  96 -> 96 3x3 @30x30 batch 64: 26.9 -> 12.2 us
-// (780 TOP/s), 64 -> 64 @56x56 batch 64 35.1 -> 21.2, 512 -> 512 1x1 @14x14 batch 16 10.9 -> 5.9.
+// addresses in every step and read their filter operand once per wave.  96 -> 96 3x3 @30x30 batch 64: 25.8 -> 12.0 us
+// (800 TOP/s), 64 -> 64 @56x56 batch 64 33.9 -> 20.7, 512 -> 512 1x1 @14x14 batch 16 10.3 -> 5.7.
 typedef int v16i __attribute__((ext_vector_type(16)));
 
 template <int CT, int PXT, int KP, bool ODD>
@@ -918,6 +918,8 @@ int conv_u8_run(const char *op, int batch, int kh, int kw, int stride, int pt, i
     // kernel above, 5.9 on this; 16 -> 176 5x5 @50x50 batch 20, 46%: 32.8 and 22.1), 16 -> 16 channels never pay (5.7, 6.4).
     // A few workgroups with a short reduction are a matter of latency (64 -> 128 3x3 @20x20 batch 2, 28 workgroups of 18 pairs:
     // 4.9 us above, 5.4 here; 1024 -> 64 1x1 @40x40 batch 2, 26 of 32 pairs: 6.5 and 6.2).
+    // (These times and the ones below are of one sweep with every width forced in turn; in it everything runs some 4% longer
+    // than in the run whose figures stand at the kernel.)
     // Channels per workgroup: fewer products on channels that do not exist, then more tiles per activation read (a
     // tile's own work is about twice the overhead of a pair), from 1.5 workgroups per compute unit on: 96 -> 96 3x3
     // @30x30 batch 64 26.9 us on the kernel above, 15.0 / 16.5 / 12.2 with 32 / 64 / 96 channels; batch 7 8.2, 6.1 / 7.4 / 8.9;
