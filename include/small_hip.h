@@ -21,7 +21,8 @@
  *     them exactly, and leave out products of at most 2^-24 of a float32 product: a sum of two or more products is as close
  *     to the exact result as float32 products rounded and added in some order (long sums are closer), a single product is
  *     within 1.7 * 2^-24 of itself instead of 2^-24.  Infinities, NaN, overflow and sums below 2^-64 are as float32 products
- *     give them; an operand below 2^-110 times one above 2^40 keeps an absolute error of 2^-133 times the latter.
+ *     give them, but for the part of an operand below 2^-133 (only operands below 2^-110 have one), which is lost where the
+ *     other factor is above 2^40 or the sum is zero without it.
  *   - Pads are given in the reference's public order: top, bottom, left, right.
  *   - Output height/width follow include/small/utils.hpp:159-165 applied to the padded input.
  *   - `stream` is a hipStream_t (NULL = the default stream).  Calls are asynchronous with

@@ -65,7 +65,8 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // Range: operands from 2^-110 up are split exactly.  Sums that are not finite, or below 2^-64 without being zero, are made
 // again with float32 MFMAs (split_odd, mfma_f32_wave): infinities and NaN of any payload, operands next to the largest finite
 // number, whose h is infinite, and operands or products among the smallest give what float32 products give.  What is
-// left: an operand below 2^-110 that is multiplied by one above 2^40 has an absolute error of 2^-133 times the latter.
+// left: the part of an operand below 2^-133, which only operands below 2^-110 have, is lost where the other factor is above 2^40 or
+// the sum is zero without it: an absolute error of 2^-133 times the other factor.
 constexpr float SPLIT_LEAST = 0x1p-64f;
 
 struct Split8

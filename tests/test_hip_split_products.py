@@ -113,7 +113,7 @@ def test_infinities_and_nan_as_float32(shape):
 
 
 def test_range():
-    """Magnitudes from 2^-100 to 2^100: float32 precision; below 2^-110 an absolute error of 2^-134 of the other factor."""
+    """Magnitudes from 2^-100 to 2^100: float32 precision; below 2^-110 an absolute error of 2^-133 of the other factor."""
     shape = (1, 1, 1, 16, 16, 4, 8)
     f = np.eye(16, dtype=np.float32).reshape(16, 16, 1, 1)
     x = synth.normal(31, 16 * 32).reshape(1, 16, 4, 8)
