@@ -28,6 +28,7 @@
 
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <vector>
 
@@ -68,8 +69,9 @@ struct FMHeader
     int n_layers;
     int in_C, in_H, in_W, in_off;        // the model input and the LDS float offset it is staged at
     int w_lds, w_floats;                 // weights: two buffers of w_floats floats at float offset w_lds
-    int pool_off;                        // 4096 + 512 floats of pooling partials
-    int zero_off;                        // 16 bytes of zeros: what a tap outside the image reads
+    int zero_off;                        // 16 bytes of zeros: what a tap outside the image reads; behind them a word of the band kernel
+    // band kernel: layers before the whole-image pooling, floats / pixels of the last one's output and where it lies in LDS
+    int n_band, band_elems, band_P, band_off;
     int in_elems, out_elems;             // floats per image in global memory
     int lds_bytes;
     FMLayer layer[MAX_LAYERS];
@@ -90,6 +92,31 @@ __device__ __forceinline__ float act_bf(float v, float neg_scale)
 {
     const float n = fmaf(v, neg_scale, 0.f);      // "+ 0": the -0 of x * 0 becomes the +0 ReLU gives
     return v > 0.f ? v : n;
+}
+
+// Values that another workgroup of the same launch reads: written through to where every XCD sees them and read from there,
+// eight bytes at a time (a fence of the whole device instead writes back and drops an L2 per wave: 3 us a band).
+__device__ __forceinline__ void store_shared(float *g, float4 v)
+{
+    unsigned long long *d = reinterpret_cast<unsigned long long *>(g);
+    const uint4 u = __builtin_bit_cast(uint4, v);
+    __hip_atomic_store(d, u.x | (unsigned long long)u.y << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(d + 1, u.z | (unsigned long long)u.w << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float4 load_shared(const float *g)
+{
+    const unsigned long long *d = reinterpret_cast<const unsigned long long *>(g);
+    const unsigned long long a = __hip_atomic_load(d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long b = __hip_atomic_load(d + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_bit_cast(float4, make_uint4((unsigned)a, (unsigned)(a >> 32), (unsigned)b, (unsigned)(b >> 32)));
+}
+
+// a layer's result quad outside LDS: the model output, or (dst_off == TO_SLOT) a tensor that the bands put together
+constexpr int TO_OUTPUT = -1, TO_SLOT = -2;
+__device__ __forceinline__ void store_out(const FMLayer &L, float *g, float4 v)
+{
+    if (L.dst_off == TO_SLOT) store_shared(g, v);
+    else *reinterpret_cast<float4 *>(g) = v;
 }
 
 // ---- model creation: weights into operand order ---------------------------------------------------------------
@@ -133,12 +160,12 @@ __global__ __launch_bounds__(256) void fm_prep_kernel(int kind, const float *__r
 // its first MFMA, so a chunk pays the LDS latency once; a tap outside the image reads the block of zeros.
 template <int TP>
 __device__ __forceinline__ void conv_layer(const FMLayer &L, float *lds, const float *wl, const float *zero, float *gout,
-                                           int wave, int lane)
+                                           int wave, int lane, int p0, int p1)
 {
     const int col = lane & 15, kq = lane >> 4;
     const int CoB = L.Co / CB, CiB = L.Ci / CB, S = L.kh * L.kw * CiB;
     const int Pin = L.H * L.W, P = L.Ho * L.Wo;
-    const int n_pt = (P + 15) >> 4, n_grp = (n_pt + TP - 1) / TP, n_work = n_grp * CoB;
+    const int n_pt = (p1 - p0 + 15) >> 4, n_grp = (n_pt + TP - 1) / TP, n_work = n_grp * CoB;
     const float *src = lds + L.src_off;
     for (int work = wave; work < n_work; work += NW)
     {
@@ -149,9 +176,9 @@ __device__ __forceinline__ void conv_layer(const FMLayer &L, float *lds, const f
 #pragma unroll
         for (int t = 0; t < TP; ++t)
         {
-            p[t] = (pg * TP + t) * 16 + col;
-            pv[t] = p[t] < P;
-            const int pc = pv[t] ? p[t] : 0;
+            p[t] = p0 + (pg * TP + t) * 16 + col;
+            pv[t] = p[t] < p1;
+            const int pc = pv[t] ? p[t] : p0;
             const int oh = (int)(((float)pc + 0.5f) * L.r_wo), ow = pc - oh * L.Wo;
             ih0[t] = oh * L.stride - L.pt;
             iw0[t] = ow * L.stride - L.pl;
@@ -205,7 +232,7 @@ __device__ __forceinline__ void conv_layer(const FMLayer &L, float *lds, const f
             const float4 v = make_float4(act_bf(acc[t][0] + bias.x, L.nscale), act_bf(acc[t][1] + bias.y, L.nscale),
                                          act_bf(acc[t][2] + bias.z, L.nscale), act_bf(acc[t][3] + bias.w, L.nscale));
             if (L.dst_off >= 0) *reinterpret_cast<float4 *>(lds + L.dst_off + apos(cob, P, p[t], kq)) = v;
-            else *reinterpret_cast<float4 *>(gout + ((size_t)cob * P + p[t]) * CB + 4 * kq) = v;
+            else store_out(L, gout + ((size_t)cob * P + p[t]) * CB + 4 * kq, v);
         }
     }
 }
@@ -216,20 +243,20 @@ __device__ __forceinline__ void conv_layer(const FMLayer &L, float *lds, const f
 // chunk), and the gathered operand serves TC output-channel blocks.
 template <int TC>
 __device__ __forceinline__ void stem_layer(const FMLayer &L, float *lds, const float *wl, const float *zero, float *gout,
-                                           int wave, int lane)
+                                           int wave, int lane, int p0, int p1)
 {
     const int col = lane & 15, kq = lane >> 4;
     const int CoB = L.Co / CB, P = L.Ho * L.Wo;
-    const int n_pt = (P + 15) >> 4, n_cg = CoB / TC, n_work = n_pt * n_cg;
+    const int n_pt = (p1 - p0 + 15) >> 4, n_cg = CoB / TC, n_work = n_pt * n_cg;
     const float r_ncg = L.r_cob * (float)TC;                 // 1 / n_cg
     const float *src = lds + L.src_off;
     const int4 *ktab = reinterpret_cast<const int4 *>(wl + L.ktab_off);
     for (int work = wave; work < n_work; work += NW)
     {
         const int pt = (int)(((float)work + 0.5f) * r_ncg), cg = work - pt * n_cg;
-        const int p = pt * 16 + col;
-        const bool pv = p < P;
-        const int pc = pv ? p : 0;
+        const int p = p0 + pt * 16 + col;
+        const bool pv = p < p1;
+        const int pc = pv ? p : p0;
         const int oh = (int)(((float)pc + 0.5f) * L.r_wo), ow = pc - oh * L.Wo;
         const int ih0 = oh * L.stride - L.pt, iw0 = ow * L.stride - L.pl;
         floatx4 acc[TC];
@@ -291,7 +318,7 @@ __device__ __forceinline__ void stem_layer(const FMLayer &L, float *lds, const f
             const float4 v = make_float4(act_bf(acc[c][0] + bias.x, L.nscale), act_bf(acc[c][1] + bias.y, L.nscale),
                                          act_bf(acc[c][2] + bias.z, L.nscale), act_bf(acc[c][3] + bias.w, L.nscale));
             if (L.dst_off >= 0) *reinterpret_cast<float4 *>(lds + L.dst_off + apos(cob, P, p, kq)) = v;
-            else *reinterpret_cast<float4 *>(gout + ((size_t)cob * P + p) * CB + 4 * kq) = v;
+            else store_out(L, gout + ((size_t)cob * P + p) * CB + 4 * kq, v);
         }
     }
 }
@@ -300,20 +327,22 @@ __device__ __forceinline__ void stem_layer(const FMLayer &L, float *lds, const f
 // share of the channel blocks.  The window's nine positions (offsets into the block, the zeros for taps outside the
 // image) are worked out once per lane; per channel block a tap costs two 16-byte LDS reads and four multiply-adds.
 template <int KH, int KW>
-__device__ __forceinline__ void dw_layer_win(const FMLayer &L, float *lds, const float *wl, const float *zero, float *gout, int tid)
+__device__ __forceinline__ void dw_layer_win(const FMLayer &L, float *lds, const float *wl, const float *zero, float *gout, int tid,
+                                             int p0, int p1)
 {
     constexpr int T = KH * KW;
     const int CiB = L.Ci / CB;
-    const int Pin = L.H * L.W, P = L.Ho * L.Wo, n_lane = P * 4;
+    const int Pin = L.H * L.W, P = L.Ho * L.Wo, n_lane = (p1 - p0) * 4;
+    const float r_lane = p1 - p0 == P ? L.r_p * 0.25f : 1.0f / (float)n_lane;
     int G = NT / n_lane;                                   // lane groups along the channel blocks
     G = G < 1 ? 1 : (G > CiB ? CiB : G);
     const int per = (CiB + G - 1) / G;                     // channel blocks per group
     const float *src = lds + L.src_off;
     for (int i = tid; i < n_lane * G; i += NT)
     {
-        const int g = (int)(((float)i + 0.5f) * L.r_p * 0.25f);      // i / n_lane
+        const int g = (int)(((float)i + 0.5f) * r_lane);             // i / n_lane
         const int r = i - g * n_lane;
-        const int q = r & 3, p = r >> 2;
+        const int q = r & 3, p = p0 + (r >> 2);
         const int oh = (int)(((float)p + 0.5f) * L.r_wo), ow = p - oh * L.Wo;
         const int ih0 = oh * L.stride - L.pt, iw0 = ow * L.stride - L.pl;
         const int cb0 = g * per, cb1 = cb0 + per < CiB ? cb0 + per : CiB;
@@ -352,7 +381,7 @@ __device__ __forceinline__ void dw_layer_win(const FMLayer &L, float *lds, const
             acc.x = act_bf(acc.x, L.nscale); acc.y = act_bf(acc.y, L.nscale);
             acc.z = act_bf(acc.z, L.nscale); acc.w = act_bf(acc.w, L.nscale);
             if (L.dst_off >= 0) *reinterpret_cast<float4 *>(lds + L.dst_off + dpos) = acc;
-            else *reinterpret_cast<float4 *>(gout + ((size_t)cb * P + p) * CB + 4 * q) = acc;
+            else store_out(L, gout + ((size_t)cb * P + p) * CB + 4 * q, acc);
             w += T * CB; bp += CB; dpos += P * CB;
         }
     }
@@ -463,21 +492,22 @@ __device__ __forceinline__ void dwpw_layer(const FMLayer &L, float *lds, const f
             const float4 v = make_float4(act_bf(acc[c][0] + bias.x, L.nscale2), act_bf(acc[c][1] + bias.y, L.nscale2),
                                          act_bf(acc[c][2] + bias.z, L.nscale2), act_bf(acc[c][3] + bias.w, L.nscale2));
             if (L.dst_off >= 0) *reinterpret_cast<float4 *>(lds + L.dst_off + apos(cob, P, p, kq)) = v;
-            else *reinterpret_cast<float4 *>(gout + ((size_t)cob * P + p) * CB + 4 * kq) = v;
+            else store_out(L, gout + ((size_t)cob * P + p) * CB + 4 * kq, v);
         }
     }
 }
 
 // depthwise convolution, any window: a lane = one output pixel x 4 channels of one block
-__device__ __forceinline__ void dw_layer_any(const FMLayer &L, float *lds, const float *wl, float *gout, int tid)
+__device__ __forceinline__ void dw_layer_any(const FMLayer &L, float *lds, const float *wl, float *gout, int tid, int p0, int p1)
 {
     const int kh = L.kh, kw = L.kw;
-    const int Pin = L.H * L.W, P = L.Ho * L.Wo, n = (L.Ci / CB) * P * 4;
+    const int Pin = L.H * L.W, P = L.Ho * L.Wo, np = p1 - p0, n = (L.Ci / CB) * np * 4;
+    const float r_np = np == P ? L.r_p : 1.0f / (float)np;
     const float *src = lds + L.src_off;
     for (int i = tid; i < n; i += NT)
     {
         const int q = i & 3, r = i >> 2;
-        const int cb = (int)(((float)r + 0.5f) * L.r_p), p = r - cb * P;
+        const int cb = (int)(((float)r + 0.5f) * r_np), p = p0 + r - cb * np;
         const int oh = (int)(((float)p + 0.5f) * L.r_wo), ow = p - oh * L.Wo;
         const int ih0 = oh * L.stride - L.pt, iw0 = ow * L.stride - L.pl;
         const float *w = wl + cb * kh * kw * CB + 4 * q;
@@ -496,7 +526,7 @@ __device__ __forceinline__ void dw_layer_any(const FMLayer &L, float *lds, const
         acc.x = act_bf(acc.x, L.nscale); acc.y = act_bf(acc.y, L.nscale);
         acc.z = act_bf(acc.z, L.nscale); acc.w = act_bf(acc.w, L.nscale);
         if (L.dst_off >= 0) *reinterpret_cast<float4 *>(lds + L.dst_off + apos(cb, P, p, q)) = acc;
-        else *reinterpret_cast<float4 *>(gout + ((size_t)cb * P + p) * CB + 4 * q) = acc;
+        else store_out(L, gout + ((size_t)cb * P + p) * CB + 4 * q, acc);
     }
 }
 
@@ -515,9 +545,8 @@ __device__ __forceinline__ float4 pool_op(bool is_max, float4 acc, float4 v)
 // A wave owns a channel quad (wave, wave + 16, ...): its lanes fold the pixels lane, lane + 64, ... in that order, then
 // the wave folds its 64 partial sums with xor-shuffles (32, 16, ... 1): a fixed order (deterministic), no barrier and no
 // LDS staging inside the layer.  (Three stages through LDS with two barriers took 2.4 us of the DS-CNN's 27.)
-__device__ __forceinline__ void pool_layer(const FMLayer &L, float *lds, float *part, float *gout, int tid)
+__device__ __forceinline__ void pool_layer(const FMLayer &L, float *lds, float *gout, int tid)
 {
-    (void)part;
     const int C4 = L.Ci / 4, P = L.H * L.W;
     const bool is_max = L.kind == K_POOL_MAX;
     const float *src = lds + L.src_off;
@@ -561,6 +590,84 @@ __device__ __forceinline__ void weights_to_lds(const float *g, float *l, int n16
     }
 }
 
+// the image into LDS and the first layer's weights behind it
+__device__ __forceinline__ void stage_image(HeaderPtr hdr, const float *blob, const float *img, float *lds, float *wbuf, int tid, int wave)
+{
+    weights_to_lds(blob + hdr->layer[0].blob_off, wbuf, hdr->layer[0].blob16, tid, wave);
+    float *x = lds + hdr->in_off;
+    if (hdr->in_C < CB)
+        for (int i = tid; i < hdr->in_elems; i += NT) x[i] = img[i];
+    else
+    {
+        const int P = hdr->in_H * hdr->in_W, n4 = hdr->in_elems >> 2;
+        for (int i = tid; i < n4; i += NT)
+        {
+            const int q = i & 3, r = i >> 2, cb = r / P, p = r - cb * P;
+            *reinterpret_cast<float4 *>(x + apos(cb, P, p, q)) = reinterpret_cast<const float4 *>(img)[i];
+        }
+    }
+    if (tid < 4) lds[hdr->zero_off + tid] = 0.f;
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+}
+
+// output pixels [p0, p1) of a layer (a whole-image pooling layer: all of it); FUSED: the list may hold K_DWPW, on whole images
+template <bool FUSED>
+__device__ __forceinline__ void run_layer(const FMLayer &L, float *lds, const float *wl, const float *zero, float *gout, int tid, int wave,
+                                          int lane, int p0, int p1)
+{
+    const int n_pt = (p1 - p0 + 15) >> 4;
+    if (L.kind == K_CONV)
+    {
+        if (n_pt * (L.Co / CB) >= 2 * NW) conv_layer<2>(L, lds, wl, zero, gout, wave, lane, p0, p1);
+        else conv_layer<1>(L, lds, wl, zero, gout, wave, lane, p0, p1);
+    }
+    else if (L.kind == K_STEM)
+    {
+        // as many output-channel blocks per gathered operand as still leave every wave a pixel tile
+        const int CoB = L.Co / CB;
+        if (CoB % 4 == 0 && n_pt * (CoB / 4) >= NW) stem_layer<4>(L, lds, wl, zero, gout, wave, lane, p0, p1);
+        else if (CoB % 2 == 0 && n_pt * (CoB / 2) >= NW) stem_layer<2>(L, lds, wl, zero, gout, wave, lane, p0, p1);
+        else stem_layer<1>(L, lds, wl, zero, gout, wave, lane, p0, p1);
+    }
+    else if (FUSED && L.kind == K_DWPW)
+    {
+        // as many output-channel blocks per depthwise result as still leave every wave a pixel tile
+        const int CoB = L.Co2 / CB;
+        if (CoB % 4 == 0 && (n_pt * (CoB / 4) >= NW || CoB == 4)) dwpw_layer<4>(L, lds, wl, zero, gout, wave, lane);
+        else if (CoB % 2 == 0) dwpw_layer<2>(L, lds, wl, zero, gout, wave, lane);
+        else dwpw_layer<1>(L, lds, wl, zero, gout, wave, lane);
+    }
+    else if (L.kind == K_DW)
+    {
+        if (L.kh == 3 && L.kw == 3) dw_layer_win<3, 3>(L, lds, wl, zero, gout, tid, p0, p1);
+        else dw_layer_any(L, lds, wl, gout, tid, p0, p1);
+    }
+    else
+        pool_layer(L, lds, gout, tid);
+}
+
+// layers [first, last) of the model on whole images, or (ranges) on the output pixels that the band needs
+template <bool FUSED>
+__device__ __forceinline__ void run_layers(HeaderPtr hdr, const float *blob, float *lds, float *wbuf, float *gout, int tid, int wave, int lane,
+                                           int first, int last, const __attribute__((address_space(4))) int2 *ranges)
+{
+    const int w_floats = hdr->w_floats;
+    const float *zero = lds + hdr->zero_off;
+    for (int li = first; li < last; ++li)
+    {
+        const FMLayer L = load_layer(hdr, li);
+        const int p0 = ranges ? ranges[li].x : 0, p1 = ranges ? ranges[li].y : L.Ho * L.Wo;
+        // the next layer's weights go from global memory straight into the other LDS buffer (no registers are held
+        // across the layer): in flight while this layer is computed, waited for before the barrier that ends it
+        if (L.next_blob16 > 0)
+            weights_to_lds(blob + L.next_blob_off, wbuf + ((li + 1) & 1) * w_floats, L.next_blob16, tid, wave);
+        run_layer<FUSED>(L, lds, wbuf + (li & 1) * w_floats, zero, gout, tid, wave, lane, p0, p1);
+        __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0): the weights have landed in LDS
+        __syncthreads();
+    }
+}
+
 __global__ __launch_bounds__(NT) void fmodel_f32_kernel(const FMHeader *__restrict__ hdr_dev, const float *__restrict__ blob,
                                                         const float *__restrict__ in, float *__restrict__ out)
 {
@@ -569,74 +676,47 @@ __global__ __launch_bounds__(NT) void fmodel_f32_kernel(const FMHeader *__restri
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const size_t n = blockIdx.x;
-    const int n_layers = hdr->n_layers;
     float *wbuf = lds + hdr->w_lds;
-    const int w_floats = hdr->w_floats;
+    stage_image(hdr, blob, in + n * (size_t)hdr->in_elems, lds, wbuf, tid, wave);
+    run_layers<true>(hdr, blob, lds, wbuf, out + n * (size_t)hdr->out_elems, tid, wave, lane, 0, hdr->n_layers, nullptr);
+}
 
-    // the first layer's weights and the image
-    {
-        weights_to_lds(blob + hdr->layer[0].blob_off, wbuf, hdr->layer[0].blob16, tid, wave);
-        const float *img = in + n * (size_t)hdr->in_elems;
-        float *x = lds + hdr->in_off;
-        if (hdr->in_C < CB)
-            for (int i = tid; i < hdr->in_elems; i += NT) x[i] = img[i];
-        else
-        {
-            const int P = hdr->in_H * hdr->in_W, n4 = hdr->in_elems >> 2;
-            for (int i = tid; i < n4; i += NT)
-            {
-                const int q = i & 3, r = i >> 2, cb = r / P, p = r - cb * P;
-                *reinterpret_cast<float4 *>(x + apos(cb, P, p, q)) = reinterpret_cast<const float4 *>(img)[i];
-            }
-        }
-    }
-    float *gout = out + n * (size_t)hdr->out_elems;
-    float *part = lds + hdr->pool_off;
-    const float *zero = lds + hdr->zero_off;
-    if (tid < 4) lds[hdr->zero_off + tid] = 0.f;
-    __builtin_amdgcn_s_waitcnt(0x0F70);
+// Few images: an image is cut into bands of rows, one workgroup each, so that it runs on several compute units.  A band computes
+// the rows of every layer that its rows of the last layer before the whole-image pooling need (the halo is computed again
+// by the neighbours), and stores its rows of that layer's output; the workgroup that finishes last takes the whole tensor back
+// and runs the pooling and what follows.  Nobody waits for anybody: the others have left.  Depthwise and 1x1 layers run one after the other
+// here (a band has too few pixel tiles for every wave to own one and make its depthwise operand itself); the sums are the
+// same in the same order, and so are the bits.
+// What bounds it: the chain of layers, about 1.3 us each whatever their size (record, addresses, LDS, MFMAs, barrier).
+__global__ __launch_bounds__(NT) void fmodel_f32_band_kernel(const FMHeader *__restrict__ hdr_dev, const float *__restrict__ blob,
+                                                             const float *__restrict__ in, float *__restrict__ out,
+                                                             const int2 *__restrict__ ranges, int bands, float *tensors, unsigned *counters)
+{
+    HeaderPtr hdr = (HeaderPtr)hdr_dev;
+    extern __shared__ __align__(16) float lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = blockIdx.x / bands, band = blockIdx.x - n * bands;
+    const int n_band = hdr->n_band, elems = hdr->band_elems;
+    float *wbuf = lds + hdr->w_lds, *gout = out + (size_t)n * hdr->out_elems, *tensor = tensors + (size_t)n * elems;
+    stage_image(hdr, blob, in + (size_t)n * hdr->in_elems, lds, wbuf, tid, wave);
+    run_layers<false>(hdr, blob, lds, wbuf, tensor, tid, wave, lane, 0, n_band,
+               (const __attribute__((address_space(4))) int2 *)(ranges + (size_t)band * n_band));
+    unsigned *last = reinterpret_cast<unsigned *>(lds + hdr->zero_off + 4);
+    // every wave has waited for its stores (run_layers: vmcnt 0, barrier) before the band is counted
+    if (tid == 0) *last = __hip_atomic_fetch_add(counters + n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-
-    for (int li = 0; li < n_layers; ++li)
+    if (*last != (unsigned)bands - 1) return;        // the whole workgroup leaves together
+    if (tid == 0) __hip_atomic_store(counters + n, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // for the next launch on this stream
+    const int P = hdr->band_P;
+    float *x = lds + hdr->band_off;
+    for (int i = tid; i < elems >> 2; i += NT)
     {
-        const FMLayer L = load_layer(hdr, li);
-        const float *wl = wbuf + (li & 1) * w_floats;
-        // the next layer's weights go from global memory straight into the other LDS buffer (no registers are held
-        // across the layer): in flight while this layer is computed, waited for before the barrier that ends it
-        if (L.next_blob16 > 0)
-            weights_to_lds(blob + L.next_blob_off, wbuf + ((li + 1) & 1) * w_floats, L.next_blob16, tid, wave);
-        if (L.kind == K_CONV)
-        {
-            const int n_tiles = ((L.Ho * L.Wo + 15) >> 4) * (L.Co / CB);
-            if (n_tiles >= 2 * NW) conv_layer<2>(L, lds, wl, zero, gout, wave, lane);
-            else conv_layer<1>(L, lds, wl, zero, gout, wave, lane);
-        }
-        else if (L.kind == K_STEM)
-        {
-            // as many output-channel blocks per gathered operand as still leave every wave a pixel tile
-            const int CoB = L.Co / CB, n_pt = (L.Ho * L.Wo + 15) >> 4;
-            if (CoB % 4 == 0 && n_pt * (CoB / 4) >= NW) stem_layer<4>(L, lds, wl, zero, gout, wave, lane);
-            else if (CoB % 2 == 0 && n_pt * (CoB / 2) >= NW) stem_layer<2>(L, lds, wl, zero, gout, wave, lane);
-            else stem_layer<1>(L, lds, wl, zero, gout, wave, lane);
-        }
-        else if (L.kind == K_DWPW)
-        {
-            // as many output-channel blocks per depthwise result as still leave every wave a pixel tile
-            const int CoB = L.Co2 / CB, n_pt = (L.Ho * L.Wo + 15) >> 4;
-            if (CoB % 4 == 0 && (n_pt * (CoB / 4) >= NW || CoB == 4)) dwpw_layer<4>(L, lds, wl, zero, gout, wave, lane);
-            else if (CoB % 2 == 0) dwpw_layer<2>(L, lds, wl, zero, gout, wave, lane);
-            else dwpw_layer<1>(L, lds, wl, zero, gout, wave, lane);
-        }
-        else if (L.kind == K_DW)
-        {
-            if (L.kh == 3 && L.kw == 3) dw_layer_win<3, 3>(L, lds, wl, zero, gout, tid);
-            else dw_layer_any(L, lds, wl, gout, tid);
-        }
-        else
-            pool_layer(L, lds, part, gout, tid);
-        __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0): the weights have landed in LDS
-        __syncthreads();
+        const int q = i & 3, r = i >> 2, cb = r / P, p = r - cb * P;
+        *reinterpret_cast<float4 *>(x + apos(cb, P, p, q)) = load_shared(tensor + 4 * (size_t)i);
     }
+    __syncthreads();
+    run_layers<false>(hdr, blob, lds, wbuf, gout, tid, wave, lane, n_band, hdr->n_layers, nullptr);
 }
 
 int align_up(int v, int a) { return (v + a - 1) / a * a; }
@@ -646,10 +726,134 @@ int align_up(int v, int a) { return (v + a - 1) / a * a; }
 struct small_hip_fmodel
 {
     FMHeader hdr;
-    void *dev = nullptr;        // [FMHeader][weights of every layer, operand order]
+    void *dev = nullptr;        // [FMHeader][FMHeader of the band kernel][its pixel ranges][weights of every layer, operand order]
     size_t blob_off = 0;
     int device = 0;
+
+    // band kernel (band_rows == 0: the model has none): what its bands exchange lies in one of a few slots, each taken for good by the first stream that needs one, so that two launches that may run at the same time never share one
+    static constexpr int SLOTS = 4;
+    static constexpr size_t SLOT_BYTES = size_t(4) << 20;
+    int band_rows = 0, band_batch = 0;               // rows of the tensor before the pooling; images a slot has room for
+    int band_lds = 0;
+    size_t band_hdr_off = 0, ranges_off = 0, slot_bytes = 0;
+    std::vector<int> ranges_first;                   // [rows per band] -> first range (int2) of that cut
+    unsigned char *slots = nullptr;                  // [SLOTS][band_batch] tensors
+    unsigned *counters = nullptr;                    // [SLOTS][band_batch]
+    mutable std::mutex mu;
+    mutable int n_slots = 0;
+    mutable hipStream_t slot_stream[SLOTS];
+
+    // the slot of this stream, or -1: others got all of them before it
+    int slot(hipStream_t s) const
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        for (int i = 0; i < n_slots; ++i)
+            if (slot_stream[i] == s) return i;
+        if (n_slots == SLOTS) return -1;
+        slot_stream[n_slots] = s;
+        return n_slots++;
+    }
 };
+
+namespace
+{
+
+// The band kernel's layer list: the layers up to a whole-image pooling are one chain of convolutions, each reading what the one
+// before wrote, and nothing behind the pooling reads any of them.  Layers keep their own tensors and stay apart.
+// `ranges`: for every number of rows per band the output pixels of each layer that each band computes.
+bool plan_bands(const small_hip_flayer *layers, const std::vector<FMLayer> &tmp, const FMHeader &whole, FMHeader &b, int *rows,
+                std::vector<int> &ranges, std::vector<int> &first)
+{
+    const int n = (int)tmp.size();
+    auto is_pool = [](const FMLayer &L) { return L.kind == K_POOL_AVG || L.kind == K_POOL_MAX; };
+    int k = 0;
+    while (k < n && !is_pool(tmp[(size_t)k])) ++k;
+    if (k == 0 || k == n) return false;
+    for (int i = 1; i < n; ++i)
+        if (layers[i].src != layers[i - 1].dst) return false;
+    const FMLayer &last = tmp[(size_t)k - 1];
+    *rows = last.Ho;
+    if (last.Ho < 6 || last.Ho > 64) return false;
+    b = whole;
+    int floats[MAX_TENSORS] = {}, max_blob = 0;
+    for (int i = 0; i < n; ++i)
+    {
+        const FMLayer &L = tmp[(size_t)i];
+        b.layer[i] = L;
+        max_blob = L.blob16 * 4 > max_blob ? L.blob16 * 4 : max_blob;
+        if (layers[i].dst >= 0 && L.Co * L.Ho * L.Wo > floats[layers[i].dst]) floats[layers[i].dst] = L.Co * L.Ho * L.Wo;
+    }
+    int off = 0, at[MAX_TENSORS];
+    b.w_lds = off; b.w_floats = max_blob; off += 2 * max_blob;
+    b.zero_off = off; off += 8;
+    b.in_off = off; off += align_up(b.in_elems, 4);
+    for (int t = 0; t < MAX_TENSORS; ++t) { at[t] = off; off += floats[t]; }
+    if ((long)off * 4 > LDS_LIMIT) return false;
+    b.lds_bytes = off * 4;
+    b.n_layers = n;
+    for (int i = 0; i < n; ++i)
+    {
+        FMLayer &L = b.layer[i];
+        L.src_off = i == 0 ? b.in_off : at[layers[i].src];
+        L.dst_off = layers[i].dst >= 0 ? at[layers[i].dst] : TO_OUTPUT;
+        L.next_blob_off = i + 1 < n ? tmp[(size_t)i + 1].blob_off : 0;
+        L.next_blob16 = i + 1 < n ? tmp[(size_t)i + 1].blob16 : 0;
+    }
+    b.n_band = k;
+    b.band_elems = last.Co * last.Ho * last.Wo;
+    b.band_P = last.Ho * last.Wo;
+    b.band_off = at[layers[k - 1].dst];
+    b.layer[k - 1].dst_off = TO_SLOT;
+    b.layer[k - 1].next_blob16 = 0;                  // the pooling has no weights; its own record fetches what follows
+    first.assign((size_t)*rows + 1, -1);
+    ranges.clear();
+    for (int rb = 1; rb <= *rows; ++rb)
+    {
+        first[(size_t)rb] = (int)ranges.size() / 2;
+        for (int r = 0; r < *rows; r += rb)
+        {
+            std::vector<int> band((size_t)k * 2);
+            int lo = r, hi = r + rb < *rows ? r + rb : *rows;
+            for (int i = k - 1; i >= 0; --i)
+            {
+                const FMLayer &L = tmp[(size_t)i];
+                if (lo >= hi) return false;          // a band that reads padding only
+                band[(size_t)i * 2] = lo * L.Wo;
+                band[(size_t)i * 2 + 1] = hi * L.Wo;
+                const int in_lo = lo * L.stride - L.pt, in_hi = (hi - 1) * L.stride - L.pt + L.kh;
+                lo = in_lo > 0 ? in_lo : 0;
+                hi = in_hi < L.H ? in_hi : L.H;
+            }
+            ranges.insert(ranges.end(), band.begin(), band.end());
+        }
+    }
+    return true;
+}
+
+// Rows per band for this batch, or 0: whole images.  As many bands as compute units; a band computes its halo again, so from a
+// sixth of the rows on they stop paying.  DS-CNN (25 rows), whole images -> bands: batch 1 (1 row) 26.8 -> 21.9 us, 8 (1) 27.3 -> 22.9,
+// 16 (2) 27.4 -> 24.0, 32 (4) 27.4 -> 25.5; 5 rows 26.6, 7 rows (batch 64) 28.7.
+int band_rows(const small_hip_fmodel *m, int batch)
+{
+    static const int force = tune_int("fmodel_band", -1);
+    if (m->band_rows == 0 || batch > m->band_batch || force == 0) return 0;
+    if (force > 0) return force < m->band_rows ? force : m->band_rows;
+    const long wanted = ((long)m->band_rows * batch + NUM_CU - 1) / NUM_CU;
+    const int rows = wanted < 1 ? 1 : (int)wanted;
+    return 6 * rows <= m->band_rows ? rows : 0;
+}
+
+// The stream's slot; none (-1) for a stream that is being captured (a graph may be replayed on any stream, at the same time as other
+// launches) and for the per-thread default stream, whose handle stands for several streams.
+int band_slot(const small_hip_fmodel *m, hipStream_t s)
+{
+    if (s == hipStreamPerThread) return -1;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) { (void)hipGetLastError(); return -1; }
+    return st == hipStreamCaptureStatusNone ? m->slot(s) : -1;
+}
+
+} // namespace
 
 extern "C" {
 
@@ -672,7 +876,6 @@ int small_hip_fmodel_create(int n_layers, const small_hip_flayer *layers, small_
     int written_by[MAX_TENSORS];
     for (int t = 0; t < MAX_TENSORS; ++t) written_by[t] = -1;
     int blob_floats = 0, max_blob = 0;
-    bool any_pool = false;
     std::vector<int> w_floats((size_t)n_layers, 0);
     for (int i = 0; i < n_layers; ++i)
     {
@@ -708,7 +911,6 @@ int small_hip_fmodel_create(int n_layers, const small_hip_flayer *layers, small_
             L.kind = l.kind == SMALL_HIP_FL_GLOBAL_AVGPOOL ? K_POOL_AVG : K_POOL_MAX;
             L.Co = Ci; L.Ho = 1; L.Wo = 1; L.kh = H; L.kw = W; L.stride = 1;
             L.norm = (float)(1.0 / ((double)H * W));
-            any_pool = true;
         }
         else
         {
@@ -822,11 +1024,10 @@ int small_hip_fmodel_create(int n_layers, const small_hip_flayer *layers, small_
         h.layer[i].next_blob16 = h.layer[i + 1].blob16;
     }
 
-    // LDS plan (floats): [weights x2][pooling partials][input][tensors]
+    // LDS plan (floats): [weights x2][zeros][input][tensors]
     int off = 0;
     h.w_lds = off; h.w_floats = max_blob; off += 2 * max_blob;
-    h.pool_off = off; off += any_pool ? NT * 4 + NT / 2 * 4 : 0;
-    h.zero_off = off; off += 4;
+    h.zero_off = off; off += 8;
     const small_hip_flayer &l0 = layers[0];
     h.in_C = l0.input_channels; h.in_H = l0.input_height; h.in_W = l0.input_width;
     h.in_elems = h.in_C * h.in_H * h.in_W;
@@ -844,7 +1045,7 @@ int small_hip_fmodel_create(int n_layers, const small_hip_flayer *layers, small_
     {
         FMLayer &L = h.layer[i];
         L.src_off = i == 0 ? h.in_off : tensor_off[dev_src[i]];
-        L.dst_off = dev_dst[i] >= 0 ? tensor_off[dev_dst[i]] : -1;
+        L.dst_off = dev_dst[i] >= 0 ? tensor_off[dev_dst[i]] : TO_OUTPUT;
     }
     const FMLayer &last = tmp[(size_t)n_layers - 1];
     h.out_elems = last.Co * last.Ho * last.Wo;
@@ -852,8 +1053,36 @@ int small_hip_fmodel_create(int n_layers, const small_hip_flayer *layers, small_
     hipStream_t s = as_stream(stream);
     hipError_t e = hipGetDevice(&m->device);
     if (e != hipSuccess) return fail(fail_hip(e, "hipGetDevice"));
-    m->blob_off = (sizeof(FMHeader) + 255) & ~(size_t)255;
-    e = hipMalloc(&m->dev, m->blob_off + (size_t)blob_floats * 4 + 256);
+    auto up256 = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    FMHeader band;
+    std::vector<int> ranges;
+    int rows = 0;
+    const bool bands = plan_bands(layers, tmp, h, band, &rows, ranges, m->ranges_first);
+    m->band_hdr_off = up256(sizeof(FMHeader));
+    m->ranges_off = m->band_hdr_off + (bands ? up256(sizeof(FMHeader)) : 0);
+    m->blob_off = m->ranges_off + (bands ? up256(ranges.size() * sizeof(int)) : 0);
+    std::vector<unsigned char> head(m->blob_off);                   // what precedes the weights, uploaded in one piece
+    std::memcpy(head.data(), &m->hdr, sizeof(FMHeader));
+    if (bands)
+    {
+        std::memcpy(head.data() + m->band_hdr_off, &band, sizeof(FMHeader));
+        std::memcpy(head.data() + m->ranges_off, ranges.data(), ranges.size() * sizeof(int));
+    }
+    // the weights, and behind them the bands' slots (without memory for those the model runs on whole images)
+    const size_t own_bytes = up256(m->blob_off + (size_t)blob_floats * 4 + 256);
+    size_t slot_bytes = 0, counter_bytes = 0;
+    if (bands)
+    {
+        const size_t per_image = (size_t)band.band_elems * 4, fit = small_hip_fmodel::SLOT_BYTES / per_image;
+        m->band_batch = (int)(fit < NUM_CU / 6 ? fit : NUM_CU / 6);
+        m->band_lds = band.lds_bytes;
+        m->slot_bytes = up256(m->band_batch * per_image);
+        slot_bytes = m->slot_bytes * small_hip_fmodel::SLOTS;
+        counter_bytes = (size_t)m->band_batch * small_hip_fmodel::SLOTS * sizeof(unsigned);
+    }
+    e = hipMalloc(&m->dev, own_bytes + slot_bytes + counter_bytes);
+    if (e == hipSuccess && bands) m->band_rows = rows;
+    else if (e == hipErrorOutOfMemory && bands) { (void)hipGetLastError(); e = hipMalloc(&m->dev, own_bytes); }
     if (e != hipSuccess)
     {
         (void)hipGetLastError();
@@ -861,6 +1090,13 @@ int small_hip_fmodel_create(int n_layers, const small_hip_flayer *layers, small_
         return fail(e == hipErrorOutOfMemory ? SMALL_HIP_ENOMEM : SMALL_HIP_EHIP);
     }
     auto fail_dev = [&](int rc) { (void)hipFree(m->dev); return fail(rc); };
+    if (m->band_rows > 0)
+    {
+        m->slots = static_cast<unsigned char *>(m->dev) + own_bytes;
+        m->counters = reinterpret_cast<unsigned *>(m->slots + slot_bytes);
+        e = hipMemsetAsync(m->counters, 0, counter_bytes, s);
+        if (e != hipSuccess) return fail_dev(fail_hip(e, "small_hip_fmodel_create: counters"));
+    }
     float *dblob = reinterpret_cast<float *>(static_cast<uint8_t *>(m->dev) + m->blob_off);
     std::vector<std::vector<int>> ktabs((size_t)n_layers);          // alive until the stream has been waited for
     for (int i = 0; i < n_layers; ++i)
@@ -888,11 +1124,13 @@ int small_hip_fmodel_create(int n_layers, const small_hip_flayer *layers, small_
             if (e != hipSuccess) return fail_dev(fail_hip(e, "small_hip_fmodel_create: tables"));
         }
     }
-    e = hipMemcpyAsync(m->dev, &m->hdr, sizeof(FMHeader), hipMemcpyHostToDevice, s);
+    e = hipMemcpyAsync(m->dev, head.data(), head.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);       // the caller's filters and the host-side tables may go
     if (e != hipSuccess) return fail_dev(fail_hip(e, "small_hip_fmodel_create: upload"));
     e = hipFuncSetAttribute(reinterpret_cast<const void *>(fmodel_f32_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                             LDS_LIMIT);
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(fmodel_f32_band_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, LDS_LIMIT);
     if (e != hipSuccess) return fail_dev(fail_hip(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)"));
     *model = m;
     return SMALL_HIP_OK;
@@ -906,7 +1144,19 @@ int small_hip_fmodel_forward(const small_hip_fmodel *model, int batch, const flo
     if (batch == 0) return SMALL_HIP_OK;
     if (!aligned16(output) || (model->hdr.in_C >= CB && !aligned16(input)))
         return einval("small_hip_fmodel_forward: misaligned pointer");
-    const float *dblob = reinterpret_cast<const float *>(static_cast<const uint8_t *>(model->dev) + model->blob_off);
+    const unsigned char *dev = static_cast<const unsigned char *>(model->dev);
+    const float *dblob = reinterpret_cast<const float *>(dev + model->blob_off);
+    const int rows = band_rows(model, batch), slot = rows > 0 ? band_slot(model, as_stream(stream)) : -1;
+    if (slot >= 0)
+    {
+        const int bands = (model->band_rows + rows - 1) / rows;
+        hipLaunchKernelGGL(fmodel_f32_band_kernel, dim3((unsigned)(batch * bands)), dim3(NT), (size_t)model->band_lds, as_stream(stream),
+                           reinterpret_cast<const FMHeader *>(dev + model->band_hdr_off), dblob, input, output,
+                           reinterpret_cast<const int2 *>(dev + model->ranges_off) + model->ranges_first[(size_t)rows], bands,
+                           reinterpret_cast<float *>(model->slots + slot * model->slot_bytes), model->counters + slot * model->band_batch);
+        SHP_LAUNCH_CHECK("small_hip_fmodel_forward");
+        return SMALL_HIP_OK;
+    }
     hipLaunchKernelGGL(fmodel_f32_kernel, dim3((unsigned)batch), dim3(NT), (size_t)model->hdr.lds_bytes, as_stream(stream),
                        static_cast<const FMHeader *>(model->dev), dblob, input, output);
     SHP_LAUNCH_CHECK("small_hip_fmodel_forward");

@@ -130,6 +130,54 @@ def test_one_launch_graph_replays_match_eager(name, batch):
     ex.close()
 
 
+def _band_net(form):
+    """float32 models with a whole-image pooling: few images run in bands of rows on several compute units."""
+    if form == "dscnn":
+        return models.dscnn()
+    b = models._Builder("bands_" + form, "f32", (3, 53, 9) if form == "strided" else (16, 14, 6), "normal")
+    if form == "strided":               # odd map, a 5x5 depthwise layer, a 3x3 convolution, strides 2: 53 -> 27 -> 27 -> 14 -> 7 rows
+        b.advance(b.conv(32, 3, 2, "same", act="leaky", slope=0.1))
+        b.dw(5, 1, act="relu")
+        b.advance(b.conv(32, 3, 2, "same", act="relu"))
+        b.dw(3, 2)
+        b.pool("maxpool", 7, 2, 1)
+    else:                               # sixteen input channels, no layer behind the pooling
+        b.advance(b.conv(16, 3, 1, "same", act="relu"))
+        b.dw(3, 1, act="relu")
+        b.advance(b.conv(32, 1, 1, "valid"))
+        b.pool("avgpool", 14, 6, 1)
+        return b.done()
+    b.dense(20)
+    return b.done()
+
+
+@pytest.mark.parametrize("form,batch", [("dscnn", 1), ("dscnn", 7), ("dscnn", 23), ("dscnn", 41), ("strided", 1), ("strided", 50), ("blocked", 1),
+                                        ("blocked", 17)])
+def test_fmodel_bands_equal_whole_images(form, batch):
+    """Bands of rows compute the same sums in the same order as whole images (which a captured call takes): the same bits, and
+    the oracle's values.  Streams past the last slot take whole images too."""
+    import torch
+    m = _band_net(form)
+    w, x = models.make_weights(m), models.make_input(m, batch)
+    ex = models.HipExecutor(m, batch, w, x)
+    ex.build_one_launch()
+    ex.capture(one_launch=True)
+    ex.one_out.zero_()
+    ex.replay()
+    whole = ex.output_one_launch().copy()
+    assert_close_f32(whole, OracleExecutor(m, batch, w, x).forward(), what="%s, batch %d vs oracle" % (m.name, batch))
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    outs = [torch.zeros_like(ex.one_out) for _ in range(3 * len(streams))]
+    torch.cuda.synchronize()
+    for i, out in enumerate(outs):      # in flight at the same time, and again on the streams that have run before
+        s = streams[i % len(streams)]
+        capi.check(ex.lib.small_hip_fmodel_forward(ex.qmodel, batch, ex._p(ex.buf["in"]), ex._p(out), C.c_void_p(s.cuda_stream)))
+    torch.cuda.synchronize()
+    for i, out in enumerate(outs):
+        assert np.array_equal(out.cpu().numpy().view(np.uint8), whole.view(np.uint8)), "launch %d differs" % i
+    ex.close()
+
+
 def _exposed_u8_net(hw, form):
     """Two or three uint8 convolutions whose bytes stay between 0 and 255 (not saturated), followed by a 1x1 convolution
     with an identity filter and a unit output scale, so that the model's output IS the last tensor, byte for byte:
