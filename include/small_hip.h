@@ -535,8 +535,8 @@ int small_hip_pool1d_u8(int is_max, int batch, int kernel_width, int stride, int
  * plus the weights of two consecutive layers within 160 KB, at most 48 KB of weights per layer; a model beyond
  * them is refused with SMALL_HIP_EINVAL and a message.  small_hip_fmodel_create() copies and re-orders filters and
  * biases (it allocates device memory and returns after its work on `stream` has finished);
- * small_hip_fmodel_forward() is one launch and allocates nothing; a batch of few images runs in bands of rows on several
- * compute units (same bits; on the first four streams that ask, not under capture).  Results are within the float32 tolerance of the
+ * small_hip_fmodel_forward() is one launch and allocates nothing; few images of a depthwise-separable chain run in
+ * bands of rows on several compute units (same bits; on the first four streams that ask, not under capture).  Results are within the float32 tolerance of the
  * layer-by-layer calls (another summation order), not bit-identical to them. */
 #define SMALL_HIP_FL_CONV 0
 #define SMALL_HIP_FL_DWCONV 1

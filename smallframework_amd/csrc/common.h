@@ -32,7 +32,7 @@ void set_error(const char *fmt, ...);
 //   fuse_form=3       convolution + depthwise pairs through an intermediate buffer: always the two launches
 //   dw_tile=0         depthwise without the LDS tile kernel                         dw_shape=N  force its tile shape
 //   convq_min_wg, convq_table_min_wg   workgroup targets of the uint8 convolution   fmodel_fuse=0  whole-model kernel without dw + 1x1 fusion
-//   fmodel_band=0|N   whole-model kernel: whole images only / bands of N rows
+//   fmodel_sep=0      whole-model kernel: separable chains in the general kernel      fmodel_band=0|N  whole images only / bands of N rows
 //   fuse_conv_dw=0|2, fuse_pool=0, one_launch=0|1   the C++ wrappers' choices (read through small_hip_tune_int)
 int tune_int(const char *key, int dflt);
 bool tune_pair(const char *key, int *a, int *b);

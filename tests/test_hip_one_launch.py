@@ -130,34 +130,48 @@ def test_one_launch_graph_replays_match_eager(name, batch):
     ex.close()
 
 
-def _band_net(form):
-    """float32 models with a whole-image pooling: few images run in bands of rows on several compute units."""
+def _chain_net(form):
+    """float32 depthwise-separable chains: few images run in bands of rows on several compute units."""
     if form == "dscnn":
         return models.dscnn()
-    b = models._Builder("bands_" + form, "f32", (3, 53, 9) if form == "strided" else (16, 14, 6), "normal")
-    if form == "strided":               # odd map, a 5x5 depthwise layer, a 3x3 convolution, strides 2: 53 -> 27 -> 27 -> 14 -> 7 rows
+    b = models._Builder("chain_" + form, "f32", (3, 53, 9) if form == "strided" else (2, 14, 6), "normal")
+    if form == "strided":               # odd maps, strides 2, 53 -> 27 -> 27 -> 14 rows, 5 -> 3 columns, two fully connected layers
         b.advance(b.conv(32, 3, 2, "same", act="leaky", slope=0.1))
-        b.dw(5, 1, act="relu")
-        b.advance(b.conv(32, 3, 2, "same", act="relu"))
-        b.dw(3, 2)
-        b.pool("maxpool", 7, 2, 1)
-    else:                               # sixteen input channels, no layer behind the pooling
-        b.advance(b.conv(16, 3, 1, "same", act="relu"))
         b.dw(3, 1, act="relu")
-        b.advance(b.conv(32, 1, 1, "valid"))
+        b.advance(b.conv(80, 1, 1, "valid", act="leaky", slope=0.2))
+        b.dw(3, 2)
+        b.advance(b.conv(48, 1, 1, "valid"))
+        b.pool("maxpool", 14, 3, 1)
+        b.dense(32)
+        b.dense(20)
+    else:                               # one pair, nothing behind the pooling
+        b.advance(b.conv(16, 5, 1, "same", act="relu"))
+        b.dw(3, 1)
+        b.advance(b.conv(64, 1, 1, "valid", act="relu"))
         b.pool("avgpool", 14, 6, 1)
-        return b.done()
-    b.dense(20)
     return b.done()
 
 
-@pytest.mark.parametrize("form,batch", [("dscnn", 1), ("dscnn", 7), ("dscnn", 23), ("dscnn", 41), ("strided", 1), ("strided", 50), ("blocked", 1),
-                                        ("blocked", 17)])
+def test_fmodel_general_kernel_on_other_models():
+    """A first layer of sixteen channels: not a chain of the separable kernel's, so the general one runs it (with the depthwise + 1x1
+    pair as one layer)."""
+    b = models._Builder("general", "f32", (16, 14, 6), "normal")
+    b.advance(b.conv(16, 3, 1, "same", act="relu"))
+    b.dw(3, 1, act="relu")
+    b.advance(b.conv(64, 1, 1, "valid"))
+    b.pool("avgpool", 14, 6, 1)
+    got, layered, want = _run(b.done(), 5)
+    assert_close_f32(got, want, what="general kernel vs oracle")
+    assert_close_f32(got, layered, what="general kernel vs layer by layer")
+
+
+@pytest.mark.parametrize("form,batch", [("dscnn", 1), ("dscnn", 7), ("dscnn", 23), ("dscnn", 41), ("dscnn", 128), ("dscnn", 300), ("strided", 1), ("strided", 30),
+                                        ("strided", 50), ("single", 1), ("single", 33)])
 def test_fmodel_bands_equal_whole_images(form, batch):
     """Bands of rows compute the same sums in the same order as whole images (which a captured call takes): the same bits, and
     the oracle's values.  Streams past the last slot take whole images too."""
     import torch
-    m = _band_net(form)
+    m = _chain_net(form)
     w, x = models.make_weights(m), models.make_input(m, batch)
     ex = models.HipExecutor(m, batch, w, x)
     ex.build_one_launch()
