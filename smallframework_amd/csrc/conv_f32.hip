@@ -140,12 +140,12 @@ __device__ __forceinline__ void mfma_split(floatx16 (&big)[COT][PXT], floatx16 (
 #undef SHP_MFMA_
 }
 #undef SHP_SPLIT_PRODUCTS_
-// big + small; true for a wave that may have to multiply again (see above; split_odd tells).  An infinity or a NaN times
-// zero is a NaN, which a chain of fused multiply-adds keeps.
+// big + small; true for a wave that may have to multiply again (see above; split_odd tells).  The largest magnitude keeps a NaN
+// (v_maximum3_f32), the smallest does not; both take two values an instruction.
 template <int COT, int PXT>
 __device__ __forceinline__ bool split_merge(floatx16 (&big)[COT][PXT], const floatx16 (&sml)[COT][PXT], const bool (&pvalid)[PXT])
 {
-    float nan = 0.f, least = 1.f;
+    float most = 0.f, least = 1.f;
 #pragma unroll
     for (int t = 0; t < PXT; ++t)
     {
@@ -153,16 +153,17 @@ __device__ __forceinline__ bool split_merge(floatx16 (&big)[COT][PXT], const flo
 #pragma unroll
         for (int c = 0; c < COT; ++c)
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
+            for (int r = 0; r < 16; r += 2)
             {
-                const float v = big[c][t][r] + sml[c][t][r];
-                nan = fmaf(v, 0.f, nan);
-                l = fminf(l, fabsf(v));
+                const float v = big[c][t][r] + sml[c][t][r], u = big[c][t][r + 1] + sml[c][t][r + 1];
+                most = __builtin_elementwise_maximum(__builtin_elementwise_maximum(most, fabsf(v)), fabsf(u));
+                l = fminf(fminf(l, fabsf(v)), fabsf(u));
                 big[c][t][r] = v;
+                big[c][t][r + 1] = u;
             }
         least = fminf(least, pvalid[t] ? l : 1.f);
     }
-    return __any(nan != 0.f || least < SPLIT_LEAST);
+    return __any(!(most <= 3.402823466e38f) || least < SPLIT_LEAST);
 }
 // cold: zeros (dead inputs, channels without weights) are told from very small sums
 template <int COT, int PXT>
