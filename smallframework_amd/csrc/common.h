@@ -28,7 +28,7 @@ void set_error(const char *fmt, ...);
 //   conv_splitk=0|1   force the split-K kernel off / on                             conv_streamk=0|N  equal-share split off / N per CU
 //   conv_streamk_min  least K-steps for the equal-share split                       stem_lds=0  first layers without the LDS kernel
 //   stem_vec=0|1      16-byte staging of first-layer patches                        smallci_valu=1  vector-ALU first layers
-//   pwdw_cot=1|2      channels (x32) per workgroup of the LDS-parked pointwise + depthwise kernel
+//   pwdw_cot=1|2      channels (x32) per workgroup (2: from 96 input channels on) of the LDS-parked pointwise + depthwise kernel
 //   fuse_form=3       convolution + depthwise pairs through an intermediate buffer: always the two launches
 //   dw_tile=0         depthwise without the LDS tile kernel                         dw_shape=N  force its tile shape
 //   convq_min_wg, convq_table_min_wg   workgroup targets of the uint8 convolution   fmodel_fuse=0  whole-model kernel without dw + 1x1 fusion

@@ -1792,13 +1792,17 @@ __global__ __launch_bounds__(256, 4) void conv_stem3x3_dw3x3_f32_kernel(const Co
 // pointwise layer's output, the largest tensor of such a pair, is neither written nor read.
 // A workgroup owns 32 * COT channels and a tile of TOH x TOW depthwise outputs of one image (14 x 14 at stride 1, 7 x 8 at
 // stride 2).  The PH x PW pointwise pixels under that tile (16 x 16 / 15 x 17, at most 256) are eight 32-pixel MFMA tiles,
-// two per wave; the filter slice of the workgroup is split and staged in LDS once, in MFMA operand order, the activation
+// two per wave (one with COT = 2); the filter slice of the workgroup is split and staged in LDS once, in MFMA operand order, the activation
 // operand goes from memory to the wave's registers and is split there as in conv_lds_tile, and the K loop is unrolled: no
 // barrier and no staging inside it.  The products are added in conv_lds_tile's order.  The activated result is parked in LDS as
 // [pixel][channel] (zeros outside the pointwise layer's map: the depthwise layer's padding) and the depthwise window
 // runs on it like dw3x3_f32_tile_kernel (a lane = four channels of one column, a run of rows, the same order of operations).
 // The halo is computed again by the neighbouring workgroups: 256 / 196 = 1.31 x the pointwise work at stride 1,
 // 255 / 224 = 1.14 x at stride 2.
+// What bounds it: the life of a workgroup is a chain (request, stage, multiply, park, window, store).  64 -> 128 @56x56 batch 64, 46.7 us:
+// without its stores 39.7, without MFMAs 35.6, without either and the window 24.  So everything that memory has to bring, the
+// depthwise taps among it, is requested first of all and parked in LDS (taps loaded after the K loop: 36.9 us for 128 -> 256 @28x28,
+// now 36.0), and more K-steps ahead where registers allow.
 template <int S>
 struct PwDwTile
 {
@@ -1818,17 +1822,18 @@ struct PwDwGeom
 };
 
 template <int S, int COT, int CIB, bool RELU = false>
-__global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kernel(const ConvArgs a, const StemDwArgs d, const PwDwGeom g)
+__global__ __launch_bounds__(256 * COT, 4) void conv_pw_dw3x3_f32_kernel(const ConvArgs a, const StemDwArgs d, const PwDwGeom g)
 {
     using TL = PwDwTile<S>;
     constexpr int TOH = TL::TOH, TOW = TL::TOW, PW = TL::PW, NPX = TL::NPX;
     constexpr int CG = 32 * COT;                             // channels of the workgroup
+    constexpr int NTH = 256 * COT, PT = 2 / COT;             // threads; pixel tiles of a wave
     constexpr int MIDP = CG + 4;                             // floats per parked pixel: 16 bytes of padding spread the banks
     constexpr int FILT_BYTES = CIB * COT * 3 * 1024;          // split filter operands: [K-step][channel tile][h, m, l][lane]
     // the filter slice is dead when the K loop ends and the parked tile is born after it: they share their LDS
     constexpr int MID_FLOATS = 256 * MIDP, FILT_FLOATS = FILT_BYTES / 4;
     __shared__ __align__(16) float lds[MID_FLOATS > FILT_FLOATS ? MID_FLOATS : FILT_FLOATS];
-    __shared__ __align__(16) float s_bias[CG];
+    __shared__ __align__(16) float s_bias[CG], s_dw[CG * 9], s_dw_bias[CG];
     unsigned char *const filt = reinterpret_cast<unsigned char *>(lds);
     float *const mid = lds;
 
@@ -1848,62 +1853,67 @@ __global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kerne
     const int HW = a.H * a.W, CoB = a.Co / CB;
     const float nscale = act_scale(a.act, a.slope);
 
-    float my_bias = 0.f;
+    // biases and depthwise taps [channel block][tap][16]: requested first of all, parked in LDS with the filter
+    float my_bias = 0.f, my_dw_bias = 0.f;
     if (tid < CG && a.bias) my_bias = a.bias[cg * CG + tid];
+    if (tid < CG && d.dw_bias) my_dw_bias = d.dw_bias[cg * CG + tid];
+    float4 my_taps = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (tid < CG * 9 / 4) my_taps = reinterpret_cast<const float4 *>(d.dw_filt + (size_t)cg * (CG * 9))[tid];
     // depthwise phase: lane = (channel quad q, column dx, row group rg)
-    constexpr int NQ = CG / 4, TCOLS = S == 1 ? 16 : 8, NRG = 256 / (NQ * TCOLS), RPG = (TOH + NRG - 1) / NRG;
+    constexpr int NQ = CG / 4, TCOLS = S == 1 ? 16 : 8, NRG = NTH / (NQ * TCOLS), RPG = (TOH + NRG - 1) / NRG;
     const int q = tid % NQ, dslot = tid / NQ, dx = dslot % TCOLS, rg = dslot / TCOLS;
     const int dcob = cg * (CG / CB) + q / 4, dq4 = (q & 3) * 4;   // channel block and first channel inside it
 
     // ---- pointwise layer on the patch --------------------------------------------------------------------------------
-    // this lane's two pixels: patch index p = (2 wave + t) * 32 + col -> position (p / PW, p % PW)
-    const float *in_px[2];
-    bool pin[2];                                             // inside the pointwise layer's map
-    int pidx[2];
+    // this lane's pixels: patch index p = (PT wave + t) * 32 + col -> position (p / PW, p % PW)
+    const float *in_px[PT];
+    bool pin[PT];                                            // inside the pointwise layer's map
+    int pidx[PT], in_step[PT];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < PT; ++t)
     {
-        const int pp = (2 * wave + t) * 32 + col;
+        const int pp = (PT * wave + t) * 32 + col;
         const int py = pp / PW, pxx = pp - py * PW;
         const int oh = py0 + py, ow = px0 + pxx;
         pin[t] = pp < NPX && (unsigned)oh < (unsigned)a.H && (unsigned)ow < (unsigned)a.W;
         pidx[t] = pp;
         in_px[t] = pin[t] ? a.in + ((size_t)n * CIB * HW + oh * a.W + ow) * CB + half * 8 : g_zero_block + half * 8;
+        in_step[t] = pin[t] ? HW * CB : 0;
     }
-    if (tid < CG) s_bias[tid] = my_bias;
     // ---- requests first: filter slice, the first two steps' pixels -----------------------------------------------
     // filter: unit u of 64 COT CIB = (operand u / 64 = K-step and channel tile, lane u % 64) is eight input channels of one
     // output channel; the thread that loads them splits them once for the whole workgroup
-    constexpr int NU = 64 * COT * CIB, UPT = (NU + 255) / 256;
+    constexpr int NU = 64 * COT * CIB, UPT = (NU + NTH - 1) / NTH;
     float fraw[UPT][8];
 #pragma unroll
     for (int r = 0; r < UPT; ++r)
     {
-        const int u = tid + r * 256, ul = u & 63, op = u >> 6, us = op / COT, uc = op - us * COT;
+        const int u = tid + r * NTH, ul = u & 63, op = u >> 6, us = op / COT, uc = op - us * COT;
         const int cob = (cg * COT + uc) * 2 + ((ul & 31) >> 4);
         const float *src = a.filt + ((size_t)cob * CIB + us) * (CB * CB) + (ul >> 5) * 8 * CB + (ul & 15);
-        if (NU % 256 == 0 || u < NU)
+        if (NU % NTH == 0 || u < NU)
 #pragma unroll
             for (int k = 0; k < 8; ++k) fraw[r][k] = src[k * CB];
     }
-    const int in_blk32 = HW * CB;
-    float4 B[2][2][2];                                       // [buffer][pixel tile][half of the eight channels]
-    auto fetch = [&](const int buf, const int cib) {
+    constexpr int PF = COT == 2 ? 3 : CIB < 2 ? CIB : 2;     // K-steps requested ahead
+    float4 B[PF][PT][2];                                     // [buffer][pixel tile][half of the eight channels]
+    auto fetch = [&](const int buf) {                        // the next channel block
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < PT; ++t)
         {
-            const float4 *p4 = reinterpret_cast<const float4 *>(in_px[t] + (pin[t] ? cib * in_blk32 : 0));
+            const float4 *p4 = reinterpret_cast<const float4 *>(in_px[t]);
             B[buf][t][0] = p4[0];
             B[buf][t][1] = p4[1];
+            in_px[t] += in_step[t];
         }
     };
-    fetch(0, 0);
-    if (CIB > 1) fetch(1, 1);
+#pragma unroll
+    for (int s = 0; s < PF; ++s) fetch(s);
 #pragma unroll
     for (int r = 0; r < UPT; ++r)
     {
-        const int u = tid + r * 256;
-        if (NU % 256 == 0 || u < NU)
+        const int u = tid + r * NTH;
+        if (NU % NTH == 0 || u < NU)
         {
             const Split8 f = split8(fraw[r]);
             unsigned char *d = filt + (u >> 6) * 3 * 1024 + (u & 63) * 16;
@@ -1912,13 +1922,15 @@ __global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kerne
             *reinterpret_cast<bf16x8 *>(d + 2048) = f.l;
         }
     }
+    if (tid < CG * 9 / 4) reinterpret_cast<float4 *>(s_dw)[tid] = my_taps;
+    if (tid < CG) { s_bias[tid] = my_bias; s_dw_bias[tid] = my_dw_bias; }
     __syncthreads();
 
-    floatx16 acc[COT][2], sml[COT][2];
+    floatx16 acc[COT][PT], sml[COT][PT];
 #pragma unroll
     for (int c = 0; c < COT; ++c)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < PT; ++t)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[c][t][r] = sml[c][t][r] = 0.f;
     auto step = [&](const int buf, const int s) {
@@ -1931,54 +1943,49 @@ __global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kerne
             A[c].m = *reinterpret_cast<const bf16x8 *>(r + 1024);
             A[c].l = *reinterpret_cast<const bf16x8 *>(r + 2048);
         }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)                          // (tile after tile: both split at once would not fit the registers)
+        if constexpr (PT == 1)
         {
-            const Split8 Bs = split8(B[buf][t][0], B[buf][t][1]);
-#pragma unroll
-            for (int c = 0; c < COT; ++c) mfma_split(acc[c][t], sml[c][t], A[c], Bs);
-            __builtin_amdgcn_sched_barrier(0);
+            const Split8 Bs[1] = {split8(B[buf][0][0], B[buf][0][1])};
+            mfma_split<COT, 1>(acc, sml, A, Bs);
         }
-        if (s + 2 < CIB) fetch(buf, s + 2);
+        else
+#pragma unroll
+            for (int t = 0; t < PT; ++t)                     // (tile after tile: both split at once would not fit the registers)
+            {
+                const Split8 Bs = split8(B[buf][t][0], B[buf][t][1]);
+                mfma_split(acc[0][t], sml[0][t], A[0], Bs);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        if (s + PF < CIB) fetch(buf);
     };
 #pragma unroll
-    for (int s = 0; s < CIB; ++s) step(s & 1, s);
+    for (int s = 0; s < CIB; ++s) step(s % PF, s);
 
-    if (__builtin_expect(split_merge<COT, 2>(acc, sml, pin), 0) && split_odd<COT, 2>(acc))
+    if (__builtin_expect(split_merge<COT, PT>(acc, sml, pin), 0) && split_odd<COT, PT>(acc))
     {
         // (positions from the lane number again: kept for this they would cost the K loop registers)
         int l = lane;
         asm("" : "+v"(l));
-        const float *img[2];
-        int ih[2], iw[2];
-        bool in[2];
+        const float *img[PT];
+        int ih[PT], iw[PT];
+        bool in[PT];
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < PT; ++t)
         {
-            const int pp = (2 * wave + t) * 32 + (l & 31), py = pp / PW;
+            const int pp = (PT * wave + t) * 32 + (l & 31), py = pp / PW;
             ih[t] = py0 + py;
             iw[t] = px0 + pp - py * PW;
             in[t] = pp < NPX;
             img[t] = a.in + (size_t)n * CIB * HW * CB + (l >> 5) * 8;
         }
-        mfma_f32_wave<COT, 2>(a, acc, cg, l & 31, l >> 5, img, ih, iw, in, 0, CIB);
+        mfma_f32_wave<COT, PT>(a, acc, cg, l & 31, l >> 5, img, ih, iw, in, 0, CIB);
     }
-    // the depthwise taps: requested here (held through the K loop they would cost a workgroup of occupancy), used after the
-    // parked tile's barrier
-    float4 w[9];
-    {
-        const float4 *wq = reinterpret_cast<const float4 *>(d.dw_filt + (size_t)dcob * (9 * CB) + dq4);
-#pragma unroll
-        for (int t = 0; t < 9; ++t) w[t] = wq[t * 4];
-    }
-    float4 dbias = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (d.dw_bias) dbias = *reinterpret_cast<const float4 *>(d.dw_bias + dcob * CB + dq4);
     __syncthreads();                                         // every wave has read its last filter operand
     // ---- bias, activation, park in LDS: a lane holds channels c*32 + 8 qq + 4 half + 0..3 of its pixel -------------
     // pixels outside the pointwise layer's map are the depthwise layer's padding: those lanes store zeros (a branch on
     // the lane mask: no select per value)
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < PT; ++t)
     {
         if (pin[t])
         {
@@ -2006,6 +2013,10 @@ __global__ __launch_bounds__(256, COT == 1 ? 4 : 2) void conv_pw_dw3x3_f32_kerne
     __syncthreads();
 
     // ---- depthwise 3x3 on the parked patch ---------------------------------------------------------------------------
+    float4 w[9];
+#pragma unroll
+    for (int t = 0; t < 9; ++t) w[t] = *reinterpret_cast<const float4 *>(&s_dw[((q / 4) * 9 + t) * CB + dq4]);
+    const float4 dbias = *reinterpret_cast<const float4 *>(&s_dw_bias[(q / 4) * CB + dq4]);
     const int dwo = tx * TOW + dx;                           // depthwise output column
     const bool dcol_ok = dx < TOW && dwo < g.Wd;
     const int dxc = dx < TOW ? dx : 0;                       // idle columns read in bounds
@@ -2540,16 +2551,19 @@ int pw_dw_f32(const char *op, int batch, int dw_stride, int dpt, int dpb, int dp
     g.tiles_x = (g.Wd + tow - 1) / tow; g.tiles_y = (g.Hd + toh - 1) / toh;
     const long nt = (long)batch * g.tiles_x * g.tiles_y;
     const StemDwArgs d{dw_filt, dw_bias};
-    // channels per workgroup: 32 (four workgroups per compute unit) is measured ahead of 64 (two; the activation operand is
-    // loaded once per 64 output channels) on every MobileNetV1 pair at batch 64, by 1-3 us.  SMALL_HIP_TUNE key pwdw_cot=1|2.
-    int cot = 1;
-    { static const int v = tune_int("pwdw_cot", 1); if (v == 1 || (v == 2 && Co % 64 == 0 && (cib == 2 || cib == 4 || cib == 8))) cot = v; }
+    // Channels per workgroup: 32 (four waves of two pixel tiles each, four workgroups per compute unit), or 64 (eight waves of one pixel
+    // tile and two channel tiles: the pixels are read and split for twice the channels) where the K loop is the larger part and there
+    // are two such workgroups for every compute unit.  32 -> 64: 128 -> 256 @28x28 batch 64 36.0 -> 33.7 us, 96 -> 192 24.3 -> 22.8, 128 -> 128
+    // @56x56 stride 2 58.3 -> 56.6, batch 16 (512 workgroups) 17.0 -> 15.9, batch 1 6.7 -> 8.5, 128 -> 128 @28x28 batch 8 (64) 8.1 -> 9.9;
+    // 64 -> 128 @56x56 batch 64 45.0 -> 45.6.  SMALL_HIP_TUNE key pwdw_cot=1|2.
+    int cot = cib >= 6 && Co % 64 == 0 && nt * (Co / 64) >= 2 * NUM_CU ? 2 : 1;
+    { static const int v = tune_int("pwdw_cot", 0); if (v == 1 || (v == 2 && Co % 64 == 0 && cib >= 6)) cot = v; }
     g.n_cg = Co / (32 * cot);
     if (nt * g.n_cg > 0x7fffffffL / 2) { set_error("%s: too many tiles for one launch", op); return SMALL_HIP_EINVAL; }
     g.n_wgs = (int)(nt * g.n_cg); g.per_xcd = (g.n_wgs + NUM_XCD - 1) / NUM_XCD;
     const dim3 grid(g.per_xcd * NUM_XCD);
     void (*k)(const ConvArgs, const StemDwArgs, const PwDwGeom) = nullptr;
-#define SHP_PD_(S_, R_) (cot == 2 ? (cib == 2 ? conv_pw_dw3x3_f32_kernel<S_, 2, 2, R_> : cib == 4 ? conv_pw_dw3x3_f32_kernel<S_, 2, 4, R_> : conv_pw_dw3x3_f32_kernel<S_, 2, 8, R_>) \
+#define SHP_PD_(S_, R_) (cot == 2 ? (cib == 6 ? conv_pw_dw3x3_f32_kernel<S_, 2, 6, R_> : conv_pw_dw3x3_f32_kernel<S_, 2, 8, R_>) \
                              : (cib == 1 ? conv_pw_dw3x3_f32_kernel<S_, 1, 1, R_> : cib == 2 ? conv_pw_dw3x3_f32_kernel<S_, 1, 2, R_> : cib == 3 ? conv_pw_dw3x3_f32_kernel<S_, 1, 3, R_> \
                                 : cib == 4 ? conv_pw_dw3x3_f32_kernel<S_, 1, 4, R_> : cib == 6 ? conv_pw_dw3x3_f32_kernel<S_, 1, 6, R_> : conv_pw_dw3x3_f32_kernel<S_, 1, 8, R_>))
 #define SHP_PD(S_) (relu ? SHP_PD_(S_, true) : SHP_PD_(S_, false))
@@ -2557,7 +2571,7 @@ int pw_dw_f32(const char *op, int batch, int dw_stride, int dpt, int dpb, int dp
     k = dw_stride == 1 ? SHP_PD(1) : SHP_PD(2);
 #undef SHP_PD_
 #undef SHP_PD
-    hipLaunchKernelGGL(k, grid, dim3(256), 0, as_stream(stream), a, d, g);
+    hipLaunchKernelGGL(k, grid, dim3(256 * cot), 0, as_stream(stream), a, d, g);
     SHP_LAUNCH_CHECK(op);
     return SMALL_HIP_OK;
 }

@@ -210,3 +210,36 @@ def test_pointwise_dw_random_shapes(lib):
         assert lib.small_hip_depthwise_conv2d_bias_act_f32(batch, 3, 3, ds, dt, db_, dl, dr, Co, H, W, hu.ptr(dmid), hu.ptr(ddf),
                                                            hu.ptr(ddb), act, 0.1, hu.ptr(d2), hu.stream()) == 0, lib.small_hip_last_error()
         assert_equal_exact(hu.host(do), hu.host(d2), what)
+
+
+@pytest.mark.parametrize("case", [  # workgroups of 64 channels (96 or 128 input channels, 512 workgroups at least) and the last size before them
+    (64, 1, 64, 96, 29, 30, True), (43, 2, 128, 96, 29, 27, False), (64, 1, 128, 128, 15, 31, False), (33, 2, 64, 128, 57, 55, True),
+    (63, 1, 64, 128, 29, 27, True), (64, 1, 96, 96, 28, 28, True)], ids=str)
+def test_pointwise_dw_sixty_four_channels(lib, case):
+    """Against float64, with the bound of a chain of Ci + 9 float32 roundings, and (96 channels: fewer than eight K-steps) against this
+    library's two launches bit for bit."""
+    import torch
+    batch, ds, Co, Ci, H, W, bias = case
+    x, f = synth.normal(1, batch * Ci * H * W), synth.he_normal(2, Co * Ci, Ci)
+    fd, b, bd = synth.he_normal(3, Co * 9, 9), synth.normal(4, Co), synth.normal(5, Co)
+    Hd, Wd = capi.out_dim(H, 1, 1, 3, ds), capi.out_dim(W, 1, 1, 3, ds)
+    dx, df, dfd, db, dbd = (hu.dev(a) for a in (x, f, fd, b, bd))
+    y, mid, y2 = hu.dev_empty(batch * Co * Hd * Wd, np.float32), hu.dev_empty(batch * Co * H * W, np.float32), hu.dev_empty(batch * Co * Hd * Wd, np.float32)
+    pb, pbd = (hu.ptr(db), hu.ptr(dbd)) if bias else (None, None)
+    capi.check(lib.small_hip_conv2d_bias_act_dwconv2d_bias_act_f32(batch, 1, 1, 1, 0, 0, 0, 0, 3, 3, ds, 1, 1, 1, 1, Co, Ci, H, W, hu.ptr(dx),
+                                                                   hu.ptr(df), pb, hu.ptr(dfd), pbd, capi.ACT_RELU, 0.0, hu.ptr(y), hu.stream()))
+    capi.check(lib.small_hip_conv2d_bias_act_f32(batch, 1, 1, 1, 0, 0, 0, 0, Co, Ci, H, W, hu.ptr(dx), hu.ptr(df), pb, capi.ACT_RELU, 0.0,
+                                                 hu.ptr(mid), hu.stream()))
+    capi.check(lib.small_hip_depthwise_conv2d_bias_act_f32(batch, 3, 3, ds, 1, 1, 1, 1, Co, H, W, hu.ptr(mid), hu.ptr(dfd), pbd, capi.ACT_RELU,
+                                                           0.0, hu.ptr(y2), hu.stream()))
+    got, two = hu.host(y), hu.host(y2)
+    if Ci < 128:
+        assert np.array_equal(got.view(np.uint8), two.view(np.uint8))
+    xs = torch.from_numpy(x).double().view(batch, Ci // 16, H, W, 16).permute(0, 1, 4, 2, 3).reshape(batch, Ci, H, W)
+    w = torch.from_numpy(f).double().view(Co // 16, Ci // 16, 16, 16).permute(0, 3, 1, 2).reshape(Co, Ci, 1, 1)
+    wd = torch.from_numpy(fd).double().view(Co // 16, 3, 3, 16).permute(0, 3, 1, 2).reshape(Co, 1, 3, 3)
+    tb, tbd = (torch.from_numpy(b).double(), torch.from_numpy(bd).double()) if bias else (None, None)
+    m = torch.relu(torch.nn.functional.conv2d(xs, w, tb))
+    want = torch.relu(torch.nn.functional.conv2d(m, wd, tbd, stride=ds, padding=1, groups=Co))
+    want = want.view(batch, Co // 16, 16, Hd, Wd).permute(0, 1, 3, 4, 2).reshape(-1).numpy()
+    assert np.linalg.norm(got - want) <= (Ci + 9) ** 0.5 * 2.0 ** -24 * np.linalg.norm(want)
