@@ -502,15 +502,13 @@ class HipExecutor:
     @staticmethod
     def _pointwise_dw_pays(op, dw):
         """A pointwise convolution in front of a 3x3 depthwise layer, where one launch is faster than two (batch 64: 32 -> 64
-        @112x112 stride 2 113 -> 51 us, 64 -> 128 @56x56 67 -> 48, 128 -> 256 @28x28 45 -> 37, 96 -> 192 @28x28 34 -> 25): up
-        to 64 input channels, or 96 / 128 in front of a stride-1 depthwise layer (the kernel is built for 16, 32, 48, 64, 96
-        and 128 input channels), and depthwise tiles (14 x 14 at stride 1, 7 x 8 at stride 2) that the output map fills to
-        70% at least.  96 / 128 channels at stride 2 stay two launches from when the products were float32 MFMAs and the
-        halo's cost more than the tensor saved (128 -> 128 @56x56 81 -> 85 us); with split bf16 products that pair is 70 -> 59."""
+        @112x112 stride 2 113 -> 48 us, 64 -> 128 @56x56 67 -> 45, 128 -> 256 @28x28 45 -> 33, 128 -> 128 @56x56 stride 2 64.7 -> 52.5,
+        96 -> 96 47.8 -> 35.2, batch 16 21.8 -> 14.3 and 16.9 -> 10.5, 128 -> 512 @14x14 stride 2 batch 64 22.6 -> 14.6): the kernel is
+        built for 16, 32, 48, 64, 96 and 128 input channels, and the output map has to fill its depthwise tiles (14 x 14 at stride 1,
+        7 x 8 at stride 2) to 70% at least."""
         if not ((op.kh, op.kw, op.stride) == (1, 1, 1) and op.pads == (0, 0, 0, 0) and op.C % CB == 0 and op.Co % 32 == 0):
             return False
-        cib = op.C // CB
-        if not (cib in (1, 2, 3, 4) or (cib in (6, 8) and dw.stride == 1)) or dw.stride not in (1, 2):
+        if op.C // CB not in (1, 2, 3, 4, 6, 8) or dw.stride not in (1, 2):
             return False
         toh, tow = (14, 14) if dw.stride == 1 else (7, 8)
         hd = capi.out_dim(op.H, dw.pads[0], dw.pads[1], 3, dw.stride)
