@@ -27,6 +27,7 @@ void set_error(const char *fmt, ...);
 //   conv_buf=0        operand streams through flat addresses instead of buffer loads (then conv_pw picks the 1x1 loop)
 //   conv_splitk=0|1   force the split-K kernel off / on                             conv_streamk=0|N  equal-share split off / N per CU
 //   conv_streamk_min  least K-steps for the equal-share split                       stem_lds=0  first layers without the LDS kernel
+//   conv_c16=0|1      the 3x3 kernel of sixteen input channels never / on every map
 //   stem_vec=0|1      16-byte staging of first-layer patches                        smallci_valu=1  vector-ALU first layers
 //   pwdw_cot=1|2      channels (x32) per workgroup (2: from 96 input channels on) of the LDS-parked pointwise + depthwise kernel
 //   fuse_form=3       convolution + depthwise pairs through an intermediate buffer: always the two launches

@@ -40,6 +40,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 // ---------------------------------------------------------------------------------------------
 // float32 products on the bf16 matrix pipes.  A float32 number is the exact sum of three bf16 numbers, x = h + m + l: h =
@@ -876,6 +877,205 @@ __global__ __launch_bounds__(256, (COT * PXT == 2 ? 3 : COT * PXT == 1 ? 4 : 2))
     const int lid = (bid % NUM_XCD) * a.per_xcd + bid / NUM_XCD;
     if (lid >= a.n_blocks) return;            // whole workgroup leaves together: no barrier is skipped
     conv_lds_tile<COT, PXT, POOL, PW, true, BUF>(a, lds_a, lid % a.n_co_groups, lid / a.n_co_groups);
+}
+
+// ---------------------------------------------------------------------------------------------
+// 3x3 stride-1 convolution of ONE block of sixteen input channels (the second layer of a detection network: a large map, nine
+// K-steps).  In conv_lds_tile every pixel is fetched and split nine times, once per tap, for at most 32 or 64 output channels, and
+// nine steps do not cover what a workgroup's start and end cost: 16 -> 32 @208x208 + pooling batch 16 took 51.5 us,
+// 124 TFLOP/s.
+// Here a workgroup owns 32 output channels and runs tile after tile of 16 x 16 pixels: the 18 x 18 patch under a tile is split once
+// (1.27 times a pixel) into LDS in MFMA operand order while the tile before it multiplies, and the nine taps' filter operands stay
+// in registers (108 of them) from the first tile to the last.  A wave has two MFMA tiles of 16 columns x 2 rows, one above the
+// other: the middle one of the five input row pairs they read is both tile 0's last and tile 1's first (45 LDS reads for 108 MFMAs).
+// Taps in the order of conv_lds_tile, the same products: the same bits.
+// Persistent workgroups, two per compute unit, each a run of consecutive tiles; runs that follow each other are on one XCD. What
+// bounds it now: matrix cycles and LDS reads of two waves a SIMD (245 registers), and runs of unequal length: batch 16 39.1 us (163 TFLOP/s, runs of
+// five and six tiles), batch 64 193 -> 129 (198 TFLOP/s), 16 -> 32 @104x104 without pooling batch 64 51.0 -> 42.7.
+constexpr int C16_T = 16, C16_PW = 18, C16_PLANE = 328;     // 18 x 18 = 324 pixels; 328: the halves of a pixel lie on different banks
+
+__device__ __forceinline__ float quad_xor1(float v)          // the value of lane ^ 1
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
+}
+
+struct C16Geom
+{
+    int tiles_x, n_tiles, n_run;       // tiles across the map, all tiles, workgroups of a channel group
+    FastDiv fd_img, fd_x;              // by the tiles of an image, by tiles_x
+};
+
+template <bool POOL>
+__global__ __launch_bounds__(256, 2) void conv3x3_c16_f32_kernel(const ConvArgs a, const C16Geom g)
+{
+    __shared__ __align__(16) bf16x8 patch[2][3][2][C16_PLANE];      // [buffer][h, m, l][channel half][pixel]
+    __shared__ __align__(16) float s_bias[32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 31, half = lane >> 5;
+    const int cg = blockIdx.y, CoB = a.Co / CB;
+    const int run = (blockIdx.x % NUM_XCD) * (g.n_run / NUM_XCD) + blockIdx.x / NUM_XCD;      // n_run is a multiple of NUM_XCD
+    const int first = (int)((long long)run * g.n_tiles / g.n_run), last = (int)((long long)(run + 1) * g.n_tiles / g.n_run);
+    if (first >= last) return;                              // the whole workgroup
+    if (tid < 32) s_bias[tid] = a.bias && cg * 32 + tid < a.Co ? a.bias[cg * 32 + tid] : 0.f;
+
+    // staging: unit u < 648 = (pixel u / 2 of the patch, channel half u & 1) is two 16-byte loads, one split, three LDS writes
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(a.in), 0, (int)((size_t)a.batch * CB * a.H * a.W * sizeof(float)), BUF_RSRC_FLAGS);
+    constexpr int NPIX = C16_PW * C16_PW, UNITS = (2 * NPIX + 255) / 256;
+    struct Place { int n, y, x; };                          // image, first row and column of a tile
+    auto place = [&](int tile) {
+        const int n = fast_div(tile, g.fd_img), r = tile - n * (int)g.tiles_x * ((a.Ho + C16_T - 1) / C16_T);
+        const int ty = fast_div(r, g.fd_x);
+        return Place{n, ty * C16_T, (r - ty * g.tiles_x) * C16_T};
+    };
+    u32x4 raw[UNITS][2];
+    auto request = [&](int tile) {
+        const Place t = place(tile);
+#pragma unroll
+        for (int i = 0; i < UNITS; ++i)
+        {
+            const int u = tid + i * 256, p = u >> 1, py = p / C16_PW, px = p - py * C16_PW;
+            const int ih = t.y - a.pt + py, iw = t.x - a.pl + px;
+            const bool ok = p < NPIX && (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
+            const unsigned off = ok ? (unsigned)(((t.n * a.H + ih) * a.W + iw) * (CB * (int)sizeof(float)) + (u & 1) * 32) : BUF_OUT_OF_RANGE;
+            raw[i][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0);
+            raw[i][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 16, 0);
+        }
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < UNITS; ++i)
+        {
+            const int u = tid + i * 256, p = u >> 1, h = u & 1;
+            const Split8 s = split8(__builtin_bit_cast(float4, raw[i][0]), __builtin_bit_cast(float4, raw[i][1]));
+            if ((i + 1) * 256 <= 2 * NPIX || p < NPIX)
+            {
+                patch[buf][0][h][p] = s.h;
+                patch[buf][1][h][p] = s.m;
+                patch[buf][2][h][p] = s.l;
+            }
+        }
+    };
+    request(first);
+
+    // filter operands: eight input channels of this lane's output channel for each tap
+    Split8 A[9];
+    {
+        const int cob = cg * 2 + (col >> 4) < CoB ? cg * 2 + (col >> 4) : CoB - 1;      // rows past Co: garbage, never stored
+        const float *w = a.filt + (size_t)cob * (9 * CB * CB) + half * 8 * CB + (col & 15);
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+        {
+            float x[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) x[k] = w[t * (CB * CB) + k * CB];
+            A[t] = split8(x);
+        }
+    }
+    stage(0);
+    if (first + 1 < last) request(first + 1);
+
+    const int ty0 = wave * 4 + (col >> 4), tx0 = col & 15;   // this lane's pixel of MFMA tile 0 in the workgroup's tile
+    const int HoWo = a.Ho * a.Wo;
+    const int slot = ty0 * C16_PW + tx0;
+    for (int tile = first, buf = 0; tile < last; ++tile, buf ^= 1)
+    {
+        __syncthreads();                                     // this patch is whole, and the other one has been read
+        const bf16x8 *ph = &patch[buf][0][half][slot];
+        floatx16 big[1][2], sml[1][2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) big[0][t][r] = sml[0][t][r] = 0.f;
+#pragma unroll
+        for (int o = 0; o < 5; ++o)                          // input row of the window of tile 0, from 2 on of tile 1 too
+#pragma unroll
+            for (int b = 0; b < 3; ++b)
+            {
+                const int at = o * C16_PW + b;
+                const Split8 B{ph[at], ph[at + 2 * C16_PLANE], ph[at + 4 * C16_PLANE]};
+                if (o <= 2) mfma_split(big[0][0], sml[0][0], A[o * 3 + b], B);
+                if (o >= 2) mfma_split(big[0][1], sml[0][1], A[(o - 2) * 3 + b], B);
+            }
+        // the next tile's patch: requested a tile ago
+        if (tile + 1 < last)
+        {
+            stage(buf ^ 1);
+            if (tile + 2 < last) request(tile + 2);
+        }
+
+        const Place at = place(tile);
+        bool pvalid[2];
+        int oh[2], ow[2];
+        const int Hs = POOL ? a.Ho & ~1 : a.Ho, Ws = POOL ? a.Wo & ~1 : a.Wo;      // pixels that a pooling window covers
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+        {
+            oh[t] = at.y + ty0 + 2 * t;
+            ow[t] = at.x + tx0;
+            pvalid[t] = oh[t] < Hs && ow[t] < Ws;
+        }
+        if (__builtin_expect(split_merge<1, 2>(big, sml, pvalid), 0) && split_odd<1, 2>(big))
+        {
+            const float *img[2];
+            int ih[2], iw[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+            {
+                img[t] = a.in + (size_t)at.n * a.H * a.W * CB + half * 8;
+                ih[t] = oh[t] - a.pt;
+                iw[t] = ow[t] - a.pl;
+            }
+            mfma_f32_wave<1, 2>(a, big, cg, col, half, img, ih, iw, pvalid, 0, 9);
+        }
+        if (!POOL)
+        {
+            unsigned ovoff[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                ovoff[t] = pvalid[t] ? (unsigned)((((size_t)at.n * CoB * HoWo + oh[t] * a.Wo + ow[t]) * CB + 4 * half) * sizeof(float)) : BUF_OUT_OF_RANGE;
+            conv_epilogue_buf<1, 2>(a, big, cg, half, HoWo, ovoff, s_bias);
+        }
+        else
+        {
+            // A window is this lane, lane ^ 1 and the same two of the next row, sixteen lanes on.  Two channel quads change rows in one
+            // instruction: the upper row's lanes end with the first quad's maxima, the lower row's with the second's, and both store.
+            const float nscale = act_scale(a.act, a.slope);
+            const int Wp = a.Wo >> 1, HpWp = (a.Ho >> 1) * Wp, row = col >> 4;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+            {
+                const bool ok = pvalid[t] && (col & 1) == 0;
+                float *o = a.out + ((size_t)at.n * CoB * HpWp + (oh[t] >> 1) * Wp + (ow[t] >> 1)) * CB + 8 * row + 4 * half;
+#pragma unroll
+                for (int q = 0; q < 4; q += 2)
+                {
+                    float v[2][4], m[4];
+#pragma unroll
+                    for (int k = 0; k < 2; ++k)
+                    {
+                        const float4 bb = *reinterpret_cast<const float4 *>(s_bias + 8 * (q + k) + 4 * half);
+                        const float b4[4] = {bb.x, bb.y, bb.z, bb.w};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                        {
+                            const float x = act_bf(big[0][t][4 * (q + k) + e] + b4[e], nscale), y = quad_xor1(x);
+                            v[k][e] = x > y ? x : y;
+                        }
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                    {
+                        const u32x2 r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v[0][e]), __builtin_bit_cast(unsigned, v[1][e]), false, false);
+                        const unsigned r0 = r[0], r1 = r[1];
+                        const float top = __builtin_bit_cast(float, r0), bottom = __builtin_bit_cast(float, r1);
+                        m[e] = top > bottom ? top : bottom;
+                    }
+                    const int cob = cg * 2 + q / 2;
+                    if (ok && cob < CoB) *reinterpret_cast<float4 *>(o + (size_t)cob * HpWp * CB) = make_float4(m[0], m[1], m[2], m[3]);
+                }
+            }
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2080,6 +2280,30 @@ bool buffer_form(const ConvArgs &a)
     return !off && a.slabs == 0 && in_bytes <= BUF_MAX_BYTES && f_bytes <= BUF_MAX_BYTES && out_bytes <= BUF_MAX_BYTES;
 }
 
+// One block of input channels, 3x3, stride 1: tiles of 16 x 16 pixels whose split patches lie in LDS (conv3x3_c16_f32_kernel).
+// false: the shape is another kernel's.  From one tile per compute unit (208x208 + pooling batch 2, 338 tiles, 12.0 -> 9.6 us; 104x104 batch 8,
+// 392, 11.5 -> 10.1; 61x47 48 channels batch 64 28.1 -> 22.5) and where the map fills its tiles to 80%: at 77% level (56x56 batch 32 17.0 -> 17.4, 64
+// 27.8 -> 27.7; 28x28 batch 256 17.4 -> 17.6), at 39% behind (20x20 batch 64 11.5 -> 14.8).  SMALL_HIP_TUNE key conv_c16=0|1 (never / wherever it can run).
+bool launch_c16(ConvArgs &a, hipStream_t s, bool pool)
+{
+    static const int force = tune_int("conv_c16", -1);
+    if (force == 0 || a.Ci != CB || a.kh != 3 || a.kw != 3 || a.stride != 1 || a.stride_h != 1 || !buffer_form(a)) return false;
+    const int tiles_x = (a.Wo + C16_T - 1) / C16_T, tiles_y = (a.Ho + C16_T - 1) / C16_T, n_cg = (a.Co + 31) / 32;
+    const long n_tiles = (long)a.batch * tiles_x * tiles_y;
+    if (n_cg > 65535) return false;
+    if (force != 1 && (n_tiles * n_cg < NUM_CU || 5L * a.Ho * a.Wo < 4L * tiles_x * tiles_y * (C16_T * C16_T))) return false;
+    C16Geom g;
+    g.tiles_x = tiles_x; g.n_tiles = (int)n_tiles;
+    const long wgs = std::max(2L * NUM_CU / n_cg, 1L), most = std::min(wgs, n_tiles);
+    g.n_run = (int)((most + NUM_XCD - 1) / NUM_XCD) * NUM_XCD;
+    g.fd_img = make_fast_div((unsigned)(tiles_x * tiles_y));
+    g.fd_x = make_fast_div((unsigned)tiles_x);
+    const dim3 grid(g.n_run, n_cg);
+    if (pool) hipLaunchKernelGGL(conv3x3_c16_f32_kernel<true>, grid, dim3(256), 0, s, a, g);
+    else hipLaunchKernelGGL(conv3x3_c16_f32_kernel<false>, grid, dim3(256), 0, s, a, g);
+    return true;
+}
+
 void launch_splitk(ConvArgs &a, hipStream_t s)
 {
     set_pixel_divisors(a, false);
@@ -2358,6 +2582,11 @@ int conv_f32(const char *op, int batch, int kh, int kw, int stride, int pt, int 
         int c2 = 0, p2 = 0;
         if (tune_pair("conv_tile", &c2, &p2)) { cot = c2; pxt = p2; }
     }
+    if (launch_c16(a, s, false))
+    {
+        SHP_LAUNCH_CHECK(op);
+        return SMALL_HIP_OK;
+    }
     // few tiles, long reduction: equal shares of the K-steps
     {
         bool done = false;
@@ -2461,6 +2690,11 @@ int conv_pool_f32(const char *op, int batch, int kh, int kw, int stride, int pt,
     a.P = (int)(nwin * 4);
     const long ntiles = (nwin + 7) / 8;
     const long tiles32 = (long)((Co + 31) / 32) * ntiles;
+    if (launch_c16(a, s, true))
+    {
+        SHP_LAUNCH_CHECK(op);
+        return SMALL_HIP_OK;
+    }
     int cot, pxt;
     wave_tile(Co, tiles32, kh * kw * (Ci / CB), &cot, &pxt);
     if (cot == 2 && pxt == 2) launch_mfma_pool<2, 2>(a, s);
