@@ -2416,44 +2416,59 @@ struct GroupSlabs
 // maps: 512 -> 1024 3x3 287 -> 264 us, 1024 -> 1024 519 -> 467 us, 256 -> 512 (144 steps) 81 -> 69 us; with 72 steps or
 // fewer the fix-up pass costs more than the balance gains).  Those are float32 MFMAs; with split products, without -> with, batch
 // 16: 512 -> 1024 162.9 -> 158.2 us, 1024 -> 1024 319.6 -> 301.3, 256 -> 512 52.8 -> 50.2 (batch 26, 20 tiles over a round: 67.0 -> 73.6),
-// and with 72 steps 40.9 -> 50.2.  SMALL_HIP_TUNE keys conv_streamk=<workgroups per compute unit> (default 3, against 2 level to 3% better; 0 = never),
-// conv_streamk_min=<steps> (default 128)
+// and with 72 steps 40.9 -> 50.2.  Wave tile 2x1, three workgroups
+// per compute unit, or 2x2, two (a sixth fewer operands to split for a product), where there are more than 256 of the 2x1 workgroup tiles and 256
+// steps: 2x1 -> 2x2, 1024 -> 1024 304.7 -> 285.2, batch 20 371.5 -> 360.8, 28 494.7 -> 475.4; 512 -> 1024 160.9 -> 154.8, batch 32 300.8 -> 285.6;
+// 512 -> 512 @28x28 batch 12 260.7 -> 247.7; fewer tiles, 512 -> 1024 batch 10 (224) 106.7 -> 110.3, 512 -> 512 @28x28 batch 4 (200)
+// 96.6 -> 104.2; fewer steps, 256 -> 512 batch 26 75.1 -> 79.7, 32 88.2 -> 90.6, 2304 -> 960 1x1 @12x11 batch 20 81.4 -> 86.8 (144).
+// SMALL_HIP_TUNE keys conv_streamk=<workgroups per compute unit> (0 = never), conv_streamk_min=<steps> (default 128)
 template <int COT, int PXT>
-size_t streamk_plan(ConvArgs &a)
+size_t streamk_cut(ConvArgs &a, int per_cu)
 {
-    static const int min_steps = tune_int("conv_streamk_min", 128);
-    static const int per_cu = tune_int("conv_streamk", 3);
-    if (per_cu <= 0 || a.slabs != 0 || a.Co % (32 * COT) != 0) return 0;
     a.n_co_groups = (a.Co + 32 * COT - 1) / (32 * COT);
     a.n_px_blocks = (a.P + 32 * PXT * 4 - 1) / (32 * PXT * 4);
     a.n_blocks = a.n_co_groups * a.n_px_blocks;
-    const int nsteps = a.kh * a.kw * (a.Ci / CB);
+    const int nsteps = a.kh * a.kw * (a.Ci / CB), chunks = per_cu * NUM_CU;
     const long total = (long)a.n_blocks * nsteps;
-    if (a.n_blocks <= NUM_CU / 2 || a.n_blocks >= 3 * NUM_CU || a.n_blocks % NUM_CU == 0 || nsteps < min_steps) return 0;
-    const int chunks = per_cu * NUM_CU;
     a.sk_chunk = (int)((total + chunks - 1) / chunks);
     a.sk_chunks = (int)((total + a.sk_chunk - 1) / a.sk_chunk);
     a.sk_parts = (nsteps + a.sk_chunk - 1) / a.sk_chunk + 1;
     a.per_xcd = (a.sk_chunks + NUM_XCD - 1) / NUM_XCD;
     return (size_t)a.n_blocks * a.sk_parts * sk_part_floats<COT, PXT>() * sizeof(float);
 }
+size_t streamk_plan(ConvArgs &a, int *pxt)
+{
+    static const int min_steps = tune_int("conv_streamk_min", 128);
+    static const int per_cu = tune_int("conv_streamk", -1);
+    if (per_cu == 0 || a.slabs != 0 || a.Co % 64 != 0) return 0;
+    const int nsteps = a.kh * a.kw * (a.Ci / CB);
+    const long tiles = (long)(a.Co / 64) * ((a.P + 127) / 128);
+    if (tiles <= NUM_CU / 2 || tiles >= 3 * NUM_CU || tiles % NUM_CU == 0 || nsteps < min_steps) return 0;
+    *pxt = tiles > NUM_CU && nsteps >= 256 ? 2 : 1;
+    return *pxt == 2 ? streamk_cut<2, 2>(a, per_cu > 0 ? per_cu : 2) : streamk_cut<2, 1>(a, per_cu > 0 ? per_cu : 3);
+}
 
 // the equal-share launch pair; *done = false: the shape does not qualify.  The first call on a stream allocates the
 // scratch block (small_hip_workspace_reserve does it ahead of time), like the uint8 convolution's filter pre-pass.
 template <int COT, int PXT>
+void launch_streamk_tile(const ConvArgs &a, hipStream_t s)
+{
+    if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_streamk_kernel<COT, PXT, true>), dim3(a.per_xcd * NUM_XCD), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((conv_mfma_f32_streamk_kernel<COT, PXT>), dim3(a.per_xcd * NUM_XCD), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((conv_streamk_fixup_kernel<COT, PXT>), dim3(a.n_blocks), dim3(256), 0, s, a);
+}
 int launch_streamk(const char *op, ConvArgs &a, hipStream_t s, bool *done)
 {
     *done = false;
     set_pixel_divisors(a, false);
-    const size_t bytes = streamk_plan<COT, PXT>(a);
+    int pxt = 1;
+    const size_t bytes = streamk_plan(a, &pxt);
     if (bytes == 0) return SMALL_HIP_OK;
     WorkspaceLease lease;            // held until both launches are enqueued
     if (int rc = lease_workspace(bytes, s, &lease)) return rc;
     a.sk_scratch = static_cast<float *>(lease.ptr);
-    if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_streamk_kernel<COT, PXT, true>), dim3(a.per_xcd * NUM_XCD), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((conv_mfma_f32_streamk_kernel<COT, PXT>), dim3(a.per_xcd * NUM_XCD), dim3(256), 0, s, a);
-    SHP_LAUNCH_CHECK(op);
-    hipLaunchKernelGGL((conv_streamk_fixup_kernel<COT, PXT>), dim3(a.n_blocks), dim3(256), 0, s, a);
+    if (pxt == 2) launch_streamk_tile<2, 2>(a, s);
+    else launch_streamk_tile<2, 1>(a, s);
     SHP_LAUNCH_CHECK(op);
     *done = true;
     return SMALL_HIP_OK;
@@ -2590,7 +2605,7 @@ int conv_f32(const char *op, int batch, int kh, int kw, int stride, int pt, int 
     // few tiles, long reduction: equal shares of the K-steps
     {
         bool done = false;
-        if (int rc = launch_streamk<2, 1>(op, a, s, &done)) return rc;
+        if (int rc = launch_streamk(op, a, s, &done)) return rc;
         if (done) return SMALL_HIP_OK;
     }
     if (cot == 2 && pxt == 2) launch_mfma<2, 2>(a, s);
@@ -2885,7 +2900,8 @@ size_t small_hip_conv2d_f32_workspace_bytes(int batch, int kh, int kw, int strid
     if (P <= 0 || P > 0x7fffffffL / 64) return 0;
     a.P = (int)P;
     if (wants_splitk((long)((Co + 31) / 32) * ((P + 31) / 32), kh * kw * (Ci / CB))) return 0;
-    return streamk_plan<2, 1>(a);
+    int pxt;
+    return streamk_plan(a, &pxt);
 }
 
 int small_hip_conv2d_dwconv2d_one_launch_f32(int batch, int kh, int kw, int stride, int pt, int pb, int pl, int pr, int dw_kh,

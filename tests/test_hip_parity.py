@@ -95,6 +95,27 @@ EQUAL_SHARE_CASES = [
 ]
 
 
+@pytest.mark.parametrize("case", [(1, 3, (1, 1, 1, 1), 512, 512, 65, 65, False), (2, 1, (0, 0, 0, 0), 576, 4096, 50, 37, True)], ids=str)
+def test_conv2d_f32_equal_share_split_larger_wave_tile(lib, case):
+    """More than 256 workgroup tiles and 256 K-steps: 64 x 256 tiles instead of 64 x 128, the last pixel block a fraction of one.  Against
+    float64 with the bound of a chain of float32 roundings."""
+    import torch
+    batch, k, (pt, pb, pl, pr), Co, Ci, H, W, partial = case
+    x, f = synth.normal(31, batch * Ci * H * W), synth.he_normal(32, Co * Ci * k * k, Ci * k * k)
+    old, bias = synth.normal(33, batch * Co * H * W), synth.normal(34, Co)
+    n_tiles, steps = (Co // 64) * -(-(batch * H * W) // 128), k * k * Ci // 16
+    assert 256 < n_tiles < 768 and n_tiles % 256 and steps >= 256, "the case would not take the larger tile"
+    dx, df, do, db = hu.dev(x), hu.dev(f), hu.dev(old), hu.dev(bias)
+    fn = lib.small_hip_partial_conv2d_bias_act_f32 if partial else lib.small_hip_conv2d_bias_act_f32
+    capi.check(fn(batch, k, k, 1, pt, pb, pl, pr, Co, Ci, H, W, hu.ptr(dx), hu.ptr(df), hu.ptr(db), capi.ACT_LEAKY, 0.1, hu.ptr(do), hu.stream()))
+    unpack = lambda a, c: torch.from_numpy(a).double().view(batch, c // CB, H, W, CB).permute(0, 1, 4, 2, 3).reshape(batch, c, H, W)
+    w = torch.from_numpy(f).double().view(Co // CB, Ci // CB, k, k, CB, CB).permute(0, 5, 1, 4, 2, 3).reshape(Co, Ci, k, k)
+    want = torch.nn.functional.conv2d(unpack(x, Ci), w, padding=pt) + torch.from_numpy(bias).double().view(1, -1, 1, 1)
+    want = want + unpack(old, Co) if partial else want
+    want = torch.where(want > 0, want, want * 0.1).view(batch, Co // CB, CB, H, W).permute(0, 1, 3, 4, 2).reshape(-1).numpy()
+    assert np.linalg.norm(hu.host(do) - want) <= (Ci * k * k) ** 0.5 * 2.0 ** -24 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("mode", ["conv", "partial", "bias_leaky"])
 @pytest.mark.parametrize("case", EQUAL_SHARE_CASES, ids=str)
 def test_conv2d_f32_equal_share_split(lib, oracle, case, mode):
