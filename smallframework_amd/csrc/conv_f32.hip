@@ -2328,20 +2328,21 @@ void launch_splitk(ConvArgs &a, hipStream_t s)
 
 // Whole rounds + cut tail (conv_mfma_f32_hybrid_kernel) or whole tiles only?  A split-K piece multiplies about half as
 // fast as a whole tile (operands straight from global memory, both split for one MFMA tile), so the cut tail wins while the
-// left-over tiles fill at most two thirds of a round.  Batch sweeps, left-over tiles of 256: us with whole tiles only -> with the
+// left-over tiles fill at most two thirds of a round, and half a round where a whole tile splits less (2x1).
+// Batch sweeps, left-over tiles of 256: us with whole tiles only -> with the
 // cut tail.  Wave tile 1x1: 128->128 1x1 @20x20 (8 K-steps) 30: 11.6 -> 10.0, 213: 9.7 -> 10.5; 192->256 @14x14 (12) 125: 11.3 ->
 // 10.5, 200: 11.6 -> 13.0; 3x3 64->128 @52x52 (36) 82: 16.9 -> 15.0, 167: 17.5 -> 16.8, 250: 18.9 -> 20.1; 3x3 128->256 @26x26
-// (72) 82: 29.4 -> 27.2, 169: 31.9 -> 30.8, 250: level.  Wave tile 2x1, which loses from half a round on already: 192->256
-// @14x14 174: 13.0 -> 14.8; 256->256 1x1 @28x28 (16) 38: 14.4 -> 11.3, 136: 15.0 -> 15.1, 186: 15.6 -> 16.5; 512->512 @14x14 (32) 112: 24.2 -> 21.5,
-// 162: 25.2 -> 26.7; 3x3 64->64 @56x56 (36) 136: 27.2 -> 28.6; 3x3 128->256 @26x26 40: 45.7 -> 37.1, 126: 49.2 -> 46.1.
+// (72) 82: 29.4 -> 27.2, 169: 31.9 -> 30.8, 250: level.  Wave tile 2x1: 1x1 512->512 @14x14 (32) 40: 22.6 -> 18.1, 88: 23.2 -> 19.9;
+// 3x3 64->64 @56x56 (36) 112: 26.1 -> 24.4, 125: 37.7 -> 39.2, 136: 26.8 -> 28.2; 3x3 96->192 @30x30 (54) 121: 54.3 -> 53.5; 3x3 128->256
+// @26x26 (72) 126: 49.2 -> 46.1; with pooling 168: 51.1 -> 54.8, 64->128 @52x52 164: 40.3 -> 43.5; 1x1 1024->1024 @7x7 (64) 144: 43.5 -> 44.5,
+// 176: 45.6 -> 48.5; 256->256 @28x28 (16) 136: level, 164: 15.2 -> 16.1, five rounds and 168: 40.0 -> 43.4; 128->256 (8) 176: 13.1 -> 15.3.
 template <int COT, int PXT>
-bool tail_pays(int n_main, int rest, int nsteps)
+bool tail_pays(int rest, int nsteps)
 {
     // SMALL_HIP_TUNE key conv_tail: 0 = never, 2 = whenever tiles are left over
     static const int knob = tune_int("conv_tail", 1);
-    (void)n_main;
     if (knob == 0 || rest == 0 || nsteps < 8) return false;
-    return knob == 2 || rest <= 11 * NUM_CU / 16;
+    return knob == 2 || rest <= (COT == 2 && PXT == 1 ? NUM_CU / 2 : 11 * NUM_CU / 16);
 }
 
 // Wave tile in 32-channel x 32-pixel MFMA tiles.  The split of the operands is what a larger tile saves: one pixel tile split
@@ -2386,7 +2387,7 @@ void launch_mfma(ConvArgs &a, hipStream_t s)
     const bool pw = !buf && !pw_off && a.kh == 1 && a.kw == 1 && a.stride == 1 && a.stride_h == 1 && a.pt == 0 && a.pl == 0 &&
                     a.Ho == a.H && a.Wo == a.W;
     const unsigned slabs_y = a.slabs > 0 ? a.slabs : 1;
-    if (tail_pays<COT, PXT>(n_main, rest, a.kh * a.kw * (a.Ci / CB)))
+    if (tail_pays<COT, PXT>(rest, a.kh * a.kw * (a.Ci / CB)))
     {
         a.n_main = n_main;
         const dim3 grid(n_main + rest * 4 * COT * PXT, slabs_y);
@@ -2625,7 +2626,7 @@ void launch_mfma_pool(ConvArgs &a, hipStream_t s)
     a.n_blocks = a.n_co_groups * a.n_px_blocks;
     a.per_xcd = (a.n_blocks + NUM_XCD - 1) / NUM_XCD;
     const int n_main = a.n_blocks / NUM_CU * NUM_CU, rest = a.n_blocks - n_main;
-    if (tail_pays<COT, PXT>(n_main, rest, a.kh * a.kw * (a.Ci / CB)))
+    if (tail_pays<COT, PXT>(rest, a.kh * a.kw * (a.Ci / CB)))
     {
         a.n_main = n_main;
         if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_hybrid_kernel<COT, PXT, true, false, true>), dim3(n_main + rest * 4 * COT * PXT), dim3(256), 0, s, a);

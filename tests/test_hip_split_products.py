@@ -53,7 +53,8 @@ SHAPES = [  # batch, window, stride, Co, Ci, H, W
     (24, 3, 1, 64, 32, 28, 28),
     (40, 1, 1, 256, 64, 28, 28),      # two channel tiles per wave
     (20, 3, 2, 128, 64, 57, 57),
-    (16, 3, 1, 128, 64, 52, 52),      # cut tail
+    (16, 3, 1, 128, 64, 52, 52),      # whole tiles, 164 of them in the last round
+    (15, 3, 1, 64, 64, 56, 56),       # cut tail: 112 left over
     (8, 3, 1, 512, 160, 13, 13),      # 90 steps: split K over eight waves
     (16, 3, 1, 512, 240, 13, 13),     # equal shares of the reduction (equal_shares below)
     (56, 3, 1, 128, 64, 56, 56),      # 2 x 2 tiles
@@ -147,7 +148,8 @@ FORMS = [
     (40, 1, 1, 256, 64, 28, 28),      # two channel tiles a wave
     (13, 3, 1, 32, 32, 105, 103),     # two pixel tiles a wave
     (56, 3, 1, 128, 64, 56, 56),      # 2 x 2
-    (16, 3, 1, 128, 64, 52, 52),      # cut tail
+    (16, 3, 1, 128, 64, 52, 52),      # whole tiles, 164 of them in the last round
+    (15, 3, 1, 64, 64, 56, 56),       # cut tail: 112 left over
     (16, 3, 1, 512, 240, 13, 13),     # equal shares of the reduction
 ]
 PAIR_CHANNELS = [16, 32, 48, 64, 96, 128]    # input channels of the pointwise + depthwise kernel
