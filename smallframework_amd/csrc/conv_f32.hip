@@ -2328,21 +2328,23 @@ void launch_splitk(ConvArgs &a, hipStream_t s)
 
 // Whole rounds + cut tail (conv_mfma_f32_hybrid_kernel) or whole tiles only?  A split-K piece multiplies about half as
 // fast as a whole tile (operands straight from global memory, both split for one MFMA tile), so the cut tail wins while the
-// left-over tiles fill at most two thirds of a round, and half a round where a whole tile splits less (2x1).
+// left-over tiles fill at most two thirds of a round, and half a round with larger wave tiles, which split less.
 // Batch sweeps, left-over tiles of 256: us with whole tiles only -> with the
 // cut tail.  Wave tile 1x1: 128->128 1x1 @20x20 (8 K-steps) 30: 11.6 -> 10.0, 213: 9.7 -> 10.5; 192->256 @14x14 (12) 125: 11.3 ->
 // 10.5, 200: 11.6 -> 13.0; 3x3 64->128 @52x52 (36) 82: 16.9 -> 15.0, 167: 17.5 -> 16.8, 250: 18.9 -> 20.1; 3x3 128->256 @26x26
 // (72) 82: 29.4 -> 27.2, 169: 31.9 -> 30.8, 250: level.  Wave tile 2x1: 1x1 512->512 @14x14 (32) 40: 22.6 -> 18.1, 88: 23.2 -> 19.9;
 // 3x3 64->64 @56x56 (36) 112: 26.1 -> 24.4, 125: 37.7 -> 39.2, 136: 26.8 -> 28.2; 3x3 96->192 @30x30 (54) 121: 54.3 -> 53.5; 3x3 128->256
 // @26x26 (72) 126: 49.2 -> 46.1; with pooling 168: 51.1 -> 54.8, 64->128 @52x52 164: 40.3 -> 43.5; 1x1 1024->1024 @7x7 (64) 144: 43.5 -> 44.5,
-// 176: 45.6 -> 48.5; 256->256 @28x28 (16) 136: level, 164: 15.2 -> 16.1, five rounds and 168: 40.0 -> 43.4; 128->256 (8) 176: 13.1 -> 15.3.
+// 176: 45.6 -> 48.5; 256->256 @28x28 (16) 136: level, 164: 15.2 -> 16.1, five rounds and 168: 40.0 -> 43.4; 128->256 (8) 176: 13.1 -> 15.3. 1x2: 3x3 96->96 @30x30 (18)
+// 91: 61.1 -> 54.8, 142: 63.0 -> 62.6, 163: 63.7 -> 65.2; 32->32 @56x56 (18) 150: 25.8 -> 27.3.  2x2: 256->256 @56x56 (144) 103: 441.8 -> 433.4,
+// 141: 534.2 -> 542.8, 152: 445.8 -> 459.0; 1x1 512->512 @28x28 (32) 152: 111.2 -> 117.9.
 template <int COT, int PXT>
 bool tail_pays(int rest, int nsteps)
 {
     // SMALL_HIP_TUNE key conv_tail: 0 = never, 2 = whenever tiles are left over
     static const int knob = tune_int("conv_tail", 1);
     if (knob == 0 || rest == 0 || nsteps < 8) return false;
-    return knob == 2 || rest <= (COT == 2 && PXT == 1 ? NUM_CU / 2 : 11 * NUM_CU / 16);
+    return knob == 2 || rest <= (COT * PXT > 1 ? NUM_CU / 2 : 11 * NUM_CU / 16);
 }
 
 // Wave tile in 32-channel x 32-pixel MFMA tiles.  The split of the operands is what a larger tile saves: one pixel tile split
