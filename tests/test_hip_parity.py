@@ -86,8 +86,7 @@ def test_conv2d_f32(lib, oracle, case, mode):
 
 # few workgroup tiles and a long reduction: the equal-share split of the K-steps (two runs per compute unit, raw
 # accumulators through a scratch block, fixed-order fix-up pass).  First case: 136 tiles x 144 steps, every tile cut into
-# four or five runs; second: 600 tiles, runs of 169 steps, so some runs hold a whole tile (written through the epilogue
-# directly) next to pieces of its neighbours; third: 5x5 window, stride 2, a ragged last pixel block.
+# four or five runs; second: 600 tiles of 144 steps, which run as whole rounds and a rest; third: 5x5 window, stride 2, a ragged last pixel block.
 EQUAL_SHARE_CASES = [
     (1, 3, 3, 1, (1, 1, 1, 1), 256, 256, 65, 65),
     (1, 3, 3, 1, (1, 1, 1, 1), 64, 256, 240, 320),
