@@ -715,7 +715,7 @@ def main():
         roof = {"bound": "mfma", "achieved": round(ach, 3), "peak": round(pk / 1e12, 1),
                 "unit": "TOP/s" if model.dtype == "u8" else "TFLOP/s",
                 "frac": round(ach / (pk / 1e12), 4), "traffic": None,
-                "kernel": "qmodel_u8_kernel" if model.dtype == "u8" else "fmodel_f32_kernel",
+                "kernel": "qmodel_u8_kernel" if model.dtype == "u8" else "fmodel_f32_sep_kernel",
                 "launches_per_step": 1, "avg_launch_ms": round(sec * 1e3, 5),
                 "algorithmic_per_launch": {"GOP": round(batch * model.flops_per_image() / 1e9, 3),
                                            "MB": round(algo / 1e6, 3)},
