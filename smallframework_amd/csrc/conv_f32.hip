@@ -1377,10 +1377,12 @@ __global__ __launch_bounds__(256, (COT * PXT == 2 ? 3 : COT * PXT == 1 ? 4 : 2))
     }
 }
 
+// A workgroup adds up one 32 x 32 tile of each wave: what bounds it is memory, and a whole workgroup tile per workgroup leaves compute
+// units idle (1024 -> 1024 @13x13 batch 16, 176 tiles of 2x2: 14.6 us, now 10.2).
 template <int COT, int PXT>
 __global__ __launch_bounds__(256) void conv_streamk_fixup_kernel(const ConvArgs a)
 {
-    const int tile = blockIdx.x;
+    const int tile = blockIdx.x, c = blockIdx.y / PXT, t = blockIdx.y % PXT;
     const int nsteps = a.kh * a.kw * (a.Ci / CB);
     const int first = (int)(((long)tile * nsteps) / a.sk_chunk);
     const int last = (int)(((long)(tile + 1) * nsteps - 1) / a.sk_chunk);
@@ -1388,36 +1390,25 @@ __global__ __launch_bounds__(256) void conv_streamk_fixup_kernel(const ConvArgs 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 31, half = lane >> 5;
     const int cg = tile % a.n_co_groups, pxb = tile / a.n_co_groups;
     const int HoWo = a.Ho * a.Wo, CoB = a.Co / CB;
-    bool pvalid[PXT];
-    size_t out_pix[PXT];
-#pragma unroll
-    for (int t = 0; t < PXT; ++t)
-    {
-        const int p = ((pxb * 4 + wave) * PXT + t) * 32 + col;
-        pvalid[t] = p < a.P;
-        const int pc = pvalid[t] ? p : 0;
-        const int n = pc / HoWo, rem = pc - n * HoWo;
-        out_pix[t] = ((size_t)n * CoB * HoWo + rem) * CB;
-    }
-    floatx16 acc[COT][PXT];
+    const int p = ((pxb * 4 + wave) * PXT + t) * 32 + col;
+    const bool pvalid[1] = {p < a.P};
+    const int pc = pvalid[0] ? p : 0, n = pc / HoWo, rem = pc - n * HoWo;
+    const size_t out_pix[1] = {((size_t)n * CoB * HoWo + rem) * CB};
+    floatx16 acc[1][1];
     const float4 *r4 = reinterpret_cast<const float4 *>(a.sk_scratch + (size_t)tile * a.sk_parts * sk_part_floats<COT, PXT>()) +
-                       (size_t)wave * (COT * PXT * 4 * WAVE) + lane;
+                       (size_t)((wave * COT + c) * PXT + t) * (4 * WAVE) + lane;
     for (int part = 0; part <= last - first; ++part)
     {
 #pragma unroll
-        for (int c = 0; c < COT; ++c)
-#pragma unroll
-            for (int t = 0; t < PXT; ++t)
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                {
-                    const float4 v = r4[((c * PXT + t) * 4 + q) * WAVE];
-                    if (part == 0) { acc[c][t][4 * q] = v.x; acc[c][t][4 * q + 1] = v.y; acc[c][t][4 * q + 2] = v.z; acc[c][t][4 * q + 3] = v.w; }
-                    else { acc[c][t][4 * q] += v.x; acc[c][t][4 * q + 1] += v.y; acc[c][t][4 * q + 2] += v.z; acc[c][t][4 * q + 3] += v.w; }
-                }
+        for (int q = 0; q < 4; ++q)
+        {
+            const float4 v = r4[q * WAVE];
+            if (part == 0) { acc[0][0][4 * q] = v.x; acc[0][0][4 * q + 1] = v.y; acc[0][0][4 * q + 2] = v.z; acc[0][0][4 * q + 3] = v.w; }
+            else { acc[0][0][4 * q] += v.x; acc[0][0][4 * q + 1] += v.y; acc[0][0][4 * q + 2] += v.z; acc[0][0][4 * q + 3] += v.w; }
+        }
         r4 += sk_part_floats<COT, PXT>() / 4;
     }
-    conv_epilogue<COT, PXT>(a, acc, cg, half, HoWo, pvalid, out_pix);
+    conv_epilogue<1, 1>(a, acc, cg * COT + c, half, HoWo, pvalid, out_pix);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2461,7 +2452,7 @@ void launch_streamk_tile(const ConvArgs &a, hipStream_t s)
 {
     if (buffer_form(a)) hipLaunchKernelGGL((conv_mfma_f32_streamk_kernel<COT, PXT, true>), dim3(a.per_xcd * NUM_XCD), dim3(256), 0, s, a);
     else hipLaunchKernelGGL((conv_mfma_f32_streamk_kernel<COT, PXT>), dim3(a.per_xcd * NUM_XCD), dim3(256), 0, s, a);
-    hipLaunchKernelGGL((conv_streamk_fixup_kernel<COT, PXT>), dim3(a.n_blocks), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((conv_streamk_fixup_kernel<COT, PXT>), dim3(a.n_blocks, COT * PXT), dim3(256), 0, s, a);
 }
 int launch_streamk(const char *op, ConvArgs &a, hipStream_t s, bool *done)
 {
