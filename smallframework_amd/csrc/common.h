@@ -9,14 +9,13 @@
 #include <mutex>
 
 #include "../../include/small_hip.h"
+#include "launch_rules.h"
 
 namespace shp
 {
 
 constexpr int CB = SMALL_HIP_CB;          // channel block of every packed tensor
 constexpr int WAVE = 64;                  // gfx950 wavefront
-constexpr int NUM_XCD = 8;                // MI355X: 8 XCDs x 32 CUs, one L2 per XCD
-constexpr int NUM_CU = 256;
 
 void set_error(const char *fmt, ...);
 

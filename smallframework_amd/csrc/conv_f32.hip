@@ -2272,21 +2272,20 @@ bool buffer_form(const ConvArgs &a)
 }
 
 // One block of input channels, 3x3, stride 1: tiles of 16 x 16 pixels whose split patches lie in LDS (conv3x3_c16_f32_kernel).
-// false: the shape is another kernel's.  From one tile per compute unit (208x208 + pooling batch 2, 338 tiles, 12.0 -> 9.6 us; 104x104 batch 8,
-// 392, 11.5 -> 10.1; 61x47 48 channels batch 64 28.1 -> 22.5) and where the map fills its tiles to 80%: at 77% level (56x56 batch 32 17.0 -> 17.4, 64
-// 27.8 -> 27.7; 28x28 batch 256 17.4 -> 17.6), at 39% behind (20x20 batch 64 11.5 -> 14.8).  SMALL_HIP_TUNE key conv_c16=0|1 (never / wherever it can run).
+// false: the shape is another kernel's, by c16_runs or because the map fills its tiles to less than 80%: at 77% level (56x56 batch 32
+// 17.0 -> 17.4, 64 27.8 -> 27.7; 28x28 batch 256 17.4 -> 17.6), at 39% behind (20x20 batch 64 11.5 -> 14.8).  SMALL_HIP_TUNE key
+// conv_c16=0|1 (never / wherever it can run).
 bool launch_c16(ConvArgs &a, hipStream_t s, bool pool)
 {
     static const int force = tune_int("conv_c16", -1);
     if (force == 0 || a.Ci != CB || a.kh != 3 || a.kw != 3 || a.stride != 1 || a.stride_h != 1 || !buffer_form(a)) return false;
     const int tiles_x = (a.Wo + C16_T - 1) / C16_T, tiles_y = (a.Ho + C16_T - 1) / C16_T, n_cg = (a.Co + 31) / 32;
     const long n_tiles = (long)a.batch * tiles_x * tiles_y;
-    if (n_cg > 65535) return false;
-    if (force != 1 && (n_tiles * n_cg < NUM_CU || 5L * a.Ho * a.Wo < 4L * tiles_x * tiles_y * (C16_T * C16_T))) return false;
+    if (force != 1 && 5L * a.Ho * a.Wo < 4L * tiles_x * tiles_y * (C16_T * C16_T)) return false;
     C16Geom g;
     g.tiles_x = tiles_x; g.n_tiles = (int)n_tiles;
-    const long wgs = std::max(2L * NUM_CU / n_cg, 1L), most = std::min(wgs, n_tiles);
-    g.n_run = (int)((most + NUM_XCD - 1) / NUM_XCD) * NUM_XCD;
+    g.n_run = c16_runs(n_tiles, n_cg, force == 1);
+    if (g.n_run == 0) return false;
     g.fd_img = make_fast_div((unsigned)(tiles_x * tiles_y));
     g.fd_x = make_fast_div((unsigned)tiles_x);
     const dim3 grid(g.n_run, n_cg);

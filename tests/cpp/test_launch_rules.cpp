@@ -1,0 +1,49 @@
+// CPU unit test of the launch rules (smallframework_amd/csrc/launch_rules.h).
+#include <cstdio>
+
+#include "../../smallframework_amd/csrc/launch_rules.h"
+
+using namespace shp;
+
+static int g_failures = 0;
+#define CHECK(c)                                                                  \
+    do                                                                            \
+    {                                                                             \
+        if (!(c))                                                                 \
+        {                                                                         \
+            std::printf("FAILED %s:%d: %s\n", __FILE__, __LINE__, #c);            \
+            ++g_failures;                                                         \
+        }                                                                         \
+    } while (0)
+
+// 3x3 convolutions of sixteen input channels: the workgroups of all channel groups are resident at once (two per compute unit), every
+// XCD has as many, and none of the tiles is left out
+static void test_c16_workgroups_are_resident_at_once()
+{
+    for (int always = 0; always < 2; ++always)
+        for (int n_cg = 1; n_cg <= 80; ++n_cg)
+            for (long n_tiles = 1; n_tiles <= 20000; n_tiles += n_tiles < 700 ? 1 : 37)
+            {
+                const int n = c16_runs(n_tiles, n_cg, always != 0);
+                CHECK(n * n_cg <= 2 * NUM_CU && n % NUM_XCD == 0 && n >= 0);
+                if (g_failures) return;
+            }
+    CHECK(c16_runs(3136, 1) == 512 && c16_runs(3136, 2) == 256 && c16_runs(3136, 3) == 168 && c16_runs(3136, 5) == 96);
+    CHECK(c16_runs(3136, 64) == 8 && c16_runs(3136, 65) == 0);
+}
+
+// few tiles, or runs of unequal length: the places are not busy enough
+static void test_c16_leaves_ragged_launches_to_the_others()
+{
+    CHECK(c16_runs(338, 1) == 344 && c16_runs(392, 1) == 392);                          // 66%, 77%
+    CHECK(c16_runs(98, 3) == 0 && c16_runs(147, 4) == 0 && c16_runs(204, 3) == 0);      // 57%, 57% (two tiles for 1.1), 60%
+    CHECK(c16_runs(98, 3, true) == 104);
+}
+
+int main()
+{
+    test_c16_workgroups_are_resident_at_once();
+    test_c16_leaves_ragged_launches_to_the_others();
+    std::printf(g_failures ? "%d CHECKS FAILED\n" : "ALL PASSED\n", g_failures);
+    return g_failures ? 1 : 0;
+}

@@ -37,10 +37,20 @@ def _packed(y):
 
 # images x tiles: one run a workgroup, runs of unequal length, channel groups that are half empty, ragged right and lower edges, pads on
 # some sides only (rows and columns that no window covers in the pooled form)
-CASES = [(4, 16, 128, 128, (1, 1, 1, 1), True, capi.ACT_RELU), (11, 32, 77, 95, (1, 1, 1, 1), True, capi.ACT_LEAKY),
-         (30, 48, 47, 61, (1, 1, 1, 1), False, capi.ACT_NONE), (3, 96, 130, 131, (0, 0, 0, 0), True, capi.ACT_RELU),
+CASES = [(6, 16, 128, 128, (1, 1, 1, 1), True, capi.ACT_RELU), (12, 32, 77, 95, (1, 1, 1, 1), True, capi.ACT_LEAKY),
+         (30, 48, 47, 61, (1, 1, 1, 1), False, capi.ACT_NONE), (4, 96, 130, 131, (0, 0, 0, 0), True, capi.ACT_RELU),
          (43, 64, 31, 33, (1, 0, 0, 1), True, capi.ACT_LEAKY), (2, 32, 209, 207, (2, 1, 0, 2), True, capi.ACT_RELU),
-         (260, 16, 16, 16, (1, 1, 1, 1), True, capi.ACT_RELU), (25, 32, 111, 110, (1, 1, 1, 1), True, capi.ACT_LEAKY)]
+         (350, 16, 16, 16, (1, 1, 1, 1), True, capi.ACT_RELU), (25, 32, 111, 110, (1, 1, 1, 1), True, capi.ACT_LEAKY),
+         (24, 80, 61, 47, (1, 1, 1, 1), True, capi.ACT_RELU), (24, 192, 61, 47, (1, 1, 1, 1), False, capi.ACT_NONE)]
+
+
+def runs(n, co, ho, wo):
+    """The launcher's rule: (workgroups of a channel group, channel groups), or None where the shape is another kernel's."""
+    tiles, groups = n * -(-ho // 16) * -(-wo // 16), -(-co // 32)
+    most = 512 // groups // 8 * 8
+    if most == 0 or 20 * tiles * groups < 13 * -(-tiles // most) * 512 or 5 * n * ho * wo < 4 * tiles * 256:
+        return None
+    return min(most, -(-tiles // 8) * 8), groups
 
 
 @pytest.mark.parametrize("case", CASES, ids=str)
@@ -49,6 +59,8 @@ def test_conv3x3_of_one_block(lib, case):
     n, co, h, w, pads, has_bias, act = case
     t, b, l, r = pads
     ho, wo = capi.out_dim(h, t, b, 3, 1), capi.out_dim(w, l, r, 3, 1)
+    grid = runs(n, co, ho, wo)
+    assert grid and grid[0] * grid[1] <= 512, "the case would run in another kernel, or in more workgroups than are resident at once"
     x, f, bias = synth.normal(1, n * 16 * h * w), synth.he_normal(2, co * 144, 144), synth.normal(3, co) if has_bias else None
     old = synth.normal(4, n * co * ho * wo)
     dx, df, db = hu.dev(x), hu.dev(f), hu.dev(bias) if has_bias else None
@@ -74,7 +86,8 @@ def test_conv3x3_of_one_block(lib, case):
 def test_conv3x3_of_one_block_special_values(lib):
     """Sums that are not finite or very small are made again with float32 products: infinities, NaN and the smallest numbers end where
     float64 puts them."""
-    n, co, h, w = 4, 32, 130, 126
+    n, co, h, w = 5, 32, 130, 126
+    assert runs(n, co, h, w)
     x, f = synth.normal(5, n * 16 * h * w), synth.he_normal(6, co * 144, 144)
     rng = np.random.RandomState(7)
     at = rng.choice(x.size, 24, replace=False)
