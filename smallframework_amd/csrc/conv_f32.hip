@@ -2404,18 +2404,8 @@ struct GroupSlabs
     int stride_h = 0;        // > 0: another vertical stride (1 for the 1-D layers)
 };
 
-// The equal-share split of a launch: fills the sk_* fields and the tile counts; returns the scratch bytes it needs, 0 when
-// the shape does not qualify.  Few tiles that do not fill whole rounds and a long reduction (measured, batch 16 on 13x13
-// maps: 512 -> 1024 3x3 287 -> 264 us, 1024 -> 1024 519 -> 467 us, 256 -> 512 (144 steps) 81 -> 69 us; with 72 steps or
-// fewer the fix-up pass costs more than the balance gains).  Those are float32 MFMAs; with split products, without -> with, batch
-// 16: 512 -> 1024 162.9 -> 158.2 us, 1024 -> 1024 319.6 -> 301.3, 256 -> 512 52.8 -> 50.2,
-// and with 72 steps 40.9 -> 50.2.  Wave tile 2x1, three workgroups
-// per compute unit, or 2x2, two (a sixth fewer operands to split for a product), where there are more than 256 of the 2x1 workgroup tiles and 256
-// steps: 2x1 -> 2x2, 1024 -> 1024 304.7 -> 285.2, batch 20 371.5 -> 360.8, 28 494.7 -> 475.4; 512 -> 1024 160.9 -> 154.8, batch 32 300.8 -> 285.6;
-// 512 -> 512 @28x28 batch 12 260.7 -> 247.7; fewer tiles, 512 -> 1024 batch 10 (224) 106.7 -> 110.3, 512 -> 512 @28x28 batch 4 (200)
-// 96.6 -> 104.2.  More than 256 tiles and fewer steps are whole rounds and a rest in the other launch (256 -> 512 batch 26, 280 tiles, 73.7 -> 67.7,
-// 32 86.9 -> 81.1, 49 123.2 -> 110.2; 2304 -> 512 1x1 117.2 -> 103.8; 256 -> 256 @30x30 batch 11 80.1 -> 76.4; with 288 steps 512 -> 1024
-// batch 13 131.0, 133.8 without equal shares, 25 224.2, 222.1, with 576 1024 -> 1024 batch 13 238.7, 264.3).
+// The equal-share split of a launch: fills the sk_* fields and the tile counts; returns the scratch bytes it needs, 0 when the shape
+// does not qualify (equal_share_pixel_tiles).  Three workgroups per compute unit with 2x1 wave tiles, two with 2x2: as many as are resident.
 // SMALL_HIP_TUNE keys conv_streamk=<workgroups per compute unit> (0 = never), conv_streamk_min=<steps> (default 128)
 template <int COT, int PXT>
 size_t streamk_cut(ConvArgs &a, int per_cu)
@@ -2436,11 +2426,8 @@ size_t streamk_plan(ConvArgs &a, int *pxt)
     static const int min_steps = tune_int("conv_streamk_min", 128);
     static const int per_cu = tune_int("conv_streamk", -1);
     if (per_cu == 0 || a.slabs != 0 || a.Co % 64 != 0) return 0;
-    const int nsteps = a.kh * a.kw * (a.Ci / CB);
-    const long tiles = (long)(a.Co / 64) * ((a.P + 127) / 128);
-    if (tiles <= NUM_CU / 2 || tiles >= 3 * NUM_CU || tiles % NUM_CU == 0 || nsteps < min_steps) return 0;
-    if (tiles > NUM_CU && nsteps < 256) return 0;
-    *pxt = tiles > NUM_CU ? 2 : 1;
+    *pxt = equal_share_pixel_tiles(a.Co / 64, a.P, a.kh * a.kw * (a.Ci / CB), min_steps);
+    if (*pxt == 0) return 0;
     return *pxt == 2 ? streamk_cut<2, 2>(a, per_cu > 0 ? per_cu : 2) : streamk_cut<2, 1>(a, per_cu > 0 ? per_cu : 3);
 }
 

@@ -26,4 +26,28 @@ inline int c16_runs(long n_tiles, int n_cg, bool always = false)
     return (int)std::min<long>(most, (n_tiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
 }
 
+// Equal shares of the reduction (conv_mfma_f32_streamk_kernel): the wave tile's pixel tiles (2x1 or 2x2), 0 where whole tiles are ahead.
+// n_cg groups of 64 output channels, P pixels, nsteps K-steps.  Between half a round and three rounds of 64 x 128 workgroup tiles that are no
+// whole rounds, and a long reduction (min_steps: 128 unless a measurement asks for another).  Float32 MFMAs, without -> with, batch 16 on 13x13 maps:
+// 512 -> 1024 3x3 287 -> 264 us, 1024 -> 1024 519 -> 467, 256 -> 512 (144 steps) 81 -> 69; with 72 steps or fewer the fix-up pass
+// costs more than the balance gains.  With split products 512 -> 1024 162.9 -> 158.2, 1024 -> 1024 319.6 -> 301.3, 256 -> 512 52.8 -> 50.2,
+// with 72 steps 40.9 -> 50.2.
+// 2x1, or 2x2 (a sixth fewer operands to split for a product) where there are more than 256 of the 2x1 workgroup tiles and 256 steps: 2x1 -> 2x2,
+// 1024 -> 1024 304.7 -> 285.2, batch 20 371.5 -> 360.8, 28 494.7 -> 475.4; 512 -> 1024 160.9 -> 154.8, batch 32 300.8 -> 285.6; 512 -> 512
+// @28x28 batch 12 260.7 -> 247.7; fewer tiles, 512 -> 1024 batch 10 (224) 106.7 -> 110.3, 512 -> 512 @28x28 batch 4 (200) 96.6 -> 104.2.  Its
+// workgroup tiles are 64 x 256, and the half of one that lies past the last pixel is multiplied all the same: at most a sixteenth of the work.
+// 2x1 -> 2x2, 1x1 4096 -> 4096 with 625 pixels (five blocks of 128 or three of 256) 128.3 -> 137.5, 8192 with 320 (three, two) 140.2 -> 173.3,
+// 20480 with 121 (one, one) 134.3 -> 213.2, 2048 with 1089 (nine, five) 112.3 -> 118.7, 1984 with 1290 (eleven, six) 132.0 -> 136.3.
+// More than 256 tiles and fewer steps are whole rounds and a rest in the other launch (256 -> 512 batch 26, 280 tiles, 73.7 -> 67.7,
+// 32 86.9 -> 81.1, 49 123.2 -> 110.2; 2304 -> 512 1x1 117.2 -> 103.8; 256 -> 256 @30x30 batch 11 80.1 -> 76.4; with 288 steps 512 -> 1024
+// batch 13 131.0, 133.8 without equal shares, 25 224.2, 222.1, with 576 1024 -> 1024 batch 13 238.7, 264.3).
+inline int equal_share_pixel_tiles(int n_cg, long P, int nsteps, int min_steps = 128)
+{
+    const long px = (P + 127) / 128, tiles = n_cg * px;
+    if (tiles <= NUM_CU / 2 || tiles >= 3 * NUM_CU || tiles % NUM_CU == 0 || nsteps < min_steps) return 0;
+    if (tiles <= NUM_CU) return 1;
+    if (nsteps < 256) return 0;
+    return 32 * ((P + 255) / 256) <= 17 * px ? 2 : 1;
+}
+
 } // namespace shp

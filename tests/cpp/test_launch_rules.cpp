@@ -40,8 +40,27 @@ static void test_c16_leaves_ragged_launches_to_the_others()
     CHECK(c16_runs(98, 3, true) == 104);
 }
 
+// equal shares of the reduction: 64 x 256 tiles only where the blocks of 256 pixels cover at most a sixteenth more than those of 128
+static void test_equal_shares_with_large_tiles_waste_no_work()
+{
+    for (int n_cg = 1; n_cg <= 768; ++n_cg)
+        for (long P = 1; P <= 98304 / n_cg + 300; P += P < 3000 ? 1 : 61)
+        {
+            const long b128 = (P + 127) / 128, b256 = (P + 255) / 256, tiles = n_cg * b128;
+            const int t = equal_share_pixel_tiles(n_cg, P, 256);
+            CHECK((t != 0) == (tiles > 128 && tiles < 768 && tiles % 256 != 0));
+            CHECK(t != 2 || (tiles > 256 && 16 * (2 * b256 - b128) <= b128));
+            CHECK(t != 1 || tiles <= 256 || 16 * (2 * b256 - b128) > b128);
+            CHECK(equal_share_pixel_tiles(n_cg, P, 255) == (tiles > 256 ? 0 : t) && equal_share_pixel_tiles(n_cg, P, 127) == 0);
+            if (g_failures) return;
+        }
+    CHECK(equal_share_pixel_tiles(64, 625, 256) == 1 && equal_share_pixel_tiles(320, 121, 256) == 1 && equal_share_pixel_tiles(128, 320, 256) == 1);
+    CHECK(equal_share_pixel_tiles(16, 2704, 288) == 2 && equal_share_pixel_tiles(64, 754, 256) == 2);
+}
+
 int main()
 {
+    test_equal_shares_with_large_tiles_waste_no_work();
     test_c16_workgroups_are_resident_at_once();
     test_c16_leaves_ragged_launches_to_the_others();
     std::printf(g_failures ? "%d CHECKS FAILED\n" : "ALL PASSED\n", g_failures);
