@@ -1339,13 +1339,13 @@ __global__ __launch_bounds__(256, (COT * PXT == 2 ? 3 : COT * PXT == 1 ? 4 : 2))
 
 // ---------------------------------------------------------------------------------------------
 // Equal shares of the reduction for launches with few tiles and a long reduction (3x3 convolutions with 512 / 1024
-// channels on a 13x13 map: 352 workgroup tiles for 256 compute units, 288 or 576 K-steps each).  Whole tiles leave a
+// channels on a 13x13 map: 352 workgroup tiles of 64 x 128 for 256 compute units, 288 or 576 K-steps each).  Whole tiles leave a
 // second round in which a third of the machine works; cutting only the left-over tiles four ways (the hybrid kernel) leaves
-// the first round with one wave per SIMD.  Here all K-steps of the launch, tile after tile, are cut into 3 x 256 equal runs;
-// a workgroup multiplies its run (the end of one tile and the start of the next, as a rule) with the LDS-staged body, three
-// workgroups per compute unit, all finishing together.  A run that is not a whole tile leaves its raw accumulators in a
-// scratch block; conv_streamk_fixup_kernel adds the runs of a tile in run order (deterministic) and applies
-// accumulate / bias / activation.
+// the first round with one wave per SIMD.  Here all K-steps of the launch, tile after tile, are cut into equal runs, as many as workgroups are
+// resident (3 x 256 with 2x1 wave tiles, 2 x 256 with 2x2: those 352 tiles are 176 of 64 x 256); a workgroup multiplies its run (the
+// end of one tile and the start of the next, as a rule) with the LDS-staged body, all finishing together.  A run is shorter than a
+// tile (streamk_cut) and leaves its raw accumulators in a scratch block; conv_streamk_fixup_kernel adds the runs of a tile in run order
+// (deterministic) and applies accumulate / bias / activation.
 template <int COT, int PXT>
 constexpr int sk_part_floats() { return 4 * COT * PXT * 16 * WAVE; }
 
@@ -1365,12 +1365,9 @@ __global__ __launch_bounds__(256, (COT * PXT == 2 ? 3 : COT * PXT == 1 ? 4 : 2))
         const int tile = (int)(k0 / nsteps);
         const int sb = (int)(k0 - (long)tile * nsteps);
         const int cnt = (int)(nsteps - sb < k1 - k0 ? nsteps - sb : k1 - k0);
-        float *raw = nullptr;
-        if (cnt != nsteps)
-        {
-            const int first = (int)(((long)tile * nsteps) / a.sk_chunk);          // the run that starts the tile
-            raw = a.sk_scratch + ((size_t)tile * a.sk_parts + (lid - first)) * sk_part_floats<COT, PXT>();
-        }
+        const int first = (int)(((long)tile * nsteps) / a.sk_chunk);              // the run that starts the tile
+        float *raw = a.sk_scratch + ((size_t)tile * a.sk_parts + (lid - first)) * sk_part_floats<COT, PXT>();
+        __builtin_assume(raw != nullptr);
         conv_lds_tile<COT, PXT, false, false, false, BUF>(a, lds_a, tile % a.n_co_groups, tile / a.n_co_groups, sb, cnt, raw);
         k0 += cnt;
         __syncthreads();                                              // the next tile stages into the same LDS buffers
@@ -1386,7 +1383,6 @@ __global__ __launch_bounds__(256) void conv_streamk_fixup_kernel(const ConvArgs 
     const int nsteps = a.kh * a.kw * (a.Ci / CB);
     const int first = (int)(((long)tile * nsteps) / a.sk_chunk);
     const int last = (int)(((long)(tile + 1) * nsteps - 1) / a.sk_chunk);
-    if (last == first) return;                  // one run covered the whole tile and wrote it through the epilogue
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 31, half = lane >> 5;
     const int cg = tile % a.n_co_groups, pxb = tile / a.n_co_groups;
     const int HoWo = a.Ho * a.Wo, CoB = a.Co / CB;
@@ -2416,6 +2412,7 @@ size_t streamk_cut(ConvArgs &a, int per_cu)
     const int nsteps = a.kh * a.kw * (a.Ci / CB), chunks = per_cu * NUM_CU;
     const long total = (long)a.n_blocks * nsteps;
     a.sk_chunk = (int)((total + chunks - 1) / chunks);
+    if (a.sk_chunk >= nsteps) return 0;              // whole tiles: nothing to share (767 tiles, or fewer workgroups asked for)
     a.sk_chunks = (int)((total + a.sk_chunk - 1) / a.sk_chunk);
     a.sk_parts = (nsteps + a.sk_chunk - 1) / a.sk_chunk + 1;
     a.per_xcd = (a.sk_chunks + NUM_XCD - 1) / NUM_XCD;
@@ -2431,8 +2428,6 @@ size_t streamk_plan(ConvArgs &a, int *pxt)
     return *pxt == 2 ? streamk_cut<2, 2>(a, per_cu > 0 ? per_cu : 2) : streamk_cut<2, 1>(a, per_cu > 0 ? per_cu : 3);
 }
 
-// the equal-share launch pair; *done = false: the shape does not qualify.  The first call on a stream allocates the
-// scratch block (small_hip_workspace_reserve does it ahead of time), like the uint8 convolution's filter pre-pass.
 template <int COT, int PXT>
 void launch_streamk_tile(const ConvArgs &a, hipStream_t s)
 {
@@ -2440,6 +2435,8 @@ void launch_streamk_tile(const ConvArgs &a, hipStream_t s)
     else hipLaunchKernelGGL((conv_mfma_f32_streamk_kernel<COT, PXT>), dim3(a.per_xcd * NUM_XCD), dim3(256), 0, s, a);
     hipLaunchKernelGGL((conv_streamk_fixup_kernel<COT, PXT>), dim3(a.n_blocks, COT * PXT), dim3(256), 0, s, a);
 }
+// the equal-share launch pair; *done = false: the shape does not qualify.  The first call on a stream allocates the
+// scratch block (small_hip_workspace_reserve does it ahead of time), like the uint8 convolution's filter pre-pass.
 int launch_streamk(const char *op, ConvArgs &a, hipStream_t s, bool *done)
 {
     *done = false;

@@ -84,26 +84,42 @@ def test_conv2d_f32(lib, oracle, case, mode):
     del cib
 
 
-# few workgroup tiles and a long reduction: the equal-share split of the K-steps (two runs per compute unit, raw
+# few workgroup tiles and a long reduction: the equal-share split of the K-steps (two or three runs per compute unit, raw
 # accumulators through a scratch block, fixed-order fix-up pass).  First case: 136 tiles x 144 steps, every tile cut into
-# four or five runs; second: 600 tiles of 144 steps, which run as whole rounds and a rest; third: 5x5 window, stride 2, a ragged last pixel block.
+# four or five runs; second: 5x5 window, stride 2, a ragged last pixel block.
 EQUAL_SHARE_CASES = [
     (1, 3, 3, 1, (1, 1, 1, 1), 256, 256, 65, 65),
-    (1, 3, 3, 1, (1, 1, 1, 1), 64, 256, 240, 320),
     (3, 5, 5, 2, (2, 2, 2, 2), 128, 96, 150, 141),
 ]
+# 600 tiles of 144 steps: whole rounds and a rest
+WHOLE_TILE_CASES = [(1, 3, 3, 1, (1, 1, 1, 1), 64, 256, 240, 320)]
 
 
-@pytest.mark.parametrize("case", [(1, 3, (1, 1, 1, 1), 512, 512, 65, 65, False), (2, 1, (0, 0, 0, 0), 576, 4096, 50, 37, True)], ids=str)
+def equal_share_bytes(lib, case):
+    """Scratch of the equal-share launch; 0: the shape is another kernel's."""
+    batch, kh, kw, s, pads, Co, Ci, H, W = case
+    return lib.small_hip_conv2d_f32_workspace_bytes(batch, kh, kw, s, *pads, Co, Ci, H, W)
+
+
+def test_equal_share_cases_take_the_split(lib):
+    assert all(equal_share_bytes(lib, c) > 0 for c in EQUAL_SHARE_CASES) and not any(equal_share_bytes(lib, c) for c in WHOLE_TILE_CASES)
+    # 767 tiles in 768 runs would be whole tiles
+    assert equal_share_bytes(lib, (1, 1, 1, 1, (0, 0, 0, 0), 767 * 64, 4096, 8, 8)) == 0
+
+
+@pytest.mark.parametrize("case", [(1, 3, (1, 1, 1, 1), 512, 512, 65, 65, False), (2, 1, (0, 0, 0, 0), 576, 4096, 50, 37, True),
+                                  (1, 1, (0, 0, 0, 0), 5504, 4096, 16, 17, True)], ids=str)
 def test_conv2d_f32_equal_share_split_larger_wave_tile(lib, case):
-    """More than 256 workgroup tiles and 256 K-steps: 64 x 256 tiles instead of 64 x 128, the last pixel block a fraction of one.  Against
-    float64 with the bound of a chain of float32 roundings."""
+    """More than 256 workgroup tiles and 256 K-steps: 64 x 256 tiles instead of 64 x 128, the last pixel block a fraction of one; third case: three
+    blocks of 128 pixels, which stay 64 x 128.  Against float64 with the bound of a chain of float32 roundings."""
     import torch
     batch, k, (pt, pb, pl, pr), Co, Ci, H, W, partial = case
     x, f = synth.normal(31, batch * Ci * H * W), synth.he_normal(32, Co * Ci * k * k, Ci * k * k)
     old, bias = synth.normal(33, batch * Co * H * W), synth.normal(34, Co)
-    n_tiles, steps = (Co // 64) * -(-(batch * H * W) // 128), k * k * Ci // 16
-    assert 256 < n_tiles < 768 and n_tiles % 256 and steps >= 256, "the case would not take the larger tile"
+    px = -(-(batch * H * W) // 128)
+    n_tiles = (Co // 64) * px
+    assert equal_share_bytes(lib, (batch, k, k, 1, (pt, pb, pl, pr), Co, Ci, H, W)) > 0
+    assert n_tiles > 256 and (16 * (px % 2) <= px) == (Co != 5504), "the case would not take this tile"
     dx, df, do, db = hu.dev(x), hu.dev(f), hu.dev(old), hu.dev(bias)
     fn = lib.small_hip_partial_conv2d_bias_act_f32 if partial else lib.small_hip_conv2d_bias_act_f32
     capi.check(fn(batch, k, k, 1, pt, pb, pl, pr, Co, Ci, H, W, hu.ptr(dx), hu.ptr(df), hu.ptr(db), capi.ACT_LEAKY, 0.1, hu.ptr(do), hu.stream()))
@@ -116,15 +132,12 @@ def test_conv2d_f32_equal_share_split_larger_wave_tile(lib, case):
 
 
 @pytest.mark.parametrize("mode", ["conv", "partial", "bias_leaky"])
-@pytest.mark.parametrize("case", EQUAL_SHARE_CASES, ids=str)
+@pytest.mark.parametrize("case", EQUAL_SHARE_CASES + WHOLE_TILE_CASES, ids=str)
 def test_conv2d_f32_equal_share_split(lib, oracle, case, mode):
     batch, kh, kw, s, (pt, pb, pl, pr), Co, Ci, H, W = case
     x = synth.normal(21, batch * Ci * H * W)
     f = synth.he_normal(22, Co * Ci * kh * kw, Ci * kh * kw)
     Ho, Wo = oracle.out_hw(kh, kw, s, pt, pb, pl, pr, H, W)
-    # the launcher's own rule: 2 x 1 wave tiles -> 64 channels x 128 pixels per workgroup tile
-    n_tiles, steps = (Co // 64) * -(-(batch * Ho * Wo) // 128), kh * kw * Ci // 16
-    assert 128 < n_tiles < 768 and n_tiles % 256 and steps >= 128, "the case would not take the equal-share launch"
     o0 = synth.normal(23, batch * Co * Ho * Wo)
     bias = synth.normal(24, Co)
     dx, df, do, db = hu.dev(x), hu.dev(f), hu.dev(o0), hu.dev(bias)

@@ -66,16 +66,14 @@ SHAPES = [  # batch, window, stride, Co, Ci, H, W
 
 
 def equal_shares(shape):
-    """The launcher's rule: one 32 x 32 tile per SIMD at least, 129 to 767 tiles of 64 channels x 128 pixels that are no whole rounds
-    of 256, and 128 K-steps."""
+    """Does the launcher cut this shape into equal shares?  Those launches alone need scratch."""
     n, k, s, co, ci, h, w = shape
-    px = n * -(-h // s) * -(-w // s)
-    tiles = co // 64 * -(-px // 128)
-    return -(-co // 32) * -(-px // 32) >= 1024 and co % 64 == 0 and 128 < tiles < 768 and tiles % 256 != 0 and k * k * ci // 16 >= 128
+    return capi.load().small_hip_conv2d_f32_workspace_bytes(n, k, k, s, *capi.calc_padding(h, k, s), *capi.calc_padding(w, k, s), co, ci, h, w) > 0
 
 
 def test_equal_share_shapes():
-    assert equal_shares((16, 3, 1, 512, 240, 13, 13)) and not equal_shares((8, 3, 1, 512, 160, 13, 13))
+    assert [s for s in SHAPES if equal_shares(s)] == [(16, 3, 1, 512, 240, 13, 13)]
+    assert [s for s in FORMS if equal_shares(s)] == [(16, 3, 1, 512, 240, 13, 13)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)
