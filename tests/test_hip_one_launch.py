@@ -169,26 +169,32 @@ def test_fmodel_general_kernel_on_other_models():
                                         ("strided", 50), ("single", 1), ("single", 33)])
 def test_fmodel_bands_equal_whole_images(form, batch):
     """Bands of rows compute the same sums in the same order as whole images (which a captured call takes): the same bits, and
-    the oracle's values.  Streams past the last slot take whole images too."""
+    the oracle's values.  Streams past the last slot take whole images too.  Consecutive launches on a stream have different inputs: rows
+    that the launch before left in the slot are wrong ones."""
     import torch
     m = _chain_net(form)
     w, x = models.make_weights(m), models.make_input(m, batch)
     ex = models.HipExecutor(m, batch, w, x)
     ex.build_one_launch()
     ex.capture(one_launch=True)
-    ex.one_out.zero_()
-    ex.replay()
-    whole = ex.output_one_launch().copy()
-    assert_close_f32(whole, OracleExecutor(m, batch, w, x).forward(), what="%s, batch %d vs oracle" % (m.name, batch))
+    inputs, whole = [ex.buf["in"].clone(), -1.5 * ex.buf["in"].flip(0)], []
+    for xi in inputs:
+        ex.buf["in"].copy_(xi)
+        ex.one_out.zero_()
+        ex.replay()
+        whole.append(ex.output_one_launch().copy())
+        assert_close_f32(whole[-1], OracleExecutor(m, batch, w, xi.cpu().numpy()).forward(), what="%s, batch %d vs oracle" % (m.name, batch))
+    assert not np.array_equal(whole[0], whole[1])
     streams = [torch.cuda.Stream() for _ in range(6)]
-    outs = [torch.zeros_like(ex.one_out) for _ in range(3 * len(streams))]
+    outs = [torch.zeros_like(ex.one_out) for _ in range(8 * len(streams))]
     torch.cuda.synchronize()
+    which = lambda i: (i // len(streams) + i) % 2
     for i, out in enumerate(outs):      # in flight at the same time, and again on the streams that have run before
         s = streams[i % len(streams)]
-        capi.check(ex.lib.small_hip_fmodel_forward(ex.qmodel, batch, ex._p(ex.buf["in"]), ex._p(out), C.c_void_p(s.cuda_stream)))
+        capi.check(ex.lib.small_hip_fmodel_forward(ex.qmodel, batch, ex._p(inputs[which(i)]), ex._p(out), C.c_void_p(s.cuda_stream)))
     torch.cuda.synchronize()
     for i, out in enumerate(outs):
-        assert np.array_equal(out.cpu().numpy().view(np.uint8), whole.view(np.uint8)), "launch %d differs" % i
+        assert np.array_equal(out.cpu().numpy().view(np.uint8), whole[which(i)].view(np.uint8)), "launch %d differs" % i
     ex.close()
 
 
