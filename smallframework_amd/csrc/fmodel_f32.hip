@@ -112,9 +112,8 @@ __device__ __forceinline__ float4 load_shared(const float *g)
     const unsigned long long b = __hip_atomic_load(d + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return __builtin_bit_cast(float4, make_uint4((unsigned)a, (unsigned)(a >> 32), (unsigned)b, (unsigned)(b >> 32)));
 }
-// Every load and store of this wave is complete, a store_shared in the place that every XCD reads; the compiler moves no memory access across.
-// With a workgroup barrier behind it this is the release in front of the (relaxed) count of a finished band.
-__device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// The compiler moves no memory access across (a builtin wait alone does not keep it from that).
+__device__ __forceinline__ void keep_order() { asm volatile("" ::: "memory"); }
 
 // ---- model creation: weights into operand order ---------------------------------------------------------------
 // kind K_CONV: packed filter [Co/16][Ci/16][taps][16 ci][16 co] -> Wt[Co/16][taps][Ci/16][kq][co16][j]
@@ -1014,7 +1013,10 @@ __global__ __launch_bounds__(NT) void fmodel_f32_sep_kernel(const SepArgs a, con
         else sep_pw<1, TO_RING>(L, lds, wl, mid, nullptr, 0, wave, lane, rg.x, rg.y);
         L = N;
         rg = rn;
-        wait_memory();                           // the weights have landed in LDS, the slot's rows in memory
+        // vmcnt(0): the weights have landed in LDS, and the slot's rows where every XCD reads them; with the barrier this is the release in front of
+        // the (relaxed) count of a finished band
+        keep_order();
+        __builtin_amdgcn_s_waitcnt(0x0F70);
         __syncthreads();
     }
 
@@ -1026,7 +1028,7 @@ __global__ __launch_bounds__(NT) void fmodel_f32_sep_kernel(const SepArgs a, con
         if (tid == 0) *last = __hip_atomic_fetch_add(counters + n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
         if (*last != (unsigned)bands - 1) return;        // the whole workgroup leaves together
-        asm volatile("" ::: "memory");                   // the bands' rows are read after the count (the acquire)
+        keep_order();                                    // the bands' rows are read after the count
         if (tid == 0) __hip_atomic_store(counters + n, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // for the next launch on this stream
         sep_pool<true>(a, lds, tensor, vec, gpool, wave, lane);
     }
