@@ -561,6 +561,8 @@ int small_hip_fmodel_forward(const small_hip_fmodel *model, int batch, const flo
 /* floats of one image's output / bytes of LDS the launch uses */
 size_t small_hip_fmodel_output_elems(const small_hip_fmodel *model);
 size_t small_hip_fmodel_lds_bytes(const small_hip_fmodel *model);
+/* bands (workgroups) that an image of such a call is cut into: 1 = whole images, 0 = bad argument; launches nothing */
+int small_hip_fmodel_bands(const small_hip_fmodel *model, int batch, small_hip_stream_t stream);
 int small_hip_fmodel_destroy(small_hip_fmodel *model);
 
 #ifdef __cplusplus

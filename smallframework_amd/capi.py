@@ -138,6 +138,7 @@ SIGNATURES = {
     "small_hip_fmodel_forward": (_i, [_p, _i, _p, _p, _p]),
     "small_hip_fmodel_output_elems": (_sz, [_p]),
     "small_hip_fmodel_lds_bytes": (_sz, [_p]),
+    "small_hip_fmodel_bands": (_i, [_p, _i, _p]),
     "small_hip_fmodel_destroy": (_i, [_p]),
     "small_hip_pack": (_i, [_i, _i] + [_u32] * 6 + [_p, _p, _sz, _p]),
     "small_hip_unpack": (_i, [_i, _i] + [_u32] * 6 + [_p, _p, _sz, _p]),

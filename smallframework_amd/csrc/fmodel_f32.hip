@@ -1068,19 +1068,21 @@ struct small_hip_fmodel
     size_t ranges_off = 0, slot_bytes = 0;
     int rows = 0, band_batch = 0;                    // rows of the last pair's output; images a slot has room for (0: no slots)
     std::vector<int> ranges_first;                   // [rows per band] -> first range (int2) of that cut, -1: not planned
+    std::vector<float> band_work;                    // [rows per band] -> work of the longest band (bands_pay)
     unsigned char *slots = nullptr;                  // [SLOTS][band_batch] tensors
     unsigned *counters = nullptr;                    // [SLOTS][band_batch]
     mutable std::mutex mu;
     mutable int n_slots = 0;
     mutable hipStream_t slot_stream[SLOTS];
 
-    // the slot of this stream, or -1: others got all of them before it
-    int slot(hipStream_t s) const
+    // the slot of this stream, or -1: others got all of them before it (take = false: the slot it would get)
+    int slot(hipStream_t s, bool take) const
     {
         std::lock_guard<std::mutex> lk(mu);
         for (int i = 0; i < n_slots; ++i)
             if (slot_stream[i] == s) return i;
         if (n_slots == SLOTS) return -1;
+        if (!take) return n_slots;
         slot_stream[n_slots] = s;
         return n_slots++;
     }
@@ -1215,6 +1217,7 @@ bool plan_separable(const small_hip_flayer *layers, const std::vector<FMLayer> &
     const int rows = at(pool).H;
     m->rows = rows;
     m->ranges_first.assign((size_t)rows + 1, -1);
+    m->band_work.assign((size_t)rows + 1, 0.f);
     for (int rb = 1; rb <= rows; rb = rb < rows && rb + 1 > (rows + 1) / 2 ? rows : rb + 1)
     {
         m->ranges_first[(size_t)rb] = (int)ranges.size() / 2;
@@ -1222,6 +1225,7 @@ bool plan_separable(const small_hip_flayer *layers, const std::vector<FMLayer> &
         {
             std::vector<int> band((size_t)(n_pairs + 1) * 2);
             int lo = r, hi = std::min(r + rb, rows);
+            float work = 0.f;
             for (int u = n_pairs; u >= 0; --u)
             {
                 if (lo >= hi) return false;          // a band that reads padding only
@@ -1229,18 +1233,21 @@ bool plan_separable(const small_hip_flayer *layers, const std::vector<FMLayer> &
                 band[(size_t)u * 2] = lo * Wo;
                 band[(size_t)u * 2 + 1] = hi * Wo;
                 if (u == 0) break;
-                const FMLayer &D = at(2 * u - 1);
+                const FMLayer &D = at(2 * u - 1), &C = at(2 * u);
+                const int np = (hi - lo) * Wo;
+                work += (float)(np * (D.Ci / 4)) / (float)NT + 0.25f * (float)((np + 15) / 16 * (C.Co / CB) * (C.Ci / CB)) / (float)NW;
                 const int in_lo = lo * D.stride - D.pt, in_hi = (hi - 1) * D.stride - D.pt + 3;
                 lo = std::max(in_lo, 0);
                 hi = std::min(in_hi, D.H);
             }
             ranges.insert(ranges.end(), band.begin(), band.end());
+            m->band_work[(size_t)rb] = std::max(m->band_work[(size_t)rb], work);
         }
     }
     return true;
 }
 
-// Rows per band for this batch (all rows: whole images): as many bands as compute units take at once.
+// Rows per band for this batch (all rows: whole images): as many bands as compute units take at once, where they pay.
 // DS-CNN (25 rows; us of a launch), general kernel / whole images here / bands: batch 1 26.9 / 25.6 / 15.6 (1 row), 16 27.4 / 25.9 / 17.9 (2),
 // 41 27.4 / 26.1 / 19.6 (5), 85 27.6 / 26.2 / 22.1 (9), 128 27.7 / 26.3 / 23.9 (13), 256 27.8 / 26.4; a second round of bands costs more than it
 // gives (batch 100 in three bands: 34.2).
@@ -1248,19 +1255,21 @@ int rows_per_band(const small_hip_fmodel *m, int batch)
 {
     static const int force = tune_int("fmodel_band", -1);
     if (batch > m->band_batch || force == 0) return m->rows;
-    const int bands = NUM_CU / batch;                // two at least: band_batch
-    const int rows = force > 0 ? force : (m->rows + bands - 1) / bands;
-    return m->ranges_first[(size_t)std::min(rows, m->rows)] >= 0 ? std::min(rows, m->rows) : m->rows;
+    const int most = NUM_CU / batch;                 // bands, two at least: band_batch
+    const int rows = std::min(force > 0 ? force : (m->rows + most - 1) / most, m->rows);
+    if (m->ranges_first[(size_t)rows] < 0) return m->rows;
+    const float saved = m->band_work[(size_t)m->rows] - m->band_work[(size_t)rows];
+    return force > 0 || bands_pay(saved, batch, (m->rows + rows - 1) / rows) ? rows : m->rows;
 }
 
 // The stream's slot; none (-1) for a stream that is being captured (a graph may be replayed on any stream, at the same time as other
 // launches) and for the per-thread default stream, whose handle stands for several streams.
-int band_slot(const small_hip_fmodel *m, hipStream_t s)
+int band_slot(const small_hip_fmodel *m, hipStream_t s, bool take)
 {
     if (s == hipStreamPerThread) return -1;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &st) != hipSuccess) { (void)hipGetLastError(); return -1; }
-    return st == hipStreamCaptureStatusNone ? m->slot(s) : -1;
+    return st == hipStreamCaptureStatusNone ? m->slot(s, take) : -1;
 }
 
 } // namespace
@@ -1489,6 +1498,7 @@ int small_hip_fmodel_create(int n_layers, const small_hip_flayer *layers, small_
     {
         const size_t per_image = (size_t)m->sep.last_elems * 4, fit = small_hip_fmodel::SLOT_BYTES / per_image;
         m->band_batch = (int)std::min<size_t>(fit, NUM_CU / 2);
+        while (m->band_batch > 0 && rows_per_band(m, m->band_batch) == m->rows) --m->band_batch;      // the largest batch whose bands pay
         m->slot_bytes = up256(m->band_batch * per_image);
         slot_bytes = m->slot_bytes * small_hip_fmodel::SLOTS;
         counter_bytes = (size_t)m->band_batch * small_hip_fmodel::SLOTS * sizeof(unsigned);
@@ -1564,7 +1574,7 @@ int small_hip_fmodel_forward(const small_hip_fmodel *model, int batch, const flo
     if (model->separable)
     {
         int rows = rows_per_band(model, batch), slot = 0;
-        if (rows < model->rows && (slot = band_slot(model, as_stream(stream))) < 0) rows = model->rows;
+        if (rows < model->rows && (slot = band_slot(model, as_stream(stream), true)) < 0) rows = model->rows;
         const int bands = (model->rows + rows - 1) / rows;
         hipLaunchKernelGGL(fmodel_f32_sep_kernel, dim3((unsigned)batch * bands), dim3(NT), (size_t)model->hdr.lds_bytes, as_stream(stream),
                            model->sep, reinterpret_cast<const SepPair *>(dev), dblob, input, output,
@@ -1581,6 +1591,14 @@ int small_hip_fmodel_forward(const small_hip_fmodel *model, int batch, const flo
 }
 
 size_t small_hip_fmodel_output_elems(const small_hip_fmodel *model) { return model ? (size_t)model->hdr.out_elems : 0; }
+int small_hip_fmodel_bands(const small_hip_fmodel *model, int batch, small_hip_stream_t stream)
+{
+    if (!model || batch <= 0) return 0;
+    if (!model->separable) return 1;
+    const int rows = rows_per_band(model, batch);
+    return rows < model->rows && band_slot(model, as_stream(stream), false) >= 0 ? (model->rows + rows - 1) / rows : 1;
+}
+
 size_t small_hip_fmodel_lds_bytes(const small_hip_fmodel *model) { return model ? (size_t)model->hdr.lds_bytes : 0; }
 
 int small_hip_fmodel_destroy(small_hip_fmodel *model)

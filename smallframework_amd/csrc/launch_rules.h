@@ -50,4 +50,13 @@ inline int equal_share_pixel_tiles(int n_cg, long P, int nsteps, int min_steps =
     return 32 * ((P + 255) / 256) <= 17 * px ? 2 : 1;
 }
 
+// Whole-model launch of a depthwise-separable chain: do bands of rows on several compute units pay for storing the last pair's rows and
+// for the workgroup that gathers them?  `saved`: what the longest band does less than a whole image, in depthwise outputs (four channels of a
+// pixel) over the 1024 lanes plus a quarter of the 16 x 16 x 16 products over the 16 waves; about a microsecond each.  The exchange is
+// one of them, and a second one when every compute unit stores at the same time.  47 chains of one to five pairs at batches 1 to 120, us of whole
+// images -> bands: DS-CNN (saved 12.8) 25.7 -> 15.6, 64 channels @13x9 and one pair to 16 (2.1) 9.1 -> 7.9, 32 @8x13 (1.5) level, batch 60 (1.2) 9.7 ->
+// 11.0; few rows, whose bands compute each other's halo: 48-64-80 @3x1 9.4 -> 10.7, 64-80-64-128 @3x7 level; tiny ones, 16 @13x6 6.5 -> 6.9, batch 60
+// 6.8 -> 7.7.  Against the faster form each time this rule loses 0.13 us at most where it cuts and 0.6 where it does not.
+inline bool bands_pay(float saved, int batch, int bands) { return saved > 1.f + (float)batch * (float)bands / NUM_CU; }
+
 } // namespace shp

@@ -58,8 +58,16 @@ static void test_equal_shares_with_large_tiles_waste_no_work()
     CHECK(equal_share_pixel_tiles(16, 2704, 288) == 2 && equal_share_pixel_tiles(64, 754, 256) == 2);
 }
 
+// bands of rows: not for a model whose bands save less than the exchange costs, and more is asked when every compute unit stores
+static void test_bands_pay()
+{
+    CHECK(bands_pay(12.8f, 1, 25) && bands_pay(6.28f, 128, 2));
+    CHECK(!bands_pay(0.9f, 1, 25) && !bands_pay(1.5f, 128, 2) && bands_pay(1.5f, 1, 8));
+}
+
 int main()
 {
+    test_bands_pay();
     test_equal_shares_with_large_tiles_waste_no_work();
     test_c16_workgroups_are_resident_at_once();
     test_c16_leaves_ragged_launches_to_the_others();

@@ -134,21 +134,21 @@ def _chain_net(form):
     """float32 depthwise-separable chains: few images run in bands of rows on several compute units."""
     if form == "dscnn":
         return models.dscnn()
-    b = models._Builder("chain_" + form, "f32", (3, 53, 9) if form == "strided" else (2, 14, 6), "normal")
+    b = models._Builder("chain_" + form, "f32", (3, 53, 9) if form == "strided" else (2, 28, 12), "normal")
     if form == "strided":               # odd maps, strides 2, 53 -> 27 -> 27 -> 14 rows, 5 -> 3 columns, two fully connected layers
         b.advance(b.conv(32, 3, 2, "same", act="leaky", slope=0.1))
         b.dw(3, 1, act="relu")
-        b.advance(b.conv(80, 1, 1, "valid", act="leaky", slope=0.2))
+        b.advance(b.conv(48, 1, 1, "valid", act="leaky", slope=0.2))
         b.dw(3, 2)
-        b.advance(b.conv(48, 1, 1, "valid"))
+        b.advance(b.conv(80, 1, 1, "valid"))
         b.pool("maxpool", 14, 3, 1)
         b.dense(32)
         b.dense(20)
     else:                               # one pair, nothing behind the pooling
-        b.advance(b.conv(16, 5, 1, "same", act="relu"))
+        b.advance(b.conv(32, 5, 1, "same", act="relu"))
         b.dw(3, 1)
-        b.advance(b.conv(64, 1, 1, "valid", act="relu"))
-        b.pool("avgpool", 14, 6, 1)
+        b.advance(b.conv(32, 1, 1, "valid", act="relu"))
+        b.pool("avgpool", 28, 12, 1)
     return b.done()
 
 
@@ -186,6 +186,8 @@ def test_fmodel_bands_equal_whole_images(form, batch):
         assert_close_f32(whole[-1], OracleExecutor(m, batch, w, xi.cpu().numpy()).forward(), what="%s, batch %d vs oracle" % (m.name, batch))
     assert not np.array_equal(whole[0], whole[1])
     streams = [torch.cuda.Stream() for _ in range(6)]
+    cut = [ex.lib.small_hip_fmodel_bands(ex.qmodel, batch, C.c_void_p(s.cuda_stream)) for s in streams]
+    assert cut[0] > 1 or batch > 128, "the launches would all be whole images"
     outs = [torch.zeros_like(ex.one_out) for _ in range(8 * len(streams))]
     torch.cuda.synchronize()
     which = lambda i: (i // len(streams) + i) % 2
@@ -195,7 +197,39 @@ def test_fmodel_bands_equal_whole_images(form, batch):
     torch.cuda.synchronize()
     for i, out in enumerate(outs):
         assert np.array_equal(out.cpu().numpy().view(np.uint8), whole[which(i)].view(np.uint8)), "launch %d differs" % i
+    # the stream that warmed the capture up and three of these hold a slot for as long as the model lives
+    now = [ex.lib.small_hip_fmodel_bands(ex.qmodel, batch, C.c_void_p(s.cuda_stream)) for s in streams]
+    assert now == [cut[0]] * 3 + [1] * 3
     ex.close()
+
+
+def _one_pair(c, h, w):
+    b = models._Builder("one_pair", "f32", (2, h, w), "normal")
+    b.advance(b.conv(c, 3, 1, "same", act="relu"))
+    b.dw(3, 1, act="relu")
+    b.advance(b.conv(16, 1, 1, "valid", act="relu"))
+    b.pool("maxpool", h, w, 1)
+    return b.done()
+
+
+def test_fmodel_bands_only_where_they_pay():
+    """The exchange between bands costs about a microsecond and a half: small models, and batches that leave a band most of an image, run as
+    whole images."""
+    def bands(m, batches):
+        ex = models.HipExecutor(m, 1)
+        ex.build_one_launch()
+        got = [ex.lib.small_hip_fmodel_bands(ex.qmodel, b, ex.stream()) for b in batches]
+        ex.close()
+        return got
+    assert bands(models.dscnn(), (0, 1, 16, 41, 85, 128, 129)) == [0, 25, 13, 5, 3, 2, 1]
+    assert bands(_one_pair(16, 13, 6), (1, 6, 60, 120)) == [1, 1, 1, 1]
+    few_rows = models._Builder("few_rows", "f32", (1, 10, 4), "normal")     # DS-CNN's layers on 5 x 2 pixels: a band computes most of them
+    few_rows.advance(few_rows.conv(64, 10, 2, "same", act="relu", kw=4))
+    for _ in range(4):
+        few_rows.dw(3, 1, act="relu")
+        few_rows.advance(few_rows.conv(64, 1, 1, "valid", act="relu"))
+    few_rows.pool("avgpool", 5, 2, 1)
+    assert bands(few_rows.done(), (1, 9, 51)) == [1, 1, 1]
 
 
 def _exposed_u8_net(hw, form):
