@@ -536,7 +536,11 @@ int small_hip_pool1d_u8(int is_max, int batch, int kernel_width, int stride, int
  * them is refused with SMALL_HIP_EINVAL and a message.  small_hip_fmodel_create() copies and re-orders filters and
  * biases (it allocates device memory and returns after its work on `stream` has finished);
  * small_hip_fmodel_forward() is one launch and allocates nothing; few images of a depthwise-separable chain run in
- * bands of rows on several compute units (same bits; on the first four streams that ask, not under capture).  Results are within the float32 tolerance of the
+ * bands of rows on several compute units where that is faster (same bits).  What the bands exchange lies in memory of
+ * the model; the first four streams that launch it so keep a part each for as long as the model lives, any further
+ * stream, a call under capture and the per-thread default stream run whole images.  A stream is known by its handle:
+ * destroy one that has launched the model when its work is done (hipStreamDestroy of ROCm 7 waits for that itself), and
+ * a later stream of the same handle takes over its part.  Results are within the float32 tolerance of the
  * layer-by-layer calls (another summation order), not bit-identical to them. */
 #define SMALL_HIP_FL_CONV 0
 #define SMALL_HIP_FL_DWCONV 1

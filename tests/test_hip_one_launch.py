@@ -203,6 +203,39 @@ def test_fmodel_bands_equal_whole_images(form, batch):
     ex.close()
 
 
+def test_fmodel_bands_on_streams_that_come_and_go():
+    """Streams created and destroyed behind their work: a handle that is given out again takes over the slot, and no launch reads rows of
+    another stream's."""
+    import torch
+    m, batch = models.dscnn(), 9
+    ex = models.HipExecutor(m, batch, models.make_weights(m), models.make_input(m, batch))
+    hip = C.CDLL(capi.LIB_PATH)              # (symbols of the runtime that the library is bound to)
+    hip.hipStreamCreate.argtypes, hip.hipStreamDestroy.argtypes = [C.POINTER(C.c_void_p)], [C.c_void_p]
+    ex.build_one_launch()
+    inputs = [ex.buf["in"].clone(), -1.5 * ex.buf["in"].flip(0)]
+    outs, handles, cut = [torch.zeros_like(ex.one_out) for _ in range(12)], set(), []
+    torch.cuda.synchronize()
+    for i, out in enumerate(outs):
+        s = C.c_void_p()
+        assert hip.hipStreamCreate(C.byref(s)) == 0
+        handles.add(s.value)
+        cut.append(ex.lib.small_hip_fmodel_bands(ex.qmodel, batch, s))
+        for _ in range(3):
+            capi.check(ex.lib.small_hip_fmodel_forward(ex.qmodel, batch, ex._p(inputs[i % 2]), ex._p(out), s))
+        assert hip.hipStreamDestroy(s) == 0
+    torch.cuda.synchronize()
+    print("handles", len(handles), "bands", cut, flush=True)
+    assert max(cut) > 1
+    want = []
+    for xi in inputs:
+        ex.buf["in"].copy_(xi)
+        ex.forward_one_launch()
+        want.append(ex.output_one_launch().copy())
+    for i, out in enumerate(outs):
+        assert np.array_equal(out.cpu().numpy().view(np.uint8), want[i % 2].view(np.uint8)), "stream %d" % i
+    ex.close()
+
+
 def _one_pair(c, h, w):
     b = models._Builder("one_pair", "f32", (2, h, w), "normal")
     b.advance(b.conv(c, 3, 1, "same", act="relu"))
