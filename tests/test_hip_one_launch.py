@@ -2,6 +2,9 @@
 uint8 (small_hip_qmodel_*): bit-exact against the CPU oracle running the same layers one after the other, and
 against the layer-by-layer GPU path.  float32 (small_hip_fmodel_*): within the float32 bar of the oracle."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -11,6 +14,7 @@ from oracle.model_exec import OracleExecutor
 from util import assert_close_f32, assert_equal_exact
 
 pytestmark = pytest.mark.gpu
+TESTS = os.path.dirname(os.path.abspath(__file__))
 
 
 def _run(model, batch, seed=99):
@@ -163,6 +167,66 @@ def test_fmodel_general_kernel_on_other_models():
     got, layered, want = _run(b.done(), 5)
     assert_close_f32(got, want, what="general kernel vs oracle")
     assert_close_f32(got, layered, what="general kernel vs layer by layer")
+
+
+def _general_net(form):
+    """Models that are no chain of the separable kernel's, for the parts of the general one."""
+    b = models._Builder(form, "f32", {"stem_conv": (3, 12, 11), "dw5": (1, 21, 8), "dw_pool": (2, 9, 13), "rings": (1, 36, 22)}[form], "normal")
+    if form == "stem_conv":              # gathered first layer, then an ordinary 3x3 convolution, pooling to LDS, two fully connected layers
+        b.advance(b.conv(32, 3, 1, "same", act="relu"))
+        b.advance(b.conv(32, 3, 2, "same", act="leaky", slope=0.1))
+        b.pool("avgpool", b.h, b.w, 1)
+        b.dense(40)
+        b.dense(10)
+    elif form == "dw5":                  # a 5x5 depthwise layer (not fused with the 1x1 behind it), one that is, maximum pooling, a dense head
+        b.advance(b.conv(32, 5, 2, "same", act="relu", kw=3))
+        b.dw(5, 1, act="leaky")
+        b.advance(b.conv(32, 1, 1, "valid", act="relu"))
+        b.dw(3, 2, act="relu")
+        b.advance(b.conv(80, 1, 1, "valid"))
+        b.pool("maxpool", b.h, b.w, 1)
+        b.dense(20)
+    elif form == "dw_pool":              # a 3x3 depthwise layer with no 1x1 behind it; the pooling is the output
+        b.advance(b.conv(16, 3, 1, "same"))
+        b.dw(3, 1, act="relu")
+        b.pool("maxpool", b.h, b.w, 1)
+    else:                                # a separable chain whose tensors with their rings of zeros do not fit LDS
+        b.advance(b.conv(32, 3, 1, "same", act="relu"))
+        b.dw(3, 2, act="relu")
+        b.advance(b.conv(16, 1, 1, "valid", act="relu"))
+        b.pool("avgpool", b.h, b.w, 1)
+        b.dense(12)
+    return b.done()
+
+
+@pytest.mark.parametrize("batch", [1, 7])
+@pytest.mark.parametrize("form", ["stem_conv", "dw5", "dw_pool", "rings"])
+def test_fmodel_general_kernel(form, batch):
+    m = _general_net(form)
+    got, layered, want = _run(m, batch)
+    assert_close_f32(got, want, what="%s, batch %d vs oracle" % (form, batch))
+    assert_close_f32(got, layered, what="%s, batch %d vs layer by layer" % (form, batch))
+    assert np.abs(want).max() > 0.05
+
+
+def test_dscnn_on_the_general_kernel():
+    """DS-CNN with the separable kernel switched off (read once per process: a child), against the oracle, and against the separable
+    kernel: the same sums in the same order."""
+    code = ("import sys; sys.path[:0] = %r\n"
+            "import numpy as np, test_hip_one_launch as t\n"
+            "from smallframework_amd import models\n"
+            "m = models.dscnn(); x = models.make_input(m, 5, seed=99)\n"
+            "ex = models.HipExecutor(m, 5, models.make_weights(m), x); ex.build_one_launch(); ex.forward_one_launch()\n"
+            "got = ex.output_one_launch(); want = t.OracleExecutor(m, 5, models.make_weights(m), x).forward()\n"
+            "t.assert_close_f32(got, want, what='DS-CNN, general kernel vs oracle')\n"
+            "print('RESULT', ex.one_launch_lds_bytes(), got.tobytes().hex())\n" % ([os.path.dirname(TESTS), TESTS],))
+    results = []
+    for tune in ("fmodel_sep=0", "fmodel_sep=1"):
+        r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100, env=dict(os.environ, SMALL_HIP_TUNE=tune))
+        assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+        results.append([l for l in r.stdout.splitlines() if l.startswith("RESULT")][0].split()[1:])
+    assert results[0][0] != results[1][0], "both ran on the same kernel"
+    assert results[0][1] == results[1][1]
 
 
 @pytest.mark.parametrize("form,batch", [("dscnn", 1), ("dscnn", 7), ("dscnn", 23), ("dscnn", 41), ("dscnn", 128), ("dscnn", 300), ("strided", 1), ("strided", 30),
