@@ -193,9 +193,11 @@ int small_hip_conv2d_bias_act_dwconv2d_bias_act_f32(int batch, int kernel_height
                                                     const float *dw_filter, const float *dw_bias, int act,
                                                     float negative_slope, float *output, small_hip_stream_t stream);
 /* Does the library run this convolution + depthwise pair as ONE launch when both are available (the rule the entry
- * point below applies; shapes only, no pointers)?  0: no (the one-launch kernels are not built for it, or the two
- * launches are faster); 1: yes, and the result equals the two launches bit for bit; 2: yes, within float32 rounding of
- * the two launches (the stand-alone convolution may add its products in another order). */
+ * point below applies; shapes only, no pointers)?  0: no (the one-launch kernels are not built for it, the two launches
+ * are faster, or its callers keep the two launches' bits: 96 and 128 input channels in front of a stride-2 depthwise
+ * layer, which the entry point above runs as one launch, the faster one); 1: yes, and the result equals the two launches
+ * bit for bit; 2: yes, within float32 rounding of the two launches (the stand-alone convolution may add its products in
+ * another order). */
 int small_hip_conv2d_dwconv2d_one_launch_f32(int batch, int kernel_height, int kernel_width, int stride, int t_pad,
                                              int b_pad, int l_pad, int r_pad, int dw_kernel_height,
                                              int dw_kernel_width, int dw_stride, int dw_t_pad, int dw_b_pad,
@@ -203,8 +205,8 @@ int small_hip_conv2d_dwconv2d_one_launch_f32(int batch, int kernel_height, int k
                                              int input_height, int input_width);
 /* The same pairing for ANY convolution + depthwise pair, given the intermediate buffer the reference's functions take
  * (`inter_output_buf`, include/small/fused_interface_abstract.hpp:1840-1850): [batch][Co/16][Ho][Wo][16], the
- * convolution's output size.  Succeeds wherever the two layers would.  One launch where a one-launch form exists and
- * is the faster choice (the two forms above; the intermediate buffer is then not touched), the two layers through
+ * convolution's output size.  Succeeds wherever the two layers would.  One launch where the rule above says so (the
+ * intermediate buffer is then not touched), the two layers through
  * `intermediate` otherwise.  input, intermediate and output must not overlap. */
 int small_hip_conv2d_bias_act_dwconv2d_bias_act_via_f32(int batch, int kernel_height, int kernel_width, int stride,
                                                         int t_pad, int b_pad, int l_pad, int r_pad, int dw_kernel_height,

@@ -2905,8 +2905,8 @@ int small_hip_conv2d_dwconv2d_one_launch_f32(int batch, int kh, int kw, int stri
     // a pointwise convolution parked in LDS under 14 x 14 (stride 2: 7 x 8) depthwise tiles (pw_dw_f32): short reductions
     // on maps that fill those tiles to 70%, where the recomputed halo costs less than the second launch.  Batch 64:
     // 32 -> 64 @112x112 stride 2 113 -> 48 us, 64 -> 128 @56x56 67 -> 45, 128 -> 256 @28x28 45 -> 33, 96 -> 192 @28x28
-    // 34 -> 22.  96 and 128 channels at stride 2 are faster as one launch too (128 -> 128 @56x56 64.7 -> 52.5); a caller who wants that
-    // asks for it (HipExecutor's plan does), this answer to the callers that leave the choice here stays what it has been
+    // 34 -> 22.  96 and 128 channels at stride 2 are faster as one launch too (128 -> 128 @56x56 64.7 -> 52.5) and are not in this rule: its callers
+    // have had the two launches and their bits; HipExecutor's plan asks for the one launch itself
     if (kh != 1 || kw != 1 || stride != 1 || pt || pb || pl || pr || Ci % CB != 0 || Co % 32 != 0 || (dw_stride != 1 && dw_stride != 2))
         return 0;
     const int cib = Ci / CB;

@@ -68,7 +68,7 @@ def test_one_launch_predicate_of_conv_dw_pairs():
     assert pw(32, 64, 112, 112, 2, (0, 1, 0, 1)) == 1          # MobileNetV1's fused pairs
     assert pw(64, 128, 56, 56) == 1
     assert pw(128, 256, 28, 28) == 2                           # eight K-steps: float32 rounding against two launches
-    assert pw(128, 128, 56, 56, 2, (0, 1, 0, 1)) == 0          # stride 2 behind eight K-steps: two launches are faster
+    assert pw(128, 128, 56, 56, 2, (0, 1, 0, 1)) == 0          # stride 2 behind eight K-steps: stays two launches for this rule's callers
     assert pw(512, 512, 14, 14) == 0 and pw(80, 64, 28, 28) == 0 and pw(32, 48, 28, 28) == 0
     assert pw(32, 64, 5, 40) == 0                              # fills the 14 x 14 tiles to 48%
     assert pw(32, 64, 28, 28, 3) == 0
