@@ -2780,12 +2780,8 @@ int pw_dw_f32(const char *op, int batch, int dw_stride, int dpt, int dpb, int dp
     g.tiles_x = (g.Wd + tow - 1) / tow; g.tiles_y = (g.Hd + toh - 1) / toh;
     const long nt = (long)batch * g.tiles_x * g.tiles_y;
     const StemDwArgs d{dw_filt, dw_bias};
-    // Channels per workgroup: 32 (four waves of two pixel tiles each, four workgroups per compute unit), or 64 (eight waves of one pixel
-    // tile and two channel tiles: the pixels are read and split for twice the channels) where the K loop is the larger part and there
-    // are two such workgroups for every compute unit.  32 -> 64: 128 -> 256 @28x28 batch 64 36.0 -> 33.7 us, 96 -> 192 24.3 -> 22.8, 128 -> 128
-    // @56x56 stride 2 58.3 -> 56.6, batch 16 (512 workgroups) 17.0 -> 15.9, batch 1 6.7 -> 8.5, 128 -> 128 @28x28 batch 8 (64) 8.1 -> 9.9;
-    // 64 -> 128 @56x56 batch 64 45.0 -> 45.6.  SMALL_HIP_TUNE key pwdw_cot=1|2.
-    int cot = cib >= 6 && Co % 64 == 0 && nt * (Co / 64) >= 2 * NUM_CU ? 2 : 1;
+    // channels per workgroup: SMALL_HIP_TUNE key pwdw_cot=1|2
+    int cot = pw_dw_channel_tiles(cib, Co, nt);
     { static const int v = tune_int("pwdw_cot", 0); if (v == 1 || (v == 2 && Co % 64 == 0 && cib >= 6)) cot = v; }
     g.n_cg = Co / (32 * cot);
     if (nt * g.n_cg > 0x7fffffffL / 2) { set_error("%s: too many tiles for one launch", op); return SMALL_HIP_EINVAL; }

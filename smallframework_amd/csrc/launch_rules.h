@@ -50,6 +50,21 @@ inline int equal_share_pixel_tiles(int n_cg, long P, int nsteps, int min_steps =
     return 32 * ((P + 255) / 256) <= 17 * px ? 2 : 1;
 }
 
+// conv_pw_dw3x3_f32_kernel: 32-channel tiles of a workgroup, 1 (four waves of two pixel tiles each, four workgroups per compute unit) or 2 (eight
+// waves of one pixel tile, two workgroups: the pixels are read and split for twice the channels).  cib blocks of input channels, n_tiles
+// spatial tiles over all images.  Two where the K loop is the larger part: 32 -> 64 channels, 128 -> 256 @28x28 batch 64 36.0 -> 33.7 us, 96 -> 192
+// 24.3 -> 22.8, 128 -> 128 @56x56 stride 2 58.3 -> 56.6; 64 -> 128 @56x56 batch 64 45.0 -> 45.6.  And where its workgroups come in rounds of one
+// per compute unit that are more than half full, or are six such rounds at least: a nearly empty round lasts as long as a full one.  128 -> 256
+// @28x28, rounds 2.0: 21.3 -> 19.7, 2.1: 24.6 -> 25.9, 2.5 level, 2.8: 28.4 -> 26.7, 3.2: 32.8 -> 33.1, 3.8: 37.1 -> 34.5, 4.1 level, 4.6: 44.9 ->
+// 42.0; 128 -> 320 @15x12 stride 2, 2.3: 9% behind.  Of 64 output channels 1 is ahead everywhere (128 -> 64 @42x41, rounds 2.0: 10%, 6.2: 2%; 96
+// -> 64 @28x14 2 to 7%).
+inline int pw_dw_channel_tiles(int cib, int Co, long n_tiles)
+{
+    const long n = n_tiles * (Co / 64), part = n % NUM_CU;
+    if (cib < 6 || Co % 64 != 0 || Co < 128 || n < 2 * NUM_CU) return 1;
+    return part == 0 || part > NUM_CU / 2 || n >= 6 * NUM_CU ? 2 : 1;
+}
+
 // Whole-model launch of a depthwise-separable chain: do bands of rows on several compute units pay for storing the last pair's rows and
 // for the workgroup that gathers them?  `saved`: what the longest band does less than a whole image, in depthwise outputs (four channels of a
 // pixel) over the 1024 lanes plus a quarter of the 16 x 16 x 16 products over the 16 waves; about a microsecond each.  The exchange is

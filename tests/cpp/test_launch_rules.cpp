@@ -58,6 +58,24 @@ static void test_equal_shares_with_large_tiles_waste_no_work()
     CHECK(equal_share_pixel_tiles(16, 2704, 288) == 2 && equal_share_pixel_tiles(64, 754, 256) == 2);
 }
 
+// pointwise + depthwise launch: workgroups of 64 channels where they fill their rounds
+static void test_workgroups_of_sixty_four_channels_fill_their_rounds()
+{
+    for (int cib = 1; cib <= 8; ++cib)
+        for (int Co = 32; Co <= 1024; Co += 32)
+            for (long nt = 1; nt <= 3000; ++nt)
+            {
+                const long n = nt * (Co / 64);
+                const int c = pw_dw_channel_tiles(cib, Co, nt);
+                CHECK(c == 1 || (c == 2 && cib >= 6 && Co % 64 == 0 && Co > 64 && n >= 512));
+                CHECK(c == 1 || n >= 1536 || (n + 255) / 256 * 256 - n < 128);
+                if (g_failures) return;
+            }
+    CHECK(pw_dw_channel_tiles(8, 256, 256) == 2 && pw_dw_channel_tiles(8, 128, 256) == 2);      // 1024 and 512 workgroups
+    CHECK(pw_dw_channel_tiles(8, 256, 136) == 1 && pw_dw_channel_tiles(8, 448, 76) == 1);       // 544 and 532: a third round of 32 and 20
+    CHECK(pw_dw_channel_tiles(8, 64, 576) == 1 && pw_dw_channel_tiles(4, 256, 256) == 1);
+}
+
 // bands of rows: not for a model whose bands save less than the exchange costs, and more is asked when every compute unit stores
 static void test_bands_pay()
 {
@@ -68,6 +86,7 @@ static void test_bands_pay()
 int main()
 {
     test_bands_pay();
+    test_workgroups_of_sixty_four_channels_fill_their_rounds();
     test_equal_shares_with_large_tiles_waste_no_work();
     test_c16_workgroups_are_resident_at_once();
     test_c16_leaves_ragged_launches_to_the_others();

@@ -212,14 +212,17 @@ def test_pointwise_dw_random_shapes(lib):
         assert_equal_exact(hu.host(do), hu.host(d2), what)
 
 
-@pytest.mark.parametrize("case", [  # workgroups of 64 channels (96 or 128 input channels, 512 workgroups at least) and the last size before them
-    (64, 1, 64, 96, 29, 30, True), (43, 2, 128, 96, 29, 27, False), (64, 1, 128, 128, 15, 31, False), (33, 2, 64, 128, 57, 55, True),
-    (63, 1, 64, 128, 29, 27, True), (64, 1, 96, 96, 28, 28, True)], ids=str)
+@pytest.mark.parametrize("case", [  # workgroups of 64 channels (96 or 128 input channels, rounds of 256 more than half full), and not
+    (66, 1, 128, 96, 29, 30, True), (60, 2, 128, 96, 29, 27, False), (64, 1, 128, 128, 15, 31, False), (39, 2, 128, 128, 57, 55, True),
+    (63, 1, 128, 128, 29, 27, True), (43, 2, 128, 96, 29, 27, False), (64, 1, 64, 96, 29, 30, True), (64, 1, 96, 96, 28, 28, True)], ids=str)
 def test_pointwise_dw_sixty_four_channels(lib, case):
     """Against float64, with the bound of a chain of Ci + 9 float32 roundings, and (96 channels: fewer than eight K-steps) against this
     library's two launches bit for bit."""
     import torch
     batch, ds, Co, Ci, H, W, bias = case
+    tiles = batch * (-(-H // 14) * -(-W // 14) if ds == 1 else -(-(-(-H // 2)) // 7) * -(-(-(-W // 2)) // 8)) * (Co // 64)
+    takes = Co % 64 == 0 and Co > 64 and tiles >= 512 and (tiles % 256 == 0 or tiles % 256 > 128 or tiles >= 1536)
+    assert takes == (case not in ((43, 2, 128, 96, 29, 27, False), (64, 1, 64, 96, 29, 30, True), (64, 1, 96, 96, 28, 28, True)))
     x, f = synth.normal(1, batch * Ci * H * W), synth.he_normal(2, Co * Ci, Ci)
     fd, b, bd = synth.he_normal(3, Co * 9, 9), synth.normal(4, Co), synth.normal(5, Co)
     Hd, Wd = capi.out_dim(H, 1, 1, 3, ds), capi.out_dim(W, 1, 1, 3, ds)
